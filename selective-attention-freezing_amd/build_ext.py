@@ -31,8 +31,10 @@ HIPCC_FLAGS = [
 # alive across their loops; with the default AGPR form the compiler parks
 # them in VGPRs and copies every one into AGPRs and back around each product
 # (hundreds of v_accvgpr moves per query block).  The VGPR form of the MFMA
-# instructions removes the copies and lowers register use.
-SOURCE_FLAGS = {"attn_bwd.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form")}
+# instructions removes the copies and lowers register use.  The float32
+# kernels hold their accumulators across loops the same way.
+SOURCE_FLAGS = {"attn_bwd.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form"),
+                "attn_f32.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form")}
 
 
 def _hipcc():

@@ -1,520 +1,766 @@
 // float32 inputs: the reference's IEEE-dot contract (kernel/fused_attn.py:36-37,
 // :128-140; tests at 2e-5 forward / 2e-4 backward, kernel/test_fused_attn.py:188-190).
 //
-// The MFMA kernels take bf16 / fp16 only; fp32 q/k/v run here, in fp32 FMAs
-// on the vector ALUs throughout (no bf16 rounding of scores, P or
-// products).  This is the precision path, not the fast one: one workgroup =
-// 256 threads over a BQ x BK tile (64 x 64, or 32 x 32 at hd 256) staged in
-// LDS; thread (tr, tc) = (tid / 16, tid % 16) owns rows tr * RPT + i and
-// keys / columns tc + 16 c, so a row's 16 threads are 16 consecutive lanes
-// and its reductions are four xor shuffles.
+// The 16-bit MFMA kernels round scores, P and products to their input type;
+// fp32 q/k/v run here on v_mfma_f32_32x32x2_f32, whose inputs, products and
+// sums are fp32 throughout (157 TFLOP/s, twice the vector ALUs' fp32 rate,
+// and one LDS or memory operand per 4096 flops).
+//
+// Every kernel gives a workgroup one 32-row tile of its output (queries for
+// out and dQ, keys for dK / dV) and its 4 waves every fourth 32-row block of
+// the other axis; the waves share nothing until their accumulators (and the
+// softmax's running max and sum) are merged through LDS at the end, so the
+// block loop has no barrier and the causal work of a tile is spread over
+// four SIMDs.  A block's operands come straight from memory into registers
+// (each is used by one wave only), each product's loads issued one product
+// (2048 cycles at hd 64) ahead into the registers the previous one freed:
+//   RowFrag  lane (m, g) holds elements 8t + 4g + 0..3 of row m: one 16-byte
+//            load feeds four MFMAs (k = the lane half, so four MFMAs walk
+//            the eight columns in the order 0|4, 1|5, 2|6, 3|7 in both operands)
+//   ColFrag  lane (m, g) holds columns NE m + 0..NE-1 of rows 8a + 4g + r:
+//            the A operand of an accumulator tile e whose rows are the
+//            columns NE m + e
+// The 32x32 product's accumulator register i of lane (n, g) is row
+// 8 (i / 4) + 4 g + i % 4 of column n, which is exactly the B operand
+// (rows 8a + r of half 0 and 8a + 4 + r of half 1) of the second product
+// over ColFrag row i: P and dS never leave their registers.
+//
+// Bound by the matrix pipe: at B=4, 12 heads (9 live), T=1000, hd 64 the
+// forward + backward takes 322 us against 1762 us on the vector ALUs
+// (64 x 64 tiles in LDS, one workgroup per tile); the forward alone at B=8,
+// 12 live heads, T=2000 runs at 115 TFLOP/s (25 before).
 //
 //   live heads     online softmax in base 2 (scale sm_scale log2 e), output
 //                  divided by the row sum, LSE = m + log2(l) as the MFMA path
 //   dense heads    P read from the (P, S, S) buffer (fp32 / bf16 / fp16)
-//   decomposed     P = exp2((alpha_j + rho_{i-j} - z_i) log2 e) in fp32
+//   decomposed     P = exp(alpha_j + rho_{i-j} - z_i) in fp32
 //                  (closed-form heads run here through their decomposed
 //                  buffers)
-//   backward       delta = rowsum(out * dout); dQ per query block; dK / dV
-//                  per key block (live heads); dV = P^T dO per key block
-//                  (frozen heads)
+//   backward       dQ per query tile, which also writes delta = rowsum(out *
+//                  dout); dK / dV per key tile (live heads); dV = P^T dO per
+//                  key tile (frozen heads)
+#include <type_traits>
+
 #include "saf_kernels.h"
 
 namespace saf {
 
 namespace {
 
-template <int HD> struct F32Tile {
-  static constexpr int B = HD <= 128 ? 64 : 32;  // rows of a query or key tile
-  static constexpr int RPT = B / 16;             // rows (or keys) per thread
-  static constexpr int DPT = HD / 16;            // columns per thread
-  static constexpr int LD = HD + 4;              // LDS row pitch (floats): float4 rows, banks spread
+constexpr int kW = 4;   // waves of a workgroup
+constexpr int kR = 32;  // rows of an output tile and of a block
+
+template <int HD> struct F32Shape {
+  static constexpr int NE = HD / 32;       // accumulator tiles (columns NE m + e)
+  static constexpr int NT = HD / 8;        // 16-byte row pieces per lane
+  static constexpr int LD = HD + 4;        // LDS pitch of a merged tile's rows (floats)
+  // operand fragments of a tile held in LDS: [NT][64 lanes] x 16 bytes
+  static constexpr int FRAG = kR * HD;     // floats
+  static constexpr int MERGE = kW * kR * LD;
+  // whole blocks of operands fit the registers beside the accumulators up to
+  // hd 128; above, they are loaded piece by piece next to their use
+  static constexpr bool kWhole = HD <= 128;
 };
 
-// rows r0 .. r0 + R - 1 of a (T, HD) fp32 matrix with row stride st -> dst
-// (rows >= T are zero)
-template <int R, int HD, int LD>
-__device__ __forceinline__ void load_rows(float (*dst)[LD], const float* base, int64_t st, int r0, int T_len,
-                                          int tid) {
-  constexpr int V4 = HD / 4;
-  for (int idx = tid; idx < R * V4; idx += 256) {
-    const int r = idx / V4, c = idx % V4;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (r0 + r < T_len) v = *reinterpret_cast<const float4*>(base + (int64_t)(r0 + r) * st + 4 * c);
-    *reinterpret_cast<float4*>(&dst[r][4 * c]) = v;
-  }
+__device__ __forceinline__ f32x16_t mfma2(float a, float b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-// acc[i][c] = sum_d a[ra + i][d] * b[rb + 16 c][d]
-template <int NI, int NC, int HD, int LD>
-__device__ __forceinline__ void dots(float (&acc)[NI][NC], const float (*a)[LD], int ra, const float (*b)[LD],
-                                     int rb) {
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned u32x3_t __attribute__((ext_vector_type(3)));
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+
+// Keeps the compiler's scheduler from moving loads across: left alone it sank
+// each load next to its use (with a full wait) to save registers.
+#define SAF_PIN() __builtin_amdgcn_sched_barrier(0)
+
+__device__ __forceinline__ float4 buf_load4(__amdgpu_buffer_rsrc_t r, int off) {
+  return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+
+// Rows r0 .. r0 + 31 of a (T, st) fp32 tensor as a row operand.
+template <int HD, bool WHOLE = F32Shape<HD>::kWhole> struct RowFrag {
+  static constexpr int NT = F32Shape<HD>::NT;
+  float4 r[WHOLE ? NT : 1];
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ void load(const float* base, int64_t st, int r0, int T_len, int off) {
+    rsrc = rows_rsrc(base, st, r0, T_len);
+    if constexpr (WHOLE) {
+      SAF_PIN();
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
+      for (int t = 0; t < NT; ++t) r[t] = buf_load4(rsrc, off + 32 * t);
+      SAF_PIN();
+    }
+  }
+  // acc[row][n] += sum_d rows[row][d] b[n][d], b's fragments in LDS
+  __device__ __forceinline__ f32x16_t dot(const float4* b, int lane, int off, f32x16_t acc) const {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[i][c] = 0.f;
-#pragma unroll 2
-  for (int d = 0; d < HD; d += 4) {
-    float4 av[NI], bv[NC];
+    for (int t0 = 0; t0 < NT; t0 += 4) {
+      float4 a[4];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) av[i] = *reinterpret_cast<const float4*>(&a[ra + i][d]);
+      for (int u = 0; u < 4; ++u) a[u] = WHOLE ? r[WHOLE ? t0 + u : 0] : buf_load4(rsrc, off + 32 * (t0 + u));
 #pragma unroll
-    for (int c = 0; c < NC; ++c) bv[c] = *reinterpret_cast<const float4*>(&b[rb + 16 * c][d]);
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        float s = acc[i][c];
-        s = fmaf(av[i].x, bv[c].x, s);
-        s = fmaf(av[i].y, bv[c].y, s);
-        s = fmaf(av[i].z, bv[c].z, s);
-        s = fmaf(av[i].w, bv[c].w, s);
-        acc[i][c] = s;
+      for (int u = 0; u < 4; ++u) {
+        const float4 q = b[(t0 + u) * 64 + lane];
+        acc = mfma2(a[u].x, q.x, acc);
+        acc = mfma2(a[u].y, q.y, acc);
+        acc = mfma2(a[u].z, q.z, acc);
+        acc = mfma2(a[u].w, q.w, acc);
       }
+      SAF_PIN();  // bounds the b fragments held ahead
+    }
+    return acc;
+  }
+};
+// this lane's byte offset of a row operand
+__device__ __forceinline__ int row_off(int64_t st, int lane) { return (int)((lane & 31) * st * 4) + 16 * (lane >> 5); }
+
+// Rows r0 .. r0 + 31 of a (T, st) fp32 tensor as a column operand.
+template <int HD, bool WHOLE = F32Shape<HD>::kWhole> struct ColFrag {
+  static constexpr int NE = F32Shape<HD>::NE;
+  float c[WHOLE ? 16 : 1][NE];
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ static void row(__amdgpu_buffer_rsrc_t rs, float (&d)[NE], int off) {
+    if constexpr (NE == 1) {
+      d[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
+    } else if constexpr (NE == 2) {
+      const u32x2_t w = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
+      d[0] = __uint_as_float(w[0]);
+      d[1] = __uint_as_float(w[1]);
+    } else if constexpr (NE == 3) {
+      const u32x3_t w = __builtin_amdgcn_raw_buffer_load_b96(rs, off, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 3; ++e) d[e] = __uint_as_float(w[e]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < NE / 4; ++u) {
+        const u32x4_t w = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * u, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[4 * u + e] = __uint_as_float(w[e]);
+      }
+    }
+  }
+  __device__ __forceinline__ void load(const float* base, int64_t st, int r0, int T_len, int off) {
+    rsrc = rows_rsrc(base, st, r0, T_len);
+    if constexpr (WHOLE) {
+      SAF_PIN();
+      // the sixteen row offsets are formed here each time: held across the
+      // loop they cost sixteen registers per operand and spilled
+      asm volatile("" : "+v"(off));
+#pragma unroll
+      for (int i = 0; i < 16; ++i) row(rsrc, c[i], off + (8 * (i >> 2) + (i & 3)) * (int)(st * 4));
+      SAF_PIN();
+    }
+  }
+  // o[e][column][n] += sum_row rows[row][NE column + e] w[row][n]
+  __device__ __forceinline__ void axpy(f32x16_t (&o)[NE], const float (&w)[16], int64_t st, int off) const {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float d[NE];
+      if constexpr (WHOLE) {
+#pragma unroll
+        for (int e = 0; e < NE; ++e) d[e] = c[WHOLE ? i : 0][e];
+      } else {
+        row(rsrc, d, off + (8 * (i >> 2) + (i & 3)) * (int)(st * 4));
+      }
+#pragma unroll
+      for (int e = 0; e < NE; ++e) o[e] = mfma2(d[e], w[i], o[e]);
+      if constexpr (!WHOLE)
+        if (i % 4 == 3) SAF_PIN();
+    }
+  }
+};
+// this lane's byte offset of a column operand
+template <int HD> __device__ __forceinline__ int col_off(int64_t st, int lane) {
+  return (int)((lane >> 5) * 4 * st * 4) + (lane & 31) * F32Shape<HD>::NE * 4;
+}
+
+// Row of accumulator register i of lane half g within a 32-row block.
+__device__ __forceinline__ int acc_row(int i, int g) { return 8 * (i >> 2) + 4 * g + (i & 3); }
+
+// The tile's own 32 rows as B fragments in LDS, each wave a quarter of the pieces.
+template <int HD>
+__device__ __forceinline__ void stage_tile(float4* dst, const float* base, int64_t st, int r0, int T_len, int wave,
+                                           int lane) {
+  const __amdgpu_buffer_rsrc_t r = rows_rsrc(base, st, r0, T_len);
+  for (int t = wave; t < F32Shape<HD>::NT; t += kW) dst[t * 64 + lane] = buf_load4(r, row_off(st, lane) + 32 * t);
+}
+
+// This wave's accumulators into its (32, HD) slab of the merge buffer, times f.
+template <int HD>
+__device__ __forceinline__ void put_tile(float* sm, const f32x16_t (&o)[F32Shape<HD>::NE], float f, int wave, int lane) {
+  constexpr int NE = F32Shape<HD>::NE, LD = F32Shape<HD>::LD;
+  float* row = sm + (wave * kR + (lane & 31)) * LD + NE * 4 * (lane >> 5);
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    float w[4 * NE];  // columns NE (8a + 4g) + 0 .. 4 NE - 1
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int e = 0; e < NE; ++e) w[NE * r + e] = o[e][4 * a + r] * f;
+#pragma unroll
+    for (int u = 0; u < NE; ++u)
+      *reinterpret_cast<float4*>(row + 8 * NE * a + 4 * u) = make_float4(w[4 * u], w[4 * u + 1], w[4 * u + 2], w[4 * u + 3]);
   }
 }
 
-__device__ __forceinline__ float group16_max(float x) {
+// The four waves' slabs summed and stored: rows r0 .. of dst, times scale
+// (per row where row_scale is given).  Rows past T are dropped.
+template <int HD>
+__device__ __forceinline__ void store_sum(const float* sm, float* dst, int64_t st, int r0, int T_len, float scale,
+                                          const float* row_scale, int tid) {
+  constexpr int V4 = HD / 4, LD = F32Shape<HD>::LD;
+  for (int idx = tid; idx < kR * V4; idx += 64 * kW) {
+    const int r = idx / V4, c = idx % V4;
+    if (r0 + r >= T_len) continue;
+    float4 s = *reinterpret_cast<const float4*>(sm + r * LD + 4 * c);
 #pragma unroll
-  for (int off = 1; off < 16; off <<= 1) x = fmaxf(x, __shfl_xor(x, off));
-  return x;
-}
-__device__ __forceinline__ float group16_sum(float x) {
-#pragma unroll
-  for (int off = 1; off < 16; off <<= 1) x += __shfl_xor(x, off);
-  return x;
+    for (int w = 1; w < kW; ++w) {
+      const float4 x = *reinterpret_cast<const float4*>(sm + (w * kR + r) * LD + 4 * c);
+      s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+    }
+    const float f = row_scale != nullptr ? row_scale[r] : scale;
+    // 8-byte stores: the outputs' rows are only 8-byte aligned by contract
+    float2* o = reinterpret_cast<float2*>(dst + (int64_t)(r0 + r) * st + 4 * c);
+    o[0] = make_float2(s.x * f, s.y * f);
+    o[1] = make_float2(s.z * f, s.w * f);
+  }
 }
 
-// frozen-head probability P[i, j] (0 outside j <= i < T)
-struct FrozenP {
-  int kind;  // 1 dense, 2 decomposed
+// Pattern inputs of frozen heads.  The element reads take any strides and
+// storage type, with indexes clamped into the buffers (the cells they stand
+// for are masked); FAST kernels (fp32 buffers with unit inner strides, every
+// model's layout) read four neighbours per 16-byte load instead: 4 loads per
+// 16 cells in place of 16, each of which cost a 64-bit address and a type
+// switch.
+struct FrozenCells {
   const void* patt;
-  int patt_dtype;
-  int64_t prow0, p_si, p_sj;  // element offset of the head's pattern, row / column strides
   const void* alpha;
   const void* rho;
   const void* z;
-  int a_dtype, r_dtype, z_dtype;
-  int64_t a0, a_ss, r0, r_ss, z0, z_ss;
-  __device__ __forceinline__ float operator()(int i, int j, int T_len) const {
-    if (j > i || i >= T_len) return 0.f;
-    if (kind == 1) return load_as_f32(patt, prow0 + (int64_t)i * p_si + (int64_t)j * p_sj, patt_dtype);
-    // alpha + rho - z with the rounding error of the sum carried (TwoSum):
-    // where P matters z is close to alpha + rho, so (s - z) is exact and the
-    // exponent keeps its low bits even for logits of scale 100+
-    const float a = load_as_f32(alpha, a0 + (int64_t)j * a_ss, a_dtype);
-    const float r = load_as_f32(rho, r0 + (int64_t)(i - j) * r_ss, r_dtype);
+  int patt_dtype, a_dtype, r_dtype, z_dtype, T_len;
+  int64_t prow0, p_si, p_sj, a0, a_ss, r0, r_ss, z0, z_ss;
+  template <typename P> __device__ __forceinline__ void init(const P& p, int ph) {
+    patt = p.patt; alpha = p.alpha; rho = p.rho; z = p.z;
+    patt_dtype = p.patt_dtype; a_dtype = p.a_dtype; r_dtype = p.r_dtype; z_dtype = p.z_dtype;
+    prow0 = (int64_t)ph * p.p_sh; p_si = p.p_si; p_sj = p.p_sj;
+    a0 = (int64_t)ph * p.a_sh; a_ss = p.a_ss;
+    r0 = (int64_t)ph * p.r_sh; r_ss = p.r_ss;
+    z0 = (int64_t)ph * p.z_sh; z_ss = p.z_ss;
+    T_len = p.T;
+  }
+  __device__ __forceinline__ float cell(int i, int j) const {
+    return load_as_f32(patt, prow0 + (int64_t)min(i, T_len - 1) * p_si + (int64_t)min(j, T_len - 1) * p_sj, patt_dtype);
+  }
+  __device__ __forceinline__ float alpha_at(int j) const {
+    return load_as_f32(alpha, a0 + (int64_t)min(j, T_len - 1) * a_ss, a_dtype);
+  }
+  __device__ __forceinline__ float rho_at(int d) const {
+    return load_as_f32(rho, r0 + (int64_t)min(max(d, 0), T_len - 1) * r_ss, r_dtype);
+  }
+  __device__ __forceinline__ float z_at(int i) const {
+    return load_as_f32(z, z0 + (int64_t)min(i, T_len - 1) * z_ss, z_dtype);
+  }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t vec(const void* v, int64_t off) const {
+    return rows_rsrc(reinterpret_cast<const float*>(v) + off, (int64_t)1, 0, T_len);
+  }
+  // the pattern from row i0 < T to column T - 1 of row T - 1 (FAST: the host
+  // has checked that 32 rows fit 32-bit offsets)
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows(int i0) const {
+    return span_rsrc(reinterpret_cast<const float*>(patt) + prow0 + (int64_t)i0 * p_si,
+                     ((int64_t)(T_len - 1 - i0) * p_si + T_len) * 4);
+  }
+  // alpha + rho - z with the rounding error of the sum carried (TwoSum):
+  // where P matters z is close to alpha + rho, so (s - z) is exact and the
+  // exponent keeps its low bits even for logits of scale 100+
+  __device__ __forceinline__ static float prob(float a, float r, float zi) {
     const float s = a + r;
-    const float zi = load_as_f32(z, z0 + (int64_t)i * z_ss, z_dtype);
-    if (!__builtin_isfinite(s)) return expf(s - zi);  // -inf logits (masked keys, windows): exact zeros
     const float bp = s - a;
     const float e = (a - (s - bp)) + (r - bp);
-    return expf((s - zi) + e);
+    // -inf logits (masked keys, windows): exact zeros
+    return expf(__builtin_isfinite(s) ? (s - zi) + e : s - zi);
   }
 };
+
+__device__ __forceinline__ void put4(float (&d)[16], int a, float4 w) {
+  d[4 * a] = w.x; d[4 * a + 1] = w.y; d[4 * a + 2] = w.z; d[4 * a + 3] = w.w;
+}
+
+// One fp32 statistic of the 16 rows this lane's accumulator registers hold,
+// rows r0 .. r0 + 31 of a vector with stride st (rows past T read as 0 or as
+// row T - 1; their cells are masked).
+__device__ __forceinline__ void load_stat(float (&d)[16], const float* base, int64_t st, int r0, int T_len, int g) {
+  if (st == 1) {
+    const __amdgpu_buffer_rsrc_t r = rows_rsrc(base, (int64_t)1, r0, T_len);
+#pragma unroll
+    for (int a = 0; a < 4; ++a) put4(d, a, buf_load4(r, 32 * a + 16 * g));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) d[i] = base[(int64_t)min(r0 + acc_row(i, g), T_len - 1) * st];
+  }
+  SAF_PIN();
+}
 
 // ---- forward -------------------------------------------------------------
 
 template <int HD>
 __global__ __launch_bounds__(256) void f32_live_kernel(const FlashParams p) {
-  using Tl = F32Tile<HD>;
-  constexpr int BQ = Tl::B, BK = Tl::B, RPT = Tl::RPT, DPT = Tl::DPT, LD = Tl::LD;
-  __shared__ __align__(16) float qs[BQ][LD];
-  __shared__ __align__(16) float ks[BK][LD];
-  __shared__ __align__(16) float vs[BK][LD];
-  __shared__ float ps[BQ][BK + 1];
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  const int nqb = (p.T + BQ - 1) / BQ;
-  const int qb = nqb - 1 - (int)blockIdx.x;  // heaviest first
-  const int slot = blockIdx.y, b = blockIdx.z;
-  const int h = p.out_head[slot];
-  const float* qbase = reinterpret_cast<const float*>(p.q) + b * p.q_sb + (int64_t)p.q_head[slot] * p.q_sh;
+  using Sh = F32Shape<HD>;
+  constexpr int NE = Sh::NE;
+  __shared__ __align__(16) float sm[Sh::MERGE > Sh::FRAG ? Sh::MERGE : Sh::FRAG];
+  __shared__ float sm_m[kW][kR], sm_l[kW][kR], sm_inv[kR];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T_len = p.T, nqt = (T_len + kR - 1) / kR, nbh = p.B * p.n_slots;
+  const int qt = nqt - 1 - (int)(blockIdx.x / nbh);  // heaviest first
+  const int bh = (int)(blockIdx.x % nbh);
+  const int b = bh / p.n_slots, slot = bh % p.n_slots;
+  const int h = p.out_head[slot], q0 = qt * kR, q = q0 + n;
   const float* kbase = reinterpret_cast<const float*>(p.k) + b * p.k_sb + (int64_t)p.k_head[slot] * p.k_sh;
   const float* vbase = reinterpret_cast<const float*>(p.v) + b * p.v_sb + (int64_t)p.v_head[slot] * p.v_sh;
-  float* obase = reinterpret_cast<float*>(p.out) + b * p.o_sb + (int64_t)h * p.o_sh;
-  const int T_len = p.T, q0 = qb * BQ;
-  const int nkb = (min(q0 + BQ, T_len) + BK - 1) / BK;
-
-  load_rows<BQ, HD, LD>(qs, qbase, p.q_st, q0, T_len, tid);
-  float m[RPT], l[RPT], o[RPT][DPT];
+  float4* const qf = reinterpret_cast<float4*>(sm);
+  stage_tile<HD>(qf, reinterpret_cast<const float*>(p.q) + b * p.q_sb + (int64_t)p.q_head[slot] * p.q_sh, p.q_st, q0,
+                 T_len, wave, lane);
+  const int ko = row_off(p.k_st, lane), vo = col_off<HD>(p.v_st, lane);
+  RowFrag<HD> kf;
+  ColFrag<HD> vf;
+  // a block past the diagonal loads nothing (an empty descriptor)
+  auto lim = [&](int jb) { return jb <= qt ? T_len : 0; };
+  kf.load(kbase, p.k_st, kR * wave, lim(wave), ko);
+  vf.load(vbase, p.v_st, kR * wave, lim(wave), vo);
+  __syncthreads();
+  float m = -INFINITY, l = 0.f;
+  f32x16_t o[NE];
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.f;
+  for (int e = 0; e < NE; ++e) o[e] = zero16();
+  for (int jb = wave; jb <= qt; jb += kW) {
+    const f32x16_t s = kf.dot(qf, lane, ko, zero16());
+    kf.load(kbase, p.k_st, kR * (jb + kW), lim(jb + kW), ko);
+    float x[16], mx = -INFINITY;
 #pragma unroll
-    for (int c = 0; c < DPT; ++c) o[i][c] = 0.f;
-  }
-  for (int jb = 0; jb < nkb; ++jb) {
-    const int j0 = jb * BK;
-    __syncthreads();  // the previous block's tiles are read
-    load_rows<BK, HD, LD>(ks, kbase, p.k_st, j0, T_len, tid);
-    load_rows<BK, HD, LD>(vs, vbase, p.v_st, j0, T_len, tid);
-    __syncthreads();
-    float s[RPT][RPT];
-    dots<RPT, RPT, HD, LD>(s, qs, tr * RPT, ks, tc);
+    for (int i = 0; i < 16; ++i) x[i] = s[i] * p.scale_log2;
+    if (jb == qt) {
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const int row = q0 + tr * RPT + i;
-      float mx = -INFINITY;
-#pragma unroll
-      for (int c = 0; c < RPT; ++c) {
-        const int key = j0 + tc + 16 * c;
-        s[i][c] = (key <= row && key < T_len) ? s[i][c] * p.scale_log2 : -INFINITY;
-        mx = fmaxf(mx, s[i][c]);
-      }
-      const float m_new = fmaxf(m[i], group16_max(mx));
-      const float corr = m_new == -INFINITY ? 1.f : fast_exp2(m[i] - m_new);
-      float sum = 0.f;
-#pragma unroll
-      for (int c = 0; c < RPT; ++c) {
-        const float e = m_new == -INFINITY ? 0.f : fast_exp2(s[i][c] - m_new);
-        ps[tr * RPT + i][tc + 16 * c] = e;
-        sum += e;
-      }
-      l[i] = l[i] * corr + group16_sum(sum);
-      m[i] = m_new;
-#pragma unroll
-      for (int c = 0; c < DPT; ++c) o[i][c] *= corr;
+      for (int i = 0; i < 16; ++i) x[i] = kR * jb + acc_row(i, g) <= q ? x[i] : -INFINITY;
     }
-    __syncthreads();
-    for (int kk = 0; kk < BK; ++kk) {
-      float vv[DPT];
 #pragma unroll
-      for (int c = 0; c < DPT; ++c) vv[c] = vs[kk][tc + 16 * c];
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, x[i]);
+    const float m_new = fmaxf(m, half_swap_max(mx));
+    const float corr = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);
+    float sum = 0.f;
 #pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const float pv = ps[tr * RPT + i][kk];
-#pragma unroll
-        for (int c = 0; c < DPT; ++c) o[i][c] = fmaf(pv, vv[c], o[i][c]);
-      }
+    for (int i = 0; i < 16; ++i) {
+      x[i] = m_new == -INFINITY ? 0.f : fast_exp2(x[i] - m_new);
+      sum += x[i];
     }
-  }
+    l = l * corr + half_swap_sum(sum);
+    m = m_new;
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int row = q0 + tr * RPT + i;
-    if (row >= T_len) continue;
-    const float inv = l[i] > 0.f ? 1.f / l[i] : 1.f;
+    for (int e = 0; e < NE; ++e)
 #pragma unroll
-    for (int c = 0; c < DPT; ++c) obase[(int64_t)row * p.o_st + tc + 16 * c] = o[i][c] * inv;
-    if (p.lse != nullptr && tc == 0)
-      p.lse[b * p.l_sb + (int64_t)h * p.l_sh + (int64_t)row * p.l_st] = m[i] + __log2f(l[i] > 0.f ? l[i] : 1.f);
+      for (int i = 0; i < 16; ++i) o[e][i] *= corr;
+    vf.axpy(o, x, p.v_st, vo);
+    vf.load(vbase, p.v_st, kR * (jb + kW), lim(jb + kW), vo);
   }
+  if (g == 0) {
+    sm_m[wave][n] = m;
+    sm_l[wave][n] = l;
+  }
+  __syncthreads();  // every wave has read Q: its LDS becomes the merge buffer
+  float M = sm_m[0][n];
+#pragma unroll
+  for (int w = 1; w < kW; ++w) M = fmaxf(M, sm_m[w][n]);
+  float L = 0.f;
+#pragma unroll
+  for (int w = 0; w < kW; ++w) {
+    const float mw = sm_m[w][n];
+    L += mw == -INFINITY ? 0.f : sm_l[w][n] * fast_exp2(mw - M);
+  }
+  put_tile<HD>(sm, o, m == -INFINITY ? 0.f : fast_exp2(m - M), wave, lane);
+  if (wave == 0 && g == 0) {
+    sm_inv[n] = L > 0.f ? 1.f / L : 1.f;
+    if (p.lse != nullptr && q < T_len)
+      p.lse[b * p.l_sb + (int64_t)h * p.l_sh + (int64_t)q * p.l_st] = M + __log2f(L > 0.f ? L : 1.f);
+  }
+  __syncthreads();
+  store_sum<HD>(sm, reinterpret_cast<float*>(p.out) + b * p.o_sb + (int64_t)h * p.o_sh, p.o_st, q0, T_len, 1.f, sm_inv,
+                tid);
 }
 
-template <int HD>
-__global__ __launch_bounds__(256) void f32_frozen_kernel(const FrozenParams p, const int mode) {
-  using Tl = F32Tile<HD>;
-  constexpr int BQ = Tl::B, BK = Tl::B, RPT = Tl::RPT, DPT = Tl::DPT, LD = Tl::LD;
-  __shared__ __align__(16) float vs[BK][LD];
-  __shared__ float ps[BQ][BK + 1];
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  const int nqb = (p.T + BQ - 1) / BQ;
-  const int qb = nqb - 1 - (int)blockIdx.x;
-  const int slot = blockIdx.y, b = blockIdx.z;
-  const int h = p.out_head[slot], ph = p.pat_head[slot];
+// out = P V of frozen heads (DENSE: P from the pattern buffer, else rebuilt);
+// the next block's pattern inputs are fetched before the current product.
+template <int HD, bool DENSE, bool FAST>
+__global__ __launch_bounds__(256) void f32_frozen_kernel(const FrozenParams p) {
+  using Sh = F32Shape<HD>;
+  constexpr int NE = Sh::NE;
+  __shared__ __align__(16) float sm[Sh::MERGE];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T_len = p.T, nqt = (T_len + kR - 1) / kR, nbh = p.B * p.n_slots;
+  const int qt = nqt - 1 - (int)(blockIdx.x / nbh);
+  const int bh = (int)(blockIdx.x % nbh);
+  const int b = bh / p.n_slots, slot = bh % p.n_slots;
+  const int q0 = qt * kR, q = q0 + n;
   const float* vbase = reinterpret_cast<const float*>(p.v) + b * p.v_sb + (int64_t)p.v_head[slot] * p.v_sh;
-  float* obase = reinterpret_cast<float*>(p.out) + b * p.o_sb + (int64_t)h * p.o_sh;
-  const int T_len = p.T, q0 = qb * BQ;
-  const int nkb = (min(q0 + BQ, T_len) + BK - 1) / BK;
-  FrozenP P{};
-  P.kind = mode == 0 ? 1 : 2;
-  P.patt = p.patt; P.patt_dtype = p.patt_dtype;
-  P.prow0 = (int64_t)ph * p.p_sh; P.p_si = p.p_si; P.p_sj = p.p_sj;
-  P.alpha = p.alpha; P.rho = p.rho; P.z = p.z;
-  P.a_dtype = p.a_dtype; P.r_dtype = p.r_dtype; P.z_dtype = p.z_dtype;
-  P.a0 = (int64_t)ph * p.a_sh; P.a_ss = p.a_ss;
-  P.r0 = (int64_t)ph * p.r_sh; P.r_ss = p.r_ss;
-  P.z0 = (int64_t)ph * p.z_sh; P.z_ss = p.z_ss;
-
-  float o[RPT][DPT];
+  FrozenCells P;
+  P.init(p, p.pat_head[slot]);
+  const int vo = col_off<HD>(p.v_st, lane);
+  ColFrag<HD> vf;
+  float u[16], w[16];  // dense: pattern cells; decomposed: alpha_j and rho_{q-j}
+  const __amdgpu_buffer_rsrc_t pr = P.rows(q0), ar = P.vec(P.alpha, P.a0), rr = P.vec(P.rho, P.r0);
+  auto fetch = [&](int jb) {
+    const int j0 = kR * jb + 4 * g;  // keys j0 + 8a + r
+    if (FAST && (DENSE || jb < qt)) {
+      // below the diagonal block every distance is >= 1, so the four
+      // distances q - j0 - 8a - 3 .. - 0 are one load; columns and distances
+      // past T belong to masked cells or dropped rows (they read the next
+      // row's values or zeros)
 #pragma unroll
-  for (int i = 0; i < RPT; ++i)
+      for (int a = 0; a < 4; ++a) {
+        if constexpr (DENSE) {
+          put4(u, a, buf_load4(pr, (int)(n * P.p_si * 4) + 4 * (j0 + 8 * a)));
+        } else {
+          put4(u, a, buf_load4(ar, 4 * (j0 + 8 * a)));
+          const float4 t = buf_load4(rr, 4 * (q - j0 - 8 * a - 3));
+          put4(w, a, make_float4(t.w, t.z, t.y, t.x));
+        }
+      }
+    } else {
 #pragma unroll
-    for (int c = 0; c < DPT; ++c) o[i][c] = 0.f;
-  for (int jb = 0; jb < nkb; ++jb) {
-    const int j0 = jb * BK;
-    __syncthreads();
-    load_rows<BK, HD, LD>(vs, vbase, p.v_st, j0, T_len, tid);
-#pragma unroll
-    for (int i = 0; i < RPT; ++i)
-#pragma unroll
-      for (int c = 0; c < RPT; ++c)
-        ps[tr * RPT + i][tc + 16 * c] = P(q0 + tr * RPT + i, j0 + tc + 16 * c, T_len);
-    __syncthreads();
-    for (int kk = 0; kk < BK; ++kk) {
-      float vv[DPT];
-#pragma unroll
-      for (int c = 0; c < DPT; ++c) vv[c] = vs[kk][tc + 16 * c];
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const float pv = ps[tr * RPT + i][kk];
-#pragma unroll
-        for (int c = 0; c < DPT; ++c) o[i][c] = fmaf(pv, vv[c], o[i][c]);
+      for (int i = 0; i < 16; ++i) {
+        const int j = kR * jb + acc_row(i, g);
+        if constexpr (DENSE) {
+          u[i] = P.cell(q, j);
+        } else {
+          u[i] = P.alpha_at(j);
+          w[i] = P.rho_at(q - j);
+        }
       }
     }
-  }
+    SAF_PIN();
+  };
+  auto lim = [&](int jb) { return jb <= qt ? T_len : 0; };
+  if (wave <= qt) fetch(wave);
+  vf.load(vbase, p.v_st, kR * wave, lim(wave), vo);
+  const float zq = DENSE ? 0.f : P.z_at(q);
+  f32x16_t o[NE];
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int row = q0 + tr * RPT + i;
-    if (row >= T_len) continue;
+  for (int e = 0; e < NE; ++e) o[e] = zero16();
+  for (int jb = wave; jb <= qt; jb += kW) {
+    float x[16];
 #pragma unroll
-    for (int c = 0; c < DPT; ++c) obase[(int64_t)row * p.o_st + tc + 16 * c] = o[i][c];
+    for (int i = 0; i < 16; ++i) x[i] = DENSE ? u[i] : FrozenCells::prob(u[i], w[i], zq);
+    if (jb == qt) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = kR * jb + acc_row(i, g) <= q ? x[i] : 0.f;
+    }
+    if (jb + kW <= qt) fetch(jb + kW);
+    vf.axpy(o, x, p.v_st, vo);
+    vf.load(vbase, p.v_st, kR * (jb + kW), lim(jb + kW), vo);
   }
+  put_tile<HD>(sm, o, 1.f, wave, lane);
+  __syncthreads();
+  store_sum<HD>(sm, reinterpret_cast<float*>(p.out) + b * p.o_sb + (int64_t)p.out_head[slot] * p.o_sh, p.o_st, q0,
+                T_len, 1.f, nullptr, tid);
 }
 
 // ---- backward ------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void f32_bwd_delta_kernel(const BwdParams p, const int HD) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t rows = (int64_t)p.B * p.n_live * p.T;
-  if (idx >= rows) return;
-  const int row = (int)(idx % p.T);
-  const int slot = (int)((idx / p.T) % p.n_live);
-  const int b = (int)(idx / ((int64_t)p.T * p.n_live));
-  const int h = p.out_head[slot];
-  const float* o = reinterpret_cast<const float*>(p.out) + b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_st;
-  const float* g = reinterpret_cast<const float*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh + (int64_t)row * p.do_st;
-  float acc = 0.f;
-  for (int d = 0; d < HD; ++d) acc = fmaf(o[d], g[d], acc);
-  p.delta[idx] = acc;
-}
+// Waves per SIMD of the dQ and dK / dV kernels: two up to hd 64 (left to the
+// compiler they took 270 to 340 registers and ran one), so one wave's softmax
+// and loads run beside the other's products.
+constexpr int f32_bwd_waves(int hd) { return hd <= 64 ? 2 : 1; }
 
+// dQ of one query tile; its prologue forms delta = rowsum(out * dout) of the
+// tile's rows and stores it for the dK / dV kernel, which runs after it.
 template <int HD>
-__global__ __launch_bounds__(256) void f32_bwd_dq_kernel(const BwdParams p) {
-  using Tl = F32Tile<HD>;
-  constexpr int BQ = Tl::B, BK = Tl::B, RPT = Tl::RPT, DPT = Tl::DPT, LD = Tl::LD;
-  __shared__ __align__(16) float qs[BQ][LD];
-  __shared__ __align__(16) float gs[BQ][LD];
-  __shared__ __align__(16) float ks[BK][LD];
-  __shared__ __align__(16) float vs[BK][LD];
-  __shared__ float ds_[BQ][BK + 1];
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  const int nqb = (p.T + BQ - 1) / BQ;
-  const int qb = nqb - 1 - (int)blockIdx.x;
-  const int slot = blockIdx.y, b = blockIdx.z;
-  const int h = p.out_head[slot], qs_h = p.q_head[slot];
-  const float* qbase = reinterpret_cast<const float*>(p.q) + b * p.q_sb + (int64_t)qs_h * p.q_sh;
-  const float* kbase = reinterpret_cast<const float*>(p.k) + b * p.k_sb + (int64_t)qs_h * p.k_sh;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_bwd_waves(HD), f32_bwd_waves(HD))))
+void f32_bwd_dq_kernel(const BwdParams p) {
+  using Sh = F32Shape<HD>;
+  constexpr int NE = Sh::NE, NT = Sh::NT;
+  __shared__ __align__(16) float sm[Sh::MERGE > 2 * Sh::FRAG ? Sh::MERGE : 2 * Sh::FRAG];
+  __shared__ float sm_d[kW][kR];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T_len = p.T, nqt = (T_len + kR - 1) / kR, nbh = p.B * p.n_live;
+  const int qt = nqt - 1 - (int)(blockIdx.x / nbh);
+  const int bh = (int)(blockIdx.x % nbh);
+  const int b = bh / p.n_live, slot = bh % p.n_live;
+  const int h = p.out_head[slot], qs = p.q_head[slot], q0 = qt * kR, q = q0 + n;
+  const float* kbase = reinterpret_cast<const float*>(p.k) + b * p.k_sb + (int64_t)qs * p.k_sh;
   const float* vbase = reinterpret_cast<const float*>(p.v) + b * p.v_sb + (int64_t)h * p.v_sh;
-  const float* gbase = reinterpret_cast<const float*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh;
-  float* dqbase = reinterpret_cast<float*>(p.dq) + b * p.dq_sb + (int64_t)qs_h * p.dq_sh;
-  const float* delta = p.delta + ((int64_t)b * p.n_live + slot) * p.T;
-  const int T_len = p.T, q0 = qb * BQ;
-  const int nkb = (min(q0 + BQ, T_len) + BK - 1) / BK;
-  load_rows<BQ, HD, LD>(qs, qbase, p.q_st, q0, T_len, tid);
-  load_rows<BQ, HD, LD>(gs, gbase, p.do_st, q0, T_len, tid);
-  float lse[RPT], dl[RPT], acc[RPT][DPT];
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int row = q0 + tr * RPT + i;
-    lse[i] = row < T_len ? p.lse[b * p.l_sb + (int64_t)h * p.l_sh + (int64_t)row * p.l_st] : 0.f;
-    dl[i] = row < T_len ? delta[row] : 0.f;
-#pragma unroll
-    for (int c = 0; c < DPT; ++c) acc[i][c] = 0.f;
-  }
-  for (int jb = 0; jb < nkb; ++jb) {
-    const int j0 = jb * BK;
-    __syncthreads();
-    load_rows<BK, HD, LD>(ks, kbase, p.k_st, j0, T_len, tid);
-    load_rows<BK, HD, LD>(vs, vbase, p.v_st, j0, T_len, tid);
-    __syncthreads();
-    float s[RPT][RPT], dp[RPT][RPT];
-    dots<RPT, RPT, HD, LD>(s, qs, tr * RPT, ks, tc);
-    dots<RPT, RPT, HD, LD>(dp, gs, tr * RPT, vs, tc);
-#pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const int row = q0 + tr * RPT + i;
-#pragma unroll
-      for (int c = 0; c < RPT; ++c) {
-        const int key = j0 + tc + 16 * c;
-        const float pr = (key <= row && row < T_len && key < T_len) ? fast_exp2(s[i][c] * p.scale_log2 - lse[i]) : 0.f;
-        ds_[tr * RPT + i][tc + 16 * c] = pr * (dp[i][c] - dl[i]);
-      }
+  float4* const qf = reinterpret_cast<float4*>(sm);
+  float4* const gf = reinterpret_cast<float4*>(sm + Sh::FRAG);
+  stage_tile<HD>(qf, reinterpret_cast<const float*>(p.q) + b * p.q_sb + (int64_t)qs * p.q_sh, p.q_st, q0, T_len, wave,
+                 lane);
+  const int ko = row_off(p.k_st, lane), vo = row_off(p.v_st, lane), co = col_off<HD>(p.k_st, lane);
+  auto lim = [&](int jb) { return jb <= qt ? T_len : 0; };
+  RowFrag<HD> kf, vf;
+  ColFrag<HD> kc;
+  {
+    const __amdgpu_buffer_rsrc_t gr =
+        rows_rsrc(reinterpret_cast<const float*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh, p.do_st, q0, T_len);
+    const __amdgpu_buffer_rsrc_t orr =
+        rows_rsrc(reinterpret_cast<const float*>(p.out) + b * p.o_sb + (int64_t)h * p.o_sh, p.o_st, q0, T_len);
+    float acc = 0.f;
+    for (int t = wave; t < NT; t += kW) {
+      const float4 d = buf_load4(gr, row_off(p.do_st, lane) + 32 * t);
+      const float4 y = buf_load4(orr, row_off(p.o_st, lane) + 32 * t);
+      gf[t * 64 + lane] = d;
+      acc = fmaf(d.x, y.x, fmaf(d.y, y.y, fmaf(d.z, y.z, fmaf(d.w, y.w, acc))));
     }
-    __syncthreads();
-    for (int kk = 0; kk < BK; ++kk) {
-      float kv[DPT];
+    acc = half_swap_sum(acc);
+    if (g == 0) sm_d[wave][n] = acc;
+  }
+  kf.load(kbase, p.k_st, kR * wave, lim(wave), ko);
+  vf.load(vbase, p.v_st, kR * wave, lim(wave), vo);
+  const float lse =
+      q < T_len ? p.lse[b * p.l_sb + (int64_t)h * p.l_sh + (int64_t)q * p.l_st] : 0.f;
+  __syncthreads();
+  const float dl = (sm_d[0][n] + sm_d[1][n]) + (sm_d[2][n] + sm_d[3][n]);
+  if (wave == 0 && g == 0 && q < T_len) p.delta[((int64_t)b * p.n_live + slot) * T_len + q] = dl;
+  f32x16_t acc[NE];
 #pragma unroll
-      for (int c = 0; c < DPT; ++c) kv[c] = ks[kk][tc + 16 * c];
+  for (int e = 0; e < NE; ++e) acc[e] = zero16();
+  for (int jb = wave; jb <= qt; jb += kW) {
+    const f32x16_t s = kf.dot(qf, lane, ko, zero16());
+    kc.load(kbase, p.k_st, kR * jb, T_len, co);
+    const f32x16_t dp = vf.dot(gf, lane, vo, zero16());
+    kf.load(kbase, p.k_st, kR * (jb + kW), lim(jb + kW), ko);
+    float x[16];
 #pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const float d = ds_[tr * RPT + i][kk];
+    for (int i = 0; i < 16; ++i) x[i] = s[i] * p.scale_log2 - lse;
+    if (jb == qt) {
 #pragma unroll
-        for (int c = 0; c < DPT; ++c) acc[i][c] = fmaf(d, kv[c], acc[i][c]);
-      }
+      for (int i = 0; i < 16; ++i) x[i] = (q < T_len && kR * jb + acc_row(i, g) <= q) ? x[i] : -INFINITY;
     }
-  }
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int row = q0 + tr * RPT + i;
-    if (row >= T_len) continue;
-#pragma unroll
-    for (int c = 0; c < DPT; ++c) dqbase[(int64_t)row * p.dq_st + tc + 16 * c] = acc[i][c] * p.sm_scale;
+    for (int i = 0; i < 16; ++i) x[i] = fast_exp2(x[i]) * (dp[i] - dl);
+    kc.axpy(acc, x, p.k_st, co);
+    vf.load(vbase, p.v_st, kR * (jb + kW), lim(jb + kW), vo);
   }
+  __syncthreads();
+  put_tile<HD>(sm, acc, 1.f, wave, lane);
+  __syncthreads();
+  store_sum<HD>(sm, reinterpret_cast<float*>(p.dq) + b * p.dq_sb + (int64_t)qs * p.dq_sh, p.dq_st, q0, T_len,
+                p.sm_scale, nullptr, tid);
 }
 
-// dK / dV of live heads (one workgroup per key block) and dV of frozen heads
-// (FROZEN: P from the pattern, no dK)
-template <int HD, bool FROZEN>
-__global__ __launch_bounds__(256) void f32_bwd_kv_kernel(const BwdParams p) {
-  using Tl = F32Tile<HD>;
-  constexpr int BQ = Tl::B, BK = Tl::B, RPT = Tl::RPT, DPT = Tl::DPT, LD = Tl::LD;
-  __shared__ __align__(16) float ks[FROZEN ? 1 : BK][LD];
-  __shared__ __align__(16) float vs[FROZEN ? 1 : BK][LD];
-  __shared__ __align__(16) float qs[FROZEN ? 1 : BQ][LD];
-  __shared__ __align__(16) float gs[BQ][LD];
-  __shared__ float pt[BK][BQ + 1];  // P^T, then dS^T, of the current query block
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  const int nkb = (p.T + BK - 1) / BK;
-  const int kb = nkb - 1 - (int)blockIdx.x;
-  const int slot = blockIdx.y, b = blockIdx.z;
-  const int T_len = p.T, k0 = kb * BK;
-  const int nqb = (T_len + BQ - 1) / BQ;
-  int h, qs_h = 0;
-  FrozenP P{};
-  if constexpr (FROZEN) {
-    h = p.f_head[slot];
-    const int ph = p.pat_head[slot];
-    P.kind = p.f_kind[slot];
-    P.patt = p.patt; P.patt_dtype = p.patt_dtype;
-    P.prow0 = (int64_t)ph * p.p_sh; P.p_si = p.p_si; P.p_sj = p.p_sj;
-    P.alpha = p.alpha; P.rho = p.rho; P.z = p.z;
-    P.a_dtype = p.a_dtype; P.r_dtype = p.r_dtype; P.z_dtype = p.z_dtype;
-    P.a0 = (int64_t)ph * p.a_sh; P.a_ss = p.a_ss;
-    P.r0 = (int64_t)ph * p.r_sh; P.r_ss = p.r_ss;
-    P.z0 = (int64_t)ph * p.z_sh; P.z_ss = p.z_ss;
-  } else {
-    h = p.out_head[slot];
-    qs_h = p.q_head[slot];
-  }
+// dK / dV of one key tile of a live head: S = Q K^T and dP = dO V^T with the
+// keys in the lanes, so the query's LSE and delta are per register.
+template <int HD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(f32_bwd_waves(HD), f32_bwd_waves(HD))))
+void f32_bwd_kv_kernel(const BwdParams p) {
+  using Sh = F32Shape<HD>;
+  constexpr int NE = Sh::NE;
+  __shared__ __align__(16) float sm[Sh::MERGE > 2 * Sh::FRAG ? Sh::MERGE : 2 * Sh::FRAG];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T_len = p.T, nqt = (T_len + kR - 1) / kR, nbh = p.B * p.n_live;
+  const int kt = (int)(blockIdx.x / nbh);  // heaviest (most queries) first
+  const int bh = (int)(blockIdx.x % nbh);
+  const int b = bh / p.n_live, slot = bh % p.n_live;
+  const int h = p.out_head[slot], qs = p.q_head[slot], k0 = kt * kR, key = k0 + n;
+  const float* qbase = reinterpret_cast<const float*>(p.q) + b * p.q_sb + (int64_t)qs * p.q_sh;
   const float* gbase = reinterpret_cast<const float*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh;
-  const float* qbase = FROZEN ? nullptr : reinterpret_cast<const float*>(p.q) + b * p.q_sb + (int64_t)qs_h * p.q_sh;
-  const float* delta = FROZEN ? nullptr : p.delta + ((int64_t)b * p.n_live + slot) * p.T;
-  if constexpr (!FROZEN) {
-    load_rows<BK, HD, LD>(ks, reinterpret_cast<const float*>(p.k) + b * p.k_sb + (int64_t)qs_h * p.k_sh, p.k_st, k0,
-                          T_len, tid);
-    load_rows<BK, HD, LD>(vs, reinterpret_cast<const float*>(p.v) + b * p.v_sb + (int64_t)h * p.v_sh, p.v_st, k0,
-                          T_len, tid);
+  const float* lse = p.lse + b * p.l_sb + (int64_t)h * p.l_sh;
+  const float* delta = p.delta + ((int64_t)b * p.n_live + slot) * T_len;
+  float4* const kf = reinterpret_cast<float4*>(sm);
+  float4* const vf = reinterpret_cast<float4*>(sm + Sh::FRAG);
+  stage_tile<HD>(kf, reinterpret_cast<const float*>(p.k) + b * p.k_sb + (int64_t)qs * p.k_sh, p.k_st, k0, T_len, wave,
+                 lane);
+  stage_tile<HD>(vf, reinterpret_cast<const float*>(p.v) + b * p.v_sb + (int64_t)h * p.v_sh, p.v_st, k0, T_len, wave,
+                 lane);
+  const int qo = row_off(p.q_st, lane), go = row_off(p.do_st, lane);
+  const int qco = col_off<HD>(p.q_st, lane), gco = col_off<HD>(p.do_st, lane);
+  auto lim = [&](int ib) { return ib < nqt ? T_len : 0; };
+  RowFrag<HD> qr, gr;
+  ColFrag<HD> qc, gc;
+  qr.load(qbase, p.q_st, kR * (kt + wave), lim(kt + wave), qo);
+  gr.load(gbase, p.do_st, kR * (kt + wave), lim(kt + wave), go);
+  __syncthreads();
+  f32x16_t dk[NE], dv[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    dk[e] = zero16();
+    dv[e] = zero16();
   }
-  float dv[RPT][DPT], dk[RPT][DPT];
+  for (int ib = kt + wave; ib < nqt; ib += kW) {
+    // dP's chain starts from -delta of each register's query
+    float ls[16], dl[16];
+    load_stat(ls, lse, p.l_st, kR * ib, T_len, g);
+    load_stat(dl, delta, 1, kR * ib, T_len, g);
+    const f32x16_t s = qr.dot(kf, lane, qo, zero16());
+    gc.load(gbase, p.do_st, kR * ib, T_len, gco);
+    f32x16_t dp;
 #pragma unroll
-  for (int i = 0; i < RPT; ++i)
+    for (int i = 0; i < 16; ++i) dp[i] = -dl[i];
+    dp = gr.dot(vf, lane, go, dp);
+    qc.load(qbase, p.q_st, kR * ib, T_len, qco);
+    float x[16], y[16];
 #pragma unroll
-    for (int c = 0; c < DPT; ++c) dv[i][c] = dk[i][c] = 0.f;
-  for (int qb = k0 / BQ; qb < nqb; ++qb) {
-    const int q0 = qb * BQ;
-    __syncthreads();
-    load_rows<BQ, HD, LD>(gs, gbase, p.do_st, q0, T_len, tid);
-    if constexpr (!FROZEN) load_rows<BQ, HD, LD>(qs, qbase, p.q_st, q0, T_len, tid);
-    __syncthreads();
-    // thread (tr, tc): keys k0 + tr * RPT + i, queries q0 + tc + 16 c
-    float s[RPT][RPT], dp[RPT][RPT];
-    if constexpr (FROZEN) {
+    for (int i = 0; i < 16; ++i) x[i] = s[i] * p.scale_log2 - ls[i];
+    if (ib == kt || ib == nqt - 1) {
 #pragma unroll
-      for (int i = 0; i < RPT; ++i)
+      for (int i = 0; i < 16; ++i) {
+        const int q = kR * ib + acc_row(i, g);
+        x[i] = (key <= q && q < T_len) ? x[i] : -INFINITY;
+      }
+    }
 #pragma unroll
-        for (int c = 0; c < RPT; ++c) s[i][c] = P(q0 + tc + 16 * c, k0 + tr * RPT + i, T_len);
+    for (int i = 0; i < 16; ++i) {
+      x[i] = fast_exp2(x[i]);
+      y[i] = x[i] * dp[i];
+    }
+    gc.axpy(dv, x, p.do_st, gco);
+    qr.load(qbase, p.q_st, kR * (ib + kW), lim(ib + kW), qo);
+    qc.axpy(dk, y, p.q_st, qco);
+    gr.load(gbase, p.do_st, kR * (ib + kW), lim(ib + kW), go);
+  }
+  __syncthreads();
+  put_tile<HD>(sm, dv, 1.f, wave, lane);
+  __syncthreads();
+  store_sum<HD>(sm, reinterpret_cast<float*>(p.dv) + b * p.dv_sb + (int64_t)h * p.dv_sh, p.dv_st, k0, T_len, 1.f,
+                nullptr, tid);
+  __syncthreads();
+  put_tile<HD>(sm, dk, 1.f, wave, lane);
+  __syncthreads();
+  store_sum<HD>(sm, reinterpret_cast<float*>(p.dk) + b * p.dk_sb + (int64_t)qs * p.dk_sh, p.dk_st, k0, T_len,
+                p.sm_scale, nullptr, tid);
+}
+
+// dV = P^T dO of one key tile of a frozen head (KIND 1 dense, 2 decomposed).
+template <int HD, int KIND, bool FAST>
+__global__ __launch_bounds__(256) void f32_bwd_frozen_kernel(const BwdParams p) {
+  using Sh = F32Shape<HD>;
+  constexpr int NE = Sh::NE;
+  __shared__ __align__(16) float sm[Sh::MERGE];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T_len = p.T, nqt = (T_len + kR - 1) / kR, nbf = p.B * p.n_frozen;
+  const int kt = (int)(blockIdx.x / nbf);
+  const int bf = (int)(blockIdx.x % nbf);
+  const int b = bf / p.n_frozen, fs = bf % p.n_frozen;
+  if (p.f_kind[fs] != KIND) return;
+  const int h = p.f_head[fs], k0 = kt * kR, key = k0 + n;
+  const float* gbase = reinterpret_cast<const float*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh;
+  FrozenCells P;
+  P.init(p, p.pat_head[fs]);
+  const int gco = col_off<HD>(p.do_st, lane);
+  ColFrag<HD> gc;
+  float u[16], w[16];  // dense: pattern cells; decomposed: rho_{i-key} and z_i
+  const __amdgpu_buffer_rsrc_t rr = P.vec(P.rho, P.r0), zr = P.vec(P.z, P.z0);
+  auto fetch = [&](int ib) {
+    const int i0 = kR * ib + 4 * g;  // queries i0 + 8a + r
+    if (FAST && KIND == 1) {
+      const __amdgpu_buffer_rsrc_t pr = P.rows(kR * ib);
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        u[i] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(pr, acc_row(i, g) * (int)(P.p_si * 4) + 4 * key, 0, 0));
+    } else if (FAST && ib > kt) {  // every distance is >= 1
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        put4(u, a, buf_load4(rr, 4 * (i0 + 8 * a - key)));
+        put4(w, a, buf_load4(zr, 4 * (i0 + 8 * a)));
+      }
     } else {
-      dots<RPT, RPT, HD, LD>(s, ks, tr * RPT, qs, tc);
-      dots<RPT, RPT, HD, LD>(dp, vs, tr * RPT, gs, tc);
 #pragma unroll
-      for (int i = 0; i < RPT; ++i)
-#pragma unroll
-        for (int c = 0; c < RPT; ++c) {
-          const int key = k0 + tr * RPT + i, q = q0 + tc + 16 * c;
-          const float lse = q < T_len ? p.lse[b * p.l_sb + (int64_t)h * p.l_sh + (int64_t)q * p.l_st] : 0.f;
-          s[i][c] = (key <= q && q < T_len && key < T_len) ? fast_exp2(s[i][c] * p.scale_log2 - lse) : 0.f;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < RPT; ++i)
-#pragma unroll
-      for (int c = 0; c < RPT; ++c) pt[tr * RPT + i][tc + 16 * c] = s[i][c];
-    __syncthreads();
-    // dV[key] += sum_q P[q, key] dO[q]
-    for (int qq = 0; qq < BQ; ++qq) {
-      float gv[DPT];
-#pragma unroll
-      for (int c = 0; c < DPT; ++c) gv[c] = gs[qq][tc + 16 * c];
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const float pv = pt[tr * RPT + i][qq];
-#pragma unroll
-        for (int c = 0; c < DPT; ++c) dv[i][c] = fmaf(pv, gv[c], dv[i][c]);
-      }
-    }
-    if constexpr (!FROZEN) {
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < RPT; ++i)
-#pragma unroll
-        for (int c = 0; c < RPT; ++c) {
-          const int q = q0 + tc + 16 * c;
-          pt[tr * RPT + i][tc + 16 * c] = s[i][c] * (dp[i][c] - (q < T_len ? delta[q] : 0.f));
-        }
-      __syncthreads();
-      // dK[key] += sum_q dS[q, key] Q[q]
-      for (int qq = 0; qq < BQ; ++qq) {
-        float qv[DPT];
-#pragma unroll
-        for (int c = 0; c < DPT; ++c) qv[c] = qs[qq][tc + 16 * c];
-#pragma unroll
-        for (int i = 0; i < RPT; ++i) {
-          const float d = pt[tr * RPT + i][qq];
-#pragma unroll
-          for (int c = 0; c < DPT; ++c) dk[i][c] = fmaf(d, qv[c], dk[i][c]);
+      for (int i = 0; i < 16; ++i) {
+        const int q = kR * ib + acc_row(i, g);
+        if constexpr (KIND == 1) {
+          u[i] = P.cell(q, key);
+        } else {
+          u[i] = P.rho_at(q - key);
+          w[i] = P.z_at(q);
         }
       }
     }
-  }
-  float* dvbase = reinterpret_cast<float*>(p.dv) + b * p.dv_sb + (int64_t)h * p.dv_sh;
-  float* dkbase = FROZEN ? nullptr : reinterpret_cast<float*>(p.dk) + b * p.dk_sb + (int64_t)qs_h * p.dk_sh;
+    SAF_PIN();
+  };
+  auto lim = [&](int ib) { return ib < nqt ? T_len : 0; };
+  if (kt + wave < nqt) fetch(kt + wave);
+  gc.load(gbase, p.do_st, kR * (kt + wave), lim(kt + wave), gco);
+  const float ak = KIND == 1 ? 0.f : P.alpha_at(key);
+  f32x16_t dv[NE];
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int key = k0 + tr * RPT + i;
-    if (key >= T_len) continue;
+  for (int e = 0; e < NE; ++e) dv[e] = zero16();
+  for (int ib = kt + wave; ib < nqt; ib += kW) {
+    float x[16];
 #pragma unroll
-    for (int c = 0; c < DPT; ++c) {
-      dvbase[(int64_t)key * p.dv_st + tc + 16 * c] = dv[i][c];
-      if constexpr (!FROZEN) dkbase[(int64_t)key * p.dk_st + tc + 16 * c] = dk[i][c] * p.sm_scale;
+    for (int i = 0; i < 16; ++i) x[i] = KIND == 1 ? u[i] : FrozenCells::prob(ak, u[i], w[i]);
+    if (ib == kt || ib == nqt - 1) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int q = kR * ib + acc_row(i, g);
+        x[i] = (key <= q && q < T_len) ? x[i] : 0.f;
+      }
     }
+    if (ib + kW < nqt) fetch(ib + kW);
+    gc.axpy(dv, x, p.do_st, gco);
+    gc.load(gbase, p.do_st, kR * (ib + kW), lim(ib + kW), gco);
   }
+  put_tile<HD>(sm, dv, 1.f, wave, lane);
+  __syncthreads();
+  store_sum<HD>(sm, reinterpret_cast<float*>(p.dv) + b * p.dv_sb + (int64_t)h * p.dv_sh, p.dv_st, k0, T_len, 1.f,
+                nullptr, tid);
+}
+
+// FAST pattern reads: fp32 buffers, unit inner strides, a pattern row pitch
+// that 32-bit offsets of a row block can hold.
+template <typename P>
+bool cells_fast(const P& p, bool dense) {
+  if (dense)
+    return p.patt_dtype == kF32 && p.p_sj == 1 && p.p_si >= 0 && p.p_si * 4 < kMaxRowBytes;
+  return p.a_dtype == kF32 && p.r_dtype == kF32 && p.z_dtype == kF32 && p.a_ss == 1 && p.r_ss == 1 && p.z_ss == 1;
 }
 
 template <int HD>
 hipError_t f32_fwd_hd(const FlashParams* fp, const FrozenParams* zp, int mode, hipStream_t s) {
-  constexpr int B = F32Tile<HD>::B;
   if (fp != nullptr) {
-    const dim3 grid((unsigned)((fp->T + B - 1) / B), (unsigned)fp->n_slots, (unsigned)fp->B);
-    hipLaunchKernelGGL((f32_live_kernel<HD>), grid, dim3(256), 0, s, *fp);
+    const dim3 grid((unsigned)((int64_t)((fp->T + kR - 1) / kR) * fp->n_slots * fp->B));
+    hipLaunchKernelGGL((f32_live_kernel<HD>), grid, dim3(64 * kW), 0, s, *fp);
   } else {
-    const dim3 grid((unsigned)((zp->T + B - 1) / B), (unsigned)zp->n_slots, (unsigned)zp->B);
-    hipLaunchKernelGGL((f32_frozen_kernel<HD>), grid, dim3(256), 0, s, *zp, mode);
+    const dim3 grid((unsigned)((int64_t)((zp->T + kR - 1) / kR) * zp->n_slots * zp->B));
+    const bool fast = cells_fast(*zp, mode == 0);
+    if (mode == 0 && fast)
+      hipLaunchKernelGGL((f32_frozen_kernel<HD, true, true>), grid, dim3(64 * kW), 0, s, *zp);
+    else if (mode == 0)
+      hipLaunchKernelGGL((f32_frozen_kernel<HD, true, false>), grid, dim3(64 * kW), 0, s, *zp);
+    else if (fast)
+      hipLaunchKernelGGL((f32_frozen_kernel<HD, false, true>), grid, dim3(64 * kW), 0, s, *zp);
+    else
+      hipLaunchKernelGGL((f32_frozen_kernel<HD, false, false>), grid, dim3(64 * kW), 0, s, *zp);
   }
   return hipGetLastError();
 }
 
 template <int HD>
 hipError_t f32_bwd_hd(const BwdParams& p, int which, hipStream_t s) {
-  constexpr int B = F32Tile<HD>::B;
-  const unsigned nb = (unsigned)((p.T + B - 1) / B);
+  const int64_t nt = (p.T + kR - 1) / kR;
+  const dim3 live((unsigned)(nt * p.n_live * p.B)), frozen((unsigned)(nt * p.n_frozen * p.B));
   switch (which) {
-    case 0: {
-      const int64_t rows = (int64_t)p.B * p.n_live * p.T;
-      hipLaunchKernelGGL(f32_bwd_delta_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, p, HD);
+    case 0:  // delta comes out of the dQ kernel
       break;
-    }
     case 1:
-      hipLaunchKernelGGL((f32_bwd_dq_kernel<HD>), dim3(nb, (unsigned)p.n_live, (unsigned)p.B), dim3(256), 0, s, p);
+      hipLaunchKernelGGL((f32_bwd_dq_kernel<HD>), live, dim3(64 * kW), 0, s, p);
       break;
     case 2:
-      hipLaunchKernelGGL((f32_bwd_kv_kernel<HD, false>), dim3(nb, (unsigned)p.n_live, (unsigned)p.B), dim3(256), 0,
-                         s, p);
+      hipLaunchKernelGGL((f32_bwd_kv_kernel<HD>), live, dim3(64 * kW), 0, s, p);
       break;
-    default:
-      hipLaunchKernelGGL((f32_bwd_kv_kernel<HD, true>), dim3(nb, (unsigned)p.n_frozen, (unsigned)p.B), dim3(256), 0,
-                         s, p);
+    default: {
+      bool kind[3] = {false, false, false};
+      for (int i = 0; i < p.n_frozen; ++i) kind[p.f_kind[i]] = true;
+      if (kind[1] && cells_fast(p, true))
+        hipLaunchKernelGGL((f32_bwd_frozen_kernel<HD, 1, true>), frozen, dim3(64 * kW), 0, s, p);
+      else if (kind[1])
+        hipLaunchKernelGGL((f32_bwd_frozen_kernel<HD, 1, false>), frozen, dim3(64 * kW), 0, s, p);
+      if (kind[2] && cells_fast(p, false))
+        hipLaunchKernelGGL((f32_bwd_frozen_kernel<HD, 2, true>), frozen, dim3(64 * kW), 0, s, p);
+      else if (kind[2])
+        hipLaunchKernelGGL((f32_bwd_frozen_kernel<HD, 2, false>), frozen, dim3(64 * kW), 0, s, p);
       break;
+    }
   }
   return hipGetLastError();
 }

@@ -315,7 +315,8 @@ hipError_t launch_bwd_frozen_dv(const BwdParams& p, int dtype, int hd, hipStream
 hipError_t launch_bwd_decomp_param(const BwdParams& p, int dtype, int hd, hipStream_t s);
 
 // float32 inputs (attn_f32.hip): the same parameter blocks, no causal split
-// (n_items 0), no work queue; which: 0 delta, 1 dQ, 2 dK / dV, 3 frozen dV.
+// (n_items 0), no work queue; which: 0 nothing (the dQ kernel writes delta),
+// 1 dQ and delta, 2 dK / dV, 3 frozen dV.
 hipError_t launch_f32_live(const FlashParams& p, int hd, hipStream_t s);
 hipError_t launch_f32_frozen(const FrozenParams& p, int hd, int mode, hipStream_t s);
 hipError_t launch_f32_bwd(const BwdParams& p, int hd, int which, hipStream_t s);
