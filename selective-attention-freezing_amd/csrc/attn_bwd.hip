@@ -68,7 +68,11 @@ struct TileOffsets {
   }
   // rows r0 .. r0+63 of a (T_len, st) tensor at base; rows >= T_len read zero
   __device__ __forceinline__ void load(const T* base, int64_t st, int r0, int T_len, char* tile, int wave) const {
-    const __amdgpu_buffer_rsrc_t r = rows_rsrc(base, st, r0, T_len);
+    load_span(base + (int64_t)r0 * st, (int64_t)(T_len - r0) * st * (int64_t)sizeof(T), tile, wave);
+  }
+  // the tile whose first row is at base, which may read `bytes` bytes
+  __device__ __forceinline__ void load_span(const T* base, int64_t bytes, char* tile, int wave) const {
+    const __amdgpu_buffer_rsrc_t r = span_rsrc(base, bytes);
 #pragma unroll
     for (int pp = 0; pp < VN; ++pp)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, SAF_LDS_PTR(tile + (kBwdWaves * pp + wave) * 1024), 16, off[pp], 0,
@@ -455,13 +459,12 @@ void bwd_dkdv_kernel(const BwdParams p) {
   }
 }
 
-// dV of the frozen heads: dV[j] = sum_{i >= j} P[i, j] dO[i].  Workgroup =
-// 4 waves x 32 keys of one (batch, frozen slot); query blocks of 64 from the
-// diagonal.  The B operand of dV^T += dO^T P is a column of P for 8
-// consecutive queries: gathered from the dense pattern (rounded to the
-// activation dtype) or rebuilt as P[i, j] = 2^((alpha_j + rho_{i-j} - z_i)
-// log2 e) for decomposed heads (closed-form heads included); cells with
-// i < j or i >= T are zero.
+// dV of the decomposed frozen heads (closed-form heads included): dV[j] =
+// sum_{i >= j} P[i, j] dO[i].  Workgroup = 4 waves x 32 keys of one (batch,
+// frozen slot); query blocks of 64 from the diagonal.  The B operand of
+// dV^T += dO^T P is a column of P for 8 consecutive queries, rebuilt as
+// P[i, j] = 2^((alpha_j + rho_{i-j} - z_i) log2 e); cells with i < j or
+// i >= T are zero.
 //
 // dO tiles arrive by DMA two blocks ahead in three static LDS slots (an
 // empty descriptor past the last block, so every block issues the same
@@ -469,8 +472,8 @@ void bwd_dkdv_kernel(const BwdParams p) {
 // block ahead, before that DMA, and written into the next block's slot.  The
 // block ends with a counted wait (the DMA two ahead stays in flight) and a
 // bare barrier: one barrier per block instead of two draining ones.
-template <typename T, int HD, int KIND>
-__global__ __launch_bounds__(256) void bwd_frozen_dv_kernel(const BwdParams p) {
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void bwd_decomp_dv_kernel(const BwdParams p) {
   constexpr int BN = kBwdWaves * 32, NDT = HD / 32, VB = VRow<HD>::BYTES;
   constexpr int VN = TileOffsets<T, HD>::VN;  // DMA loads per wave per dO tile
   __shared__ __align__(16) char o0[VB], o1[VB], o2[VB];
@@ -485,7 +488,7 @@ __global__ __launch_bounds__(256) void bwd_frozen_dv_kernel(const BwdParams p) {
   const int r = blockIdx.x % nbf;
   const int kb = (int)(blockIdx.x / nbf);
   const int b = r / p.n_frozen, fs = r % p.n_frozen;
-  if (p.f_kind[fs] != KIND) return;
+  if (p.f_kind[fs] != 2) return;
   const int h = p.f_head[fs], ph = p.pat_head[fs];
   const T* dobase = reinterpret_cast<const T*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh;
   T* dvbase = reinterpret_cast<T*>(p.dv) + b * p.dv_sb + (int64_t)h * p.dv_sh;
@@ -493,7 +496,7 @@ __global__ __launch_bounds__(256) void bwd_frozen_dv_kernel(const BwdParams p) {
   const int kk = k0w + n;
   const bool kv = kk < T_len;
   float alpha_k = 0.f;
-  if (KIND == 2 && kv) alpha_k = load_as_f32(p.alpha, (int64_t)ph * p.a_sh + (int64_t)kk * p.a_ss, p.a_dtype) * kLog2e;
+  if (kv) alpha_k = load_as_f32(p.alpha, (int64_t)ph * p.a_sh + (int64_t)kk * p.a_ss, p.a_dtype) * kLog2e;
   f32x16_t dva[NDT];
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) dva[dt] = zero16();
@@ -543,11 +546,8 @@ __global__ __launch_bounds__(256) void bwd_frozen_dv_kernel(const BwdParams p) {
     const int dmin = dmin_of(i);
     // the next block's z / rho, then the dO tile two blocks ahead: waiting
     // for the register loads leaves that DMA in flight
-    uint32_t nz = 0u, nr = 0u;
-    if (KIND == 2) {
-      nz = z_bits(64 * (i + 1) + min(tid, 63));
-      nr = rho_bits(dmin + 64 + min(tid, 64 + BN - 2));
-    }
+    const uint32_t nz = z_bits(64 * (i + 1) + min(tid, 63));
+    const uint32_t nr = rho_bits(dmin + 64 + min(tid, 64 + BN - 2));
     asm volatile("" ::: "memory");
     load_do(i + 2, std::integral_constant<int, (R + 2) % 3>());
     asm volatile("" ::: "memory");
@@ -564,19 +564,11 @@ __global__ __launch_bounds__(256) void bwd_frozen_dv_kernel(const BwdParams p) {
         for (int e = 0; e < 8; ++e) {
           const int qq = q0 + 8 * g + e;
           const bool ok = !decltype(masked)::value || (kv && qq >= kk && qq < T_len);
-          float v = 0.f;
-          if (KIND == 1) {
-            if (ok)
-              v = load_as_f32(p.patt, (int64_t)ph * p.p_sh + (int64_t)qq * p.p_si + (int64_t)kk * p.p_sj,
-                              p.patt_dtype);
-          } else {
-            // every (query, key) pair of the block indexes inside the staged
-            // rho window and z row, so the reads need no guard; masked pairs
-            // take exp2(-inf) = 0
-            const float x = alpha_k + rs[qq - kk - dmin] - zs[qq - 64 * i];
-            v = fast_exp2(ok ? x : -__builtin_inff());
-          }
-          e8[e] = v;
+          // every (query, key) pair of the block indexes inside the staged
+          // rho window and z row, so the reads need no guard; masked pairs
+          // take exp2(-inf) = 0
+          const float x = alpha_k + rs[qq - kk - dmin] - zs[qq - 64 * i];
+          e8[e] = fast_exp2(ok ? x : -__builtin_inff());
         }
       };
       if (q0 >= k0w + 31 && k0w + 31 < T_len && q0 + 15 < T_len)
@@ -588,19 +580,16 @@ __global__ __launch_bounds__(256) void bwd_frozen_dv_kernel(const BwdParams p) {
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) dva[dt] = Elem<T>::mfma(tile_col_op<HD>(ot, ks, dt, cof), bop, dva[dt]);
     }
-    if (KIND == 2) {  // the next block's slot was last read two blocks ago
-      constexpr int RN = (R + 1) % 3;
-      if (tid < 64) zs3[RN][tid] = bits_to_f32(nz, p.z_dtype) * kLog2e;
-      if (tid < 64 + BN - 1) rs3[RN][tid] = bits_to_f32(nr, p.r_dtype) * kLog2e;
-    }
+    // the next block's slot was last read two blocks ago
+    constexpr int RN = (R + 1) % 3;
+    if (tid < 64) zs3[RN][tid] = bits_to_f32(nz, p.z_dtype) * kLog2e;
+    if (tid < 64 + BN - 1) rs3[RN][tid] = bits_to_f32(nr, p.r_dtype) * kLog2e;
     meet();
   };
 
   if (ib0 < nqb) {
-    if (KIND == 2) {
-      if (tid < 64) zs3[0][tid] = z_of(64 * ib0 + tid);
-      if (tid < 64 + BN - 1) rs3[0][tid] = rho_of(dmin_of(ib0) + tid);
-    }
+    if (tid < 64) zs3[0][tid] = z_of(64 * ib0 + tid);
+    if (tid < 64 + BN - 1) rs3[0][tid] = rho_of(dmin_of(ib0) + tid);
     asm volatile("" ::: "memory");
     load_do(ib0, std::integral_constant<int, 0>());
     load_do(ib0 + 1, std::integral_constant<int, 1>());
@@ -621,6 +610,174 @@ __global__ __launch_bounds__(256) void bwd_frozen_dv_kernel(const BwdParams p) {
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
   }
   if (kv) store_out_tile<T, HD>(dvbase + (int64_t)kk * p.dv_st, dva, 1.f, g);
+}
+
+// dV of the dense frozen heads, dV[j] = sum_{i >= j} P[i, j] dO[i].  The
+// contraction runs down P's columns while P is stored by rows, so the
+// workgroup (4 waves x 32 keys) stages each 64 x 128 block of P in LDS in the
+// VRow layout, in the activation dtype, and reads its B operands (8
+// consecutive queries of a lane's key) with the same transposing reads that
+// give dO's columns.  How P gets there (PM):
+//   0  pattern in the activation dtype with 16-byte rows: DMA two blocks
+//      ahead in three slots, like dO
+//   1  fp32 pattern with 16-byte rows (the model's default storage): eight
+//      16-byte loads per thread two blocks ahead, rounded and written one
+//      block ahead
+//   2  any other storage type or stride: element loads, as 1
+// Cells with i < j (the buffer may hold anything there) are cleared in the
+// operand on diagonal blocks; rows and columns past T read zeros or fall on
+// keys that are not stored.  Work per block is small (8 MFMAs per wave at hd
+// 64), so the two blocks in flight and a bare barrier per block set the pace:
+// B=12, 3 heads, T=1024, hd 64, fp32 pattern: 172 us (one gathered element
+// per lane and key) -> 20 us.  The batch elements of a (key block, head) run
+// 8 workgroups apart, on one XCD, and share the pattern through its L2.
+template <typename T, int HD, int PM>
+__global__ __launch_bounds__(256) void bwd_dense_dv_kernel(const BwdParams p) {
+  constexpr int BN = kBwdWaves * 32, NDT = HD / 32, VB = VRow<HD>::BYTES;
+  constexpr int PB = VRow<BN>::BYTES, PP = VRow<BN>::PITCH;
+  constexpr int VN = TileOffsets<T, HD>::VN, PN = TileOffsets<T, BN>::VN;
+  // P loads per thread per block that the block-end wait leaves in flight (the
+  // element loads are not counted: the compiler may merge them)
+  constexpr int NPL = PM == 0 ? PN : (PM == 1 ? 8 : 0);
+  __shared__ __align__(16) char o0[VB], o1[VB], o2[VB], p0[PB], p1[PB], p2[PB];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, g = lane >> 5;
+  const int T_len = p.T;
+  const int nkb = (T_len + BN - 1) / BN;
+  const int x = blockIdx.x & 7, t8 = blockIdx.x >> 3;
+  const int b = t8 % p.B, unit = 8 * (t8 / p.B) + x;  // units heaviest (most queries) first
+  if (unit >= nkb * p.n_frozen) return;
+  const int kb = unit / p.n_frozen, fs = unit % p.n_frozen;
+  if (p.f_kind[fs] != 1) return;
+  const int h = p.f_head[fs];
+  const int64_t patt0 = (int64_t)p.pat_head[fs] * p.p_sh;
+  const T* dobase = reinterpret_cast<const T*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh;
+  T* dvbase = reinterpret_cast<T*>(p.dv) + b * p.dv_sb + (int64_t)h * p.dv_sh;
+  const int k0w = kb * BN + wave * 32;
+  const int kk = k0w + n;
+  f32x16_t dva[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) dva[dt] = zero16();
+  TileOffsets<T, HD> oo;
+  oo.init(wave, lane, p.do_st);
+  TileOffsets<T, BN> po;
+  if constexpr (PM == 0) po.init(wave, lane, p.p_si);
+  ColOffsets<HD> cof;
+  cof.init(lane);
+  const int pcl = vt_read_offset<BN>(lane, wave, 0), pch = vt_read_offset<BN>(lane, wave, 1);
+  const int ib0 = (kb * BN) / 64, nqb = (T_len + 63) / 64;
+
+  // rows 64 i .. of the pattern start at element pfirst(i) and end pleft(i)
+  // elements on, with the 16-byte piece of row T - 1 that holds column T - 1
+  constexpr int PE = PM == 1 ? 4 : 8;  // elements of a piece
+  auto pfirst = [&](int i) { return patt0 + (int64_t)(64 * i) * p.p_si + kb * BN; };
+  auto pleft = [&](int i) {
+    return 64 * i < T_len ? (int64_t)(T_len - 1 - 64 * i) * p.p_si + (T_len - kb * BN + PE - 1) / PE * PE : (int64_t)0;
+  };
+  float pr[3][PM == 0 ? 1 : 32];  // PM 1, 2: raw pattern pieces of the blocks in flight
+  auto load_block = [&](int i, auto slotc) {
+    constexpr int S = decltype(slotc)::value;
+    if constexpr (PM == 0) {
+      po.load_span(reinterpret_cast<const T*>(p.patt) + pfirst(i), pleft(i) * (int64_t)sizeof(T),
+                   S == 0 ? p0 : (S == 1 ? p1 : p2), wave);
+    } else if constexpr (PM == 1) {
+      const __amdgpu_buffer_rsrc_t r = span_rsrc(reinterpret_cast<const float*>(p.patt) + pfirst(i), pleft(i) * 4);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {  // row tid / 16 + 16 (u / 2), columns 8 (tid % 16) + 4 (u % 2) ..
+        const auto w = __builtin_amdgcn_raw_buffer_load_b128(
+            r, ((tid >> 4) + 16 * (u >> 1)) * (int)(p.p_si * 4) + 32 * (tid & 15) + 16 * (u & 1), 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pr[S][4 * u + e] = __uint_as_float(w[e]);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {  // indexes clamped: such cells are cleared or not stored
+          const int row = min(64 * i + (tid >> 4) + 16 * u, T_len - 1);
+          const int col = min(kb * BN + 8 * (tid & 15) + e, T_len - 1);
+          pr[S][8 * u + e] =
+              load_as_f32(p.patt, patt0 + (int64_t)row * p.p_si + (int64_t)col * p.p_sj, p.patt_dtype);
+        }
+    }
+    asm volatile("" ::: "memory");
+    oo.load(dobase, p.do_st, 64 * i, i < nqb ? T_len : 0, S == 0 ? o0 : (S == 1 ? o1 : o2), wave);
+    asm volatile("" ::: "memory");
+  };
+  // PM 1, 2: the pieces of a block, rounded, into P slot S.  (16-byte writes:
+  // 8-byte ones were merged in pairs that the compiler no longer told apart
+  // from the DMA's targets, and it waited for every load in flight.)
+  auto write_block = [&](auto slotc) {
+    constexpr int S = decltype(slotc)::value;
+    char* const pt = S == 0 ? p0 : (S == 1 ? p1 : p2);
+    if constexpr (PM != 0) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int row = (tid >> 4) + 16 * u;
+        const float* const e = &pr[S][8 * u];
+        *reinterpret_cast<uint4*>(pt + row * PP + 16 * ((tid & 15) ^ VRow<BN>::swz(row))) =
+            make_uint4(Elem<T>::pack2(e[0], e[1]), Elem<T>::pack2(e[2], e[3]), Elem<T>::pack2(e[4], e[5]),
+                       Elem<T>::pack2(e[6], e[7]));
+      }
+    }
+  };
+  auto meet = [&]() {  // the next block has landed (the one after stays in flight)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(VN + NPL));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto block = [&](const int i, auto phase) {
+    constexpr int R = decltype(phase)::value;
+    const char* const ot = R == 0 ? o0 : (R == 1 ? o1 : o2);
+    const char* const pt = R == 0 ? p0 : (R == 1 ? p1 : p2);
+    load_block(i + 2, std::integral_constant<int, (R + 2) % 3>());
+    auto products = [&](auto masked) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const char* const pbase = pt + 16 * ks * PP;
+        const uint2 lo = ds_read_tr16(pbase + pcl), hi = ds_read_tr16(pbase + pch);
+        uint32_t w[4] = {lo.x, lo.y, hi.x, hi.y};
+        if constexpr (decltype(masked)::value) {
+          const int first = kk - (64 * i + 16 * ks + 8 * g);  // queries before the key: cleared
+#pragma unroll
+          for (int m = 0; m < 4; ++m)
+            w[m] &= (2 * m >= first ? 0xffffu : 0u) | (2 * m + 1 >= first ? 0xffff0000u : 0u);
+        }
+        const uint4 bop = make_uint4(w[0], w[1], w[2], w[3]);
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) dva[dt] = Elem<T>::mfma(tile_col_op<HD>(ot, ks, dt, cof), bop, dva[dt]);
+      }
+    };
+    if (64 * i >= k0w + 31)
+      products(std::false_type());
+    else if (64 * i + 63 >= k0w)  // else every query precedes this wave's keys
+      products(std::true_type());
+    write_block(std::integral_constant<int, (R + 1) % 3>());  // last read two blocks ago
+    meet();
+  };
+
+  // every key block has queries (kb BN < T)
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
+  using P2 = std::integral_constant<int, 2>;
+  load_block(ib0, P0());
+  load_block(ib0 + 1, P1());
+  write_block(P0());
+  meet();
+  for (int i = ib0;;) {
+    if (i >= nqb) break;
+    block(i++, P0());
+    if (i >= nqb) break;
+    block(i++, P1());
+    if (i >= nqb) break;
+    block(i++, P2());
+  }
+  // the last (empty) DMAs land before the workgroup's LDS is released
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+  if (kk < T_len) store_out_tile<T, HD>(dvbase + (int64_t)kk * p.dv_st, dva, 1.f, g);
 }
 
 // Parameter gradients of decomposed frozen heads (trainable alpha / rho,
@@ -759,8 +916,10 @@ __global__ __launch_bounds__(256) void bwd_decomp_param_kernel(const BwdParams p
   template __global__ void bwd_delta_kernel<T, HD>(const BwdParams);                    \
   template __global__ void bwd_dq_kernel<T, HD>(const BwdParams);                       \
   template __global__ void bwd_dkdv_kernel<T, HD>(const BwdParams);                     \
-  template __global__ void bwd_frozen_dv_kernel<T, HD, 1>(const BwdParams);             \
-  template __global__ void bwd_frozen_dv_kernel<T, HD, 2>(const BwdParams);             \
+  template __global__ void bwd_decomp_dv_kernel<T, HD>(const BwdParams);                \
+  template __global__ void bwd_dense_dv_kernel<T, HD, 0>(const BwdParams);              \
+  template __global__ void bwd_dense_dv_kernel<T, HD, 1>(const BwdParams);              \
+  template __global__ void bwd_dense_dv_kernel<T, HD, 2>(const BwdParams);              \
   template __global__ void bwd_decomp_param_kernel<T, HD>(const BwdParams);
 #define SAF_BWD_INST_T(T) SAF_BWD_INST(T, 32) SAF_BWD_INST(T, 64) SAF_BWD_INST(T, 96) SAF_BWD_INST(T, 128)
 SAF_BWD_INST_T(__bf16)
@@ -788,9 +947,23 @@ static hipError_t bwd_launch_hd(const BwdParams& p, int which, hipStream_t s) {
       hipLaunchKernelGGL((bwd_dkdv_kernel<T, HD>), dim3((unsigned)(nk * p.B * p.n_live)), dim3(256), 0, s, p);
       break;
     case 3: {
-      const dim3 grid((unsigned)(nk * p.B * p.n_frozen));
-      hipLaunchKernelGGL((bwd_frozen_dv_kernel<T, HD, 1>), grid, dim3(256), 0, s, p);
-      hipLaunchKernelGGL((bwd_frozen_dv_kernel<T, HD, 2>), grid, dim3(256), 0, s, p);
+      bool dense = false, decomp = false;
+      for (int i = 0; i < p.n_frozen; ++i) (p.f_kind[i] == 1 ? dense : decomp) = true;
+      if (decomp)
+        hipLaunchKernelGGL((bwd_decomp_dv_kernel<T, HD>), dim3((unsigned)(nk * p.B * p.n_frozen)), dim3(256), 0, s, p);
+      if (dense) {
+        const dim3 grid((unsigned)(8 * p.B * ((nk * p.n_frozen + 7) / 8)));
+        // 16-byte rows (the DMA and the vector loads; 32-bit offsets of 64 rows)
+        const int es = p.patt_dtype == kF32 ? 4 : 2;
+        const bool vec = p.p_sj == 1 && reinterpret_cast<uintptr_t>(p.patt) % 16 == 0 && (p.p_sh * es) % 16 == 0 &&
+                         (p.p_si * es) % 16 == 0 && p.p_si >= 0 && p.p_si * es < kMaxRowBytes;
+        if (vec && p.patt_dtype == (Elem<T>::is_bf16 ? kBF16 : kF16))
+          hipLaunchKernelGGL((bwd_dense_dv_kernel<T, HD, 0>), grid, dim3(256), 0, s, p);
+        else if (vec && p.patt_dtype == kF32)
+          hipLaunchKernelGGL((bwd_dense_dv_kernel<T, HD, 1>), grid, dim3(256), 0, s, p);
+        else
+          hipLaunchKernelGGL((bwd_dense_dv_kernel<T, HD, 2>), grid, dim3(256), 0, s, p);
+      }
       break;
     }
     default:

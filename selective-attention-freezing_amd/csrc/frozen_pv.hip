@@ -733,6 +733,16 @@ __device__ inline uint4 p_chunk(const FrozenParams& p, const PT* prow, int kstar
                     Elem<T>::pack2(e[6], e[7]));
 }
 
+// The P^T operands of one 64-key block for one query tile, as loaded: one
+// 16-byte piece per 16-key step, or (fp32 patterns on the fast path) the raw
+// values of its eight keys, rounded where the block is multiplied.
+template <bool RAW> struct DenseOps {
+  uint4 w[2][2];
+};
+template <> struct DenseOps<true> {
+  uint4 w[2][2][2];
+};
+
 // Per-wave state of the dense P.V kernel (below): the lane's pattern rows,
 // the V DMA and V^T read offsets, and the O^T accumulators of NB sequences.
 template <typename T, typename PT, int HD, int QT, int NB, int NW, bool FAST>
@@ -744,7 +754,9 @@ struct DenseState {
   static_assert(VRow<HD>::CHP % NW == 0, "V tile chunks must split evenly over the waves");
   // end-of-block wait: this wave's V_{j+1} DMA has landed.  Fast path: the
   // loads issued after it (P_{j+1}, V_{j+2}, P_{j+2}) may stay in flight.
-  static constexpr int kWaitV = waitcnt_vm(FAST ? 8 * QT + NB * VN : 0);
+  static constexpr bool RAW = FAST && !std::is_same<PT, T>::value;
+  static constexpr int kWaitV = waitcnt_vm(FAST ? (RAW ? 16 : 8) * QT + NB * VN : 0);
+  using Ops = DenseOps<RAW>;
   const T* vbase[NB];
   int64_t v_st;
   int T_len, wave, g, q0w;
@@ -769,40 +781,66 @@ struct DenseState {
     }
   }
 
-  // P^T operand of key step (ks, sh) of block j for query tile qt.  Fast
-  // path: one raw buffer load; keys past the row and rows past T are
-  // cleared at use (mask_p).  General path: masked and widened here.
-  __device__ __forceinline__ uint4 p_op(const FrozenParams& p, int j, int ks, int sh, int qt) const {
-    if constexpr (FAST) {
-      // per-lane part in the VGPR offset (row, 8g, step), the block in the
-      // scalar offset: no per-block address arithmetic in vector registers
-      return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                           prs, poff[qt] + (uint32_t)(64 * ks + 32 * sh), 128 * j, 0));
-    } else {
-      const int kstart = 64 * j + 32 * ks + 16 * sh + 8 * g;
-      const int nvalid = row[qt] < T_len ? min(row[qt] - kstart + 1, 8) : 0;
-      return p_chunk<T, PT>(p, prow[qt], kstart, nvalid);
-    }
-  }
-  __device__ __forceinline__ void load_p(const FrozenParams& p, uint4 (&pb)[2][2][QT], int j) const {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int sh = 0; sh < 2; ++sh)
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) pb[ks][sh][qt] = p_op(p, j, ks, sh, qt);
-  }
-  __device__ __forceinline__ void mask_p(uint4 (&pb)[2][2][QT], int j) const {
+  // P^T operands of block j.  Fast path: raw buffer loads; keys past the row
+  // and rows past T are cleared at use (operands).  General path: masked and
+  // widened here.
+  __device__ __forceinline__ void load_p(const FrozenParams& p, Ops (&pb)[QT], int j) const {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
       for (int sh = 0; sh < 2; ++sh)
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
-          const int kstart = 64 * j + 32 * ks + 16 * sh + 8 * g;
-          const int nvalid = row[qt] < T_len ? min(row[qt] - kstart + 1, 8) : 0;
-          pb[ks][sh][qt] = keep_leading(pb[ks][sh][qt], nvalid);
+          // per-lane part in the VGPR offset (row, 8g, step), the block in the
+          // scalar offset: no per-block address arithmetic in vector registers
+          if constexpr (RAW) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+              pb[qt].w[ks][sh][u] = __builtin_bit_cast(
+                  uint4, __builtin_amdgcn_raw_buffer_load_b128(prs, poff[qt] + (uint32_t)(128 * ks + 64 * sh + 16 * u),
+                                                               256 * j, 0));
+          } else if constexpr (FAST) {
+            pb[qt].w[ks][sh] = __builtin_bit_cast(
+                uint4, __builtin_amdgcn_raw_buffer_load_b128(prs, poff[qt] + (uint32_t)(64 * ks + 32 * sh), 128 * j, 0));
+          } else {
+            const int kstart = 64 * j + 32 * ks + 16 * sh + 8 * g;
+            const int nvalid = row[qt] < T_len ? min(row[qt] - kstart + 1, 8) : 0;
+            pb[qt].w[ks][sh] = p_chunk<T, PT>(p, prow[qt], kstart, nvalid);
+          }
         }
+  }
+  // The loaded operands of block j in the activation dtype; masked: a
+  // diagonal block or the last rows.
+  __device__ __forceinline__ void operands(const Ops (&pb)[QT], uint4 (&w)[2][2][QT], int j, bool masked) const {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int sh = 0; sh < 2; ++sh)
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          if constexpr (RAW) {
+            const uint4 a = pb[qt].w[ks][sh][0], b = pb[qt].w[ks][sh][1];
+            w[ks][sh][qt] = make_uint4(Elem<T>::pack2(__uint_as_float(a.x), __uint_as_float(a.y)),
+                                       Elem<T>::pack2(__uint_as_float(a.z), __uint_as_float(a.w)),
+                                       Elem<T>::pack2(__uint_as_float(b.x), __uint_as_float(b.y)),
+                                       Elem<T>::pack2(__uint_as_float(b.z), __uint_as_float(b.w)));
+          } else {
+            w[ks][sh][qt] = pb[qt].w[ks][sh];
+          }
+        }
+    if (FAST && masked) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int sh = 0; sh < 2; ++sh)
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) {
+            const int kstart = 64 * j + 32 * ks + 16 * sh + 8 * g;
+            const int nvalid = row[qt] < T_len ? min(row[qt] - kstart + 1, 8) : 0;
+            w[ks][sh][qt] = keep_leading(w[ks][sh][qt], nvalid);
+          }
+    }
   }
 
   // V^T operands of every d tile for 16-key step k (keys 16k..16k+15 of the
@@ -849,18 +887,16 @@ struct DenseState {
   // used), so the compiler's own waits before the MFMAs count exactly the
   // loads issued after P_j.
   __device__ __forceinline__ void block(const FrozenParams& p, int j, int kb1, int kb1_w, const char* cur,
-                                        char* fut, uint4 (&pc)[2][2][QT], uint4 (&pf)[2][2][QT]) {
+                                        char* fut, Ops (&pc)[QT], Ops (&pf)[QT]) {
     if (FAST || j + 2 < kb1) load_v(j + 2, fut);
     asm volatile("" ::: "memory");
     if (FAST || j + 2 < kb1_w) load_p(p, pf, j + 2);
     asm volatile("" ::: "memory");
     if (j < kb1_w) {
-      if (FAST && (64 * j + 63 > q0w || q0w + 32 * QT > T_len)) {
-        // a diagonal block or the last rows: clear keys past each row and rows past T
-        asm volatile("" ::: "memory");
-        mask_p(pc, j);
-      }
-      mma_block(cur, pc);
+      // a diagonal block or the last rows: keys past each row and rows past T are cleared
+      uint4 w[2][2][QT];
+      operands(pc, w, j, 64 * j + 63 > q0w || q0w + 32 * QT > T_len);
+      mma_block(cur, w);
     }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(kWaitV);
@@ -887,7 +923,9 @@ struct DenseState {
 // one unconditional buffer load, so a wave knows how many loads were issued
 // after its V_{j+1} DMA: it waits for exactly those to remain (vmcnt) and
 // meets the others at a bare s_barrier; a __syncthreads would drain the
-// pattern loads at every block.  Other pattern dtypes wait for vmcnt 0.
+// pattern loads at every block.  fp32 patterns with 16-byte rows (the model's
+// default storage) go the same way as two loads per operand, rounded where
+// they are used.  Other pattern types and strides wait for vmcnt 0.
 // Work items cover a key segment of a query block; split blocks write fp32
 // partials that the combine kernel sums.
 template <typename T, typename PT, int HD, int QT, int NB, bool FAST>
@@ -898,7 +936,8 @@ void frozen_dense_kernel(const FrozenParams p) {
   constexpr int BM = NW * 32 * QT;
   constexpr int NDT = St::NDT;
   static_assert(NB * QT * NDT <= 8, "accumulators must fit two waves per SIMD");
-  static_assert(!FAST || std::is_same<T, PT>::value, "the fast path loads the pattern in the activation dtype");
+  static_assert(!FAST || std::is_same<T, PT>::value || std::is_same<PT, float>::value,
+                "the fast path loads the pattern in the activation dtype or fp32");
   __shared__ __align__(16) char vs0[NB * St::VB], vs1[NB * St::VB], vs2[NB * St::VB];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -958,7 +997,7 @@ void frozen_dense_kernel(const FrozenParams p) {
     st.row[qt] = st.q0w + 32 * qt + n;
     const int rc = min(st.row[qt], T_len - 1);
     st.prow[qt] = pbase + (int64_t)rc * p.p_si;
-    st.poff[qt] = (uint32_t)((int64_t)(rc - q0) * p.p_si * (int64_t)sizeof(PT)) + 16u * g;
+    st.poff[qt] = (uint32_t)((int64_t)(rc - q0) * p.p_si * (int64_t)sizeof(PT)) + 8u * (uint32_t)sizeof(PT) * g;
   }
   const int64_t pfirst = pat_off + (int64_t)q0 * p.p_si;
   st.prs = span_rsrc(reinterpret_cast<const PT*>(p.patt) + pfirst, (p.patt_elems - pfirst) * (int64_t)sizeof(PT));
@@ -970,7 +1009,7 @@ void frozen_dense_kernel(const FrozenParams p) {
       for (int dt = 0; dt < NDT; ++dt) st.o[nb][qt][dt] = zero16();
 
   // prologue: blocks kb0 and kb0+1 in flight, then V_kb0 landed everywhere
-  uint4 pA[2][2][QT], pB[2][2][QT], pC[2][2][QT];
+  typename St::Ops pA[QT], pB[QT], pC[QT];
   st.load_v(kb0, vs0);
   asm volatile("" ::: "memory");
   if (FAST || kb0 < kb1_w) st.load_p(p, pA, kb0);
@@ -1023,7 +1062,9 @@ static void launch_dense_t(const FrozenParams& p, hipStream_t s) {
   constexpr int QT = dense_qtiles(HD, NB);
   const int64_t groups = (int64_t)(p.n_items ? p.n_items : p.n_qblk) * p.n_slots;
   const dim3 grid((unsigned)(8 * (p.B / NB) * ((groups + 7) / 8)));
-  if constexpr (std::is_same<T, PT>::value) {
+  // fp32 patterns take the fast path where their raw operands fit the
+  // registers (hd <= 128; half the batch group)
+  if constexpr (std::is_same<T, PT>::value || (std::is_same<PT, float>::value && NB * (HD / 32) <= 4)) {
     if (p.patt_vec) {
       hipLaunchKernelGGL((frozen_dense_kernel<T, PT, HD, QT, NB, true>), grid, dim3(64 * kDenseWaves), 0, s, p);
       return;
@@ -1034,14 +1075,15 @@ static void launch_dense_t(const FrozenParams& p, hipStream_t s) {
 
 template <typename T, typename PT, int HD>
 static void launch_dense_nb(const FrozenParams& p, hipStream_t s) {
-  if constexpr (HD <= 64) {
-    if (dense_batch_group(p.B, HD) == 4) {
+  constexpr bool wide = std::is_same<PT, float>::value;
+  if constexpr (dense_batch_group(4, HD, wide) >= 4) {
+    if (p.batch_group == 4) {
       launch_dense_t<T, PT, HD, 4>(p, s);
       return;
     }
   }
-  if constexpr (HD <= 128) {
-    if (dense_batch_group(p.B, HD) == 2) {
+  if constexpr (dense_batch_group(4, HD, wide) >= 2) {
+    if (p.batch_group == 2) {
       launch_dense_t<T, PT, HD, 2>(p, s);
       return;
     }

@@ -444,11 +444,27 @@ int frozen_qtiles(int hd) { return hd <= 64 ? 2 : 1; }
 int decomp_resident(int hd) { return hd > 64 ? 2 : 3; }
 
 // Dense P.V work plan: query blocks of the kernel's shape, balanced over the
-// batch groups that share a pattern (dense_batch_group).
-FlashPlan plan_dense(int B, int n_slots, int T, int HD) {
-  const int nb = dense_batch_group(B, HD);
-  return plan_flash(B / nb, n_slots, T, HD, dense_block_rows(B, HD), kDenseResident, nb);
+// batch groups that share a pattern.  Larger groups read the pattern fewer
+// times; where the plan has nothing to split (short sequences, or no
+// workspace for partials) and the groups leave CUs without a workgroup, the
+// group is halved (B=12, 3 heads, T=1024, fp32 patterns: 36 workgroups of four
+// sequences 60 us, 144 of one, with the 16-byte pattern loads, 40 us).
+struct DensePlan {
+  FlashPlan fp;
+  int group = 1;
+};
+DensePlan plan_dense(int B, int n_slots, int T, int HD, bool wide, bool can_split) {
+  DensePlan d;
+  const int nqb = (T + dense_block_rows(B, HD) - 1) / dense_block_rows(B, HD);
+  for (d.group = dense_batch_group(B, HD, wide);; d.group /= 2) {
+    d.fp = can_split ? plan_flash(B / d.group, n_slots, T, HD, dense_block_rows(B, HD), kDenseResident, d.group)
+                     : FlashPlan();
+    if (d.group == 1 || d.fp.n_items || (int64_t)nqb * n_slots * (B / d.group) >= cu_count()) return d;
+  }
 }
+
+// A pattern in fp32 for 16-bit activations.
+bool dense_wide(const saf_tensor_t& patt, int act_dtype) { return patt.dtype == SAF_F32 && act_dtype != SAF_F32; }
 
 // Dense P.V over the heads listed; with a workspace large enough for the
 // plan's partials, long query blocks are split into key segments (the flash
@@ -476,9 +492,13 @@ int run_dense(const saf_tensor_t& patt, const saf_tensor_t& v, const saf_tensor_
     p.v_head[i] = (int16_t)v_head[i];
     p.pat_head[i] = (int16_t)pat_head[i];
   }
-  FlashPlan fp = plan_dense(B, p.n_slots, T, HD);
-  if (dtype != SAF_F32 && fp.n_items && ws != nullptr && ws_bytes >= fp.part_bytes &&
-      reinterpret_cast<uintptr_t>(ws) % 16 == 0) {
+  const bool wide = dense_wide(patt, dtype);
+  DensePlan dp = plan_dense(B, p.n_slots, T, HD, wide, true);
+  if (dp.fp.n_items && (ws == nullptr || ws_bytes < dp.fp.part_bytes || reinterpret_cast<uintptr_t>(ws) % 16 != 0))
+    dp = plan_dense(B, p.n_slots, T, HD, wide, false);
+  p.batch_group = dp.group;
+  FlashPlan& fp = dp.fp;
+  if (dtype != SAF_F32 && fp.n_items) {
     p.n_items = fp.n_items;
     p.seg_len = fp.seg_len;
     p.n_part_per_head = fp.n_part_per_head;
@@ -522,7 +542,8 @@ int64_t part_region_bytes(const saf_mixed_attn_args* args, const Plan& pl) {
     part = kQueueBytes + fp.part_bytes;
   }
   if (!pl.dense.empty())
-    part = std::max(part, plan_dense(pl.B, (int)pl.dense.size(), pl.T, pl.HD).part_bytes);
+    part = std::max(part, plan_dense(pl.B, (int)pl.dense.size(), pl.T, pl.HD, dense_wide(args->patt, pl.dtype), true)
+                              .fp.part_bytes);
   if (!pl.decomp.empty())
     part = std::max(part, plan_flash(pl.B, (int)pl.decomp.size(), pl.T, pl.HD, block_rows(frozen_qtiles(pl.HD)),
                                      decomp_resident(pl.HD)).part_bytes);

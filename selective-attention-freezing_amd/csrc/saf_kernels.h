@@ -113,6 +113,7 @@ struct FrozenParams {
   // fp32 partials of split query blocks summed by the combine kernel;
   // n_items == 0: one item per query block, heaviest first
   int n_items, seg_len, n_part_per_head;
+  int batch_group;  // dense: batch elements per workgroup (NB of the kernel)
   float* part_o;
   int32_t items[kMaxItems];
   int16_t part_base[kMaxQblk];
@@ -326,13 +327,15 @@ inline int block_rows(int qt) { return 4 * 32 * qt; }
 
 // Dense P.V shape: a workgroup of kDenseWaves waves (two per SIMD, one
 // query tile of 32 rows each) serves a group of NB batch elements that share
-// every pattern operand, as many as 128 accumulator registers per wave
-// allow: 4 at hd <= 64 (batch a multiple of 4), 2 at hd <= 128 (even batch),
-// else 1; one workgroup per CU (its three V slots fill most of the LDS at
-// hd 128).
+// every pattern operand, at most as many as 128 accumulator registers per
+// wave allow: 4 at hd <= 64 (batch a multiple of 4), 2 at hd <= 128 (even
+// batch), else 1; half of that for fp32 patterns, whose raw operands take
+// twice the registers.  One workgroup per CU (its three V slots fill most of
+// the LDS at hd 128).
 constexpr int kDenseWaves = 8;
-constexpr int dense_batch_group(int B, int hd) {
-  return B % 4 == 0 && hd <= 64 ? 4 : (B % 2 == 0 && hd <= 128 ? 2 : 1);
+constexpr int dense_batch_group(int B, int hd, bool wide) {
+  const int cap = (hd <= 64 ? 4 : (hd <= 128 ? 2 : 1)) / (wide && hd <= 128 ? 2 : 1);
+  return B % 4 == 0 && cap >= 4 ? 4 : (B % 2 == 0 && cap >= 2 ? 2 : 1);
 }
 constexpr int dense_qtiles(int, int) { return 1; }
 constexpr int dense_block_rows(int, int) { return kDenseWaves * 32; }
