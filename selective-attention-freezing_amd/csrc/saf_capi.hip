@@ -484,6 +484,10 @@ int run_dense(const saf_tensor_t& patt, const saf_tensor_t& v, const saf_tensor_
   const int es = elem_size(patt.dtype);
   p.patt_vec = patt.stride[2] == 1 && reinterpret_cast<uintptr_t>(patt.data) % 16 == 0 &&
                (patt.stride[1] * es) % 16 == 0 && (patt.stride[0] * es) % 16 == 0;
+  // the descriptor ends with the 16-byte piece that holds the last element: an
+  // odd count of 16-bit elements would end inside a 32-bit word, which then
+  // reads as zero
+  if (p.patt_vec) p.patt_elems = (p.patt_elems + 16 / es - 1) / (16 / es) * (16 / es);
   p.n_slots = (int)out_head.size();
   const int BM = dense_block_rows(B, HD);
   p.n_qblk = (T + BM - 1) / BM;
