@@ -1,0 +1,66 @@
+"""Row normalisers and their gradients at the edges of the kernels' 256-row
+blocks, 2048-key chunks and 4-key steps, in the product form and where blocks
+fall back to the direct one, against the float64 oracle.
+
+z: each row sums at most S positive fp32 products in two levels, well under
+1e-5 relative, so |dz| <= 1e-5 (1 + |z|) covers the sum, the fp32 exponent
+arguments and the result's rounding.  Gradients: the terms' exponents carry
+the rounding of values up to |z| (2^-23 |x| each), the sums run over S signed
+terms: 1e-5 in relative L2."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import saf_oracle as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _inputs(kind, H, S):
+    g = torch.Generator().manual_seed(S + H)
+    a = 0.5 * torch.randn(H, S, generator=g)
+    r = -0.7 * torch.log1p(torch.arange(S, dtype=torch.float32)) + 0.2 * torch.randn(H, S, generator=g)
+    if kind == "decay":     # distances far apart in exponent
+        a = torch.zeros(H, S)
+        r = -0.1 * torch.arange(S, dtype=torch.float32).repeat(H, 1)
+    elif kind == "window":  # exact zeros and whole -inf chunks
+        r = torch.where(torch.arange(S) < 70, r, torch.tensor(float("-inf")))
+    elif kind == "spike":   # a key far above the rest: rows before it lie below its chunk's scale
+        a[:, S // 2] = 120.0
+    elif kind == "wide":    # logits of scale 40
+        a, r = 80 * a, 40 * torch.randn(H, S, generator=g)
+    elif kind == "late":    # the first keys absent: rows without any key
+        a[:, : min(S - 1, 130)] = float("-inf")
+    return a, r
+
+
+@pytest.mark.parametrize("kind", ["learned", "decay", "window", "spike", "wide", "late"])
+@pytest.mark.parametrize("S", [1, 5, 255, 256, 257, 2047, 2050, 2305, 4099])
+def test_logz_blocks(kind, S):
+    import kernel
+    H = 2
+    a, r = _inputs(kind, H, S)
+    gz = torch.randn(H, S, generator=torch.Generator().manual_seed(1))
+    ad, rd = a.to(DEV).requires_grad_(), r.to(DEV).requires_grad_()
+    z = kernel.decomp_log_normalizers(ad, rd)
+    ref = orc.decomposed_logz(a.double().numpy(), r.double().numpy())
+    zh = z.detach().double().cpu().numpy()
+    fin = np.isfinite(ref)
+    assert np.array_equal(fin, np.isfinite(zh))
+    assert (np.abs(zh - ref)[fin] <= 1e-5 * (1 + np.abs(ref[fin]))).all()
+    da, dr = torch.autograd.grad(z, (ad, rd), gz.to(DEV))
+    # the float64 gradients from the kernel's own z, as its backward takes it
+    zz = torch.from_numpy(np.where(fin, zh, np.inf))
+    wa, wr = torch.zeros(H, S, dtype=torch.float64), torch.zeros(H, S, dtype=torch.float64)
+    for i in range(S):
+        p = gz[:, i, None].double() * torch.exp(a[:, : i + 1].double() + r[:, : i + 1].double().flip(1) - zz[:, i, None])
+        wa[:, : i + 1] += p
+        wr[:, : i + 1] += p.flip(1)
+    for got, want, name in ((da, wa, "dalpha"), (dr, wr, "drho")):
+        got = got.double().cpu()
+        assert torch.isfinite(got).all(), name
+        err = float((got - want).norm()) / max(float(want.norm()), 1e-30)
+        # exponent arguments of magnitude x round by 2^-23 |x|
+        mag = float(torch.nan_to_num(a, neginf=0.0).abs().max() + torch.nan_to_num(r, neginf=0.0).abs().max())
+        assert err <= 1e-5 + 2.0 ** -21 * mag, f"{name}: {err:.2e}"
