@@ -126,8 +126,9 @@ typedef struct saf_mixed_attn_args {
                                    workgroup per query block on the library's side stream
                                    beside the live-head kernel when live heads share the call
                                    (its workgroups fill the slots the causal imbalance leaves
-                                   idle); otherwise, and in saf_frozen_decomp_fwd, their long
-                                   query blocks are split into key segments (fp32 partials in
+                                   idle) and they are long enough to pay for the fork
+                                   (8 GFLOP); otherwise, and in saf_frozen_decomp_fwd, their
+                                   long query blocks are split into key segments (fp32 partials in
                                    the workspace region the live-head and dense kernels also
                                    use, then a combine);
                                    1 = one workgroup per query block, no partials, so a
@@ -137,10 +138,11 @@ typedef struct saf_mixed_attn_args {
 } saf_mixed_attn_args;
 
 /* All head kinds: live flash, dense P.V, decomposed P.V, closed-form scan.
- * The closed-form scan and (see decomp_unsplit) the decomposed heads run on a
- * second stream of the library (one per device, default priority), forked
- * from and joined back into `stream` by events within the call, so the call
- * is ordered on `stream` like a single kernel. */
+ * In calls long enough to pay for it the closed-form scan and (see
+ * decomp_unsplit) the decomposed heads run on a second stream of the library
+ * (one per device, default priority), forked from and joined back into
+ * `stream` by events within the call, so the call is ordered on `stream` like
+ * a single kernel. */
 int saf_mixed_attn_fwd(const saf_mixed_attn_args* args, void* stream);
 
 /* saf_mixed_attn_fwd without a caller workspace, for callers that cannot

@@ -753,8 +753,25 @@ int side_join_locked(SideStream* ss, hipStream_t s) {
   return SAF_OK;
 }
 
-// The head kinds of `which`.  With may_fork (saf_mixed_attn_fwd), the
-// HBM-bound closed-form scan and, when live heads share the call, the
+// Flops of one causal P.V product over n heads of every sequence.
+double pv_flops(const Plan& pl, size_t n) { return (double)pl.B * (double)n * pl.HD * (double)pl.T * pl.T; }
+
+// When forking pays: a fork and join cost about 35 us of host time and a few
+// us on the caller's stream, against which the side kernel's time is hidden.
+// Decomposed heads (and the backward's frozen dV) of 8 GFLOP and more run
+// beside the live heads: B=8, T=3001 (13.8 GFLOP) 142 us forked, 146 in
+// order; forward + backward at B=8, T=4096 (26 GFLOP) 851 against 902; B=4,
+// T=2048 (3.2 GFLOP) 71 either way, with its backward 249 against 223.
+constexpr double kSideMinFlops = 8e9;
+// The scan (10 us or so) runs beside the other kernels when these take about
+// 240 us: one 16384-token layer 347 us either way and a 12-layer prefill of
+// them 7.40 against 7.45 ms, but B=8, T=4096 185 us forked, 184 in order;
+// 14 query heads at B=4, T=4096 123 against 118; T=2048 62 against 37; T=100
+// 62 against 24.
+constexpr double kSideMinMainUs = 240;
+
+// The head kinds of `which`.  With may_fork (saf_mixed_attn_fwd) and work
+// enough (above), the HBM-bound closed-form scan and, when live heads share the call, the
 // decomposed heads (one workgroup per query block, unless decomp_unsplit < 0)
 // run on the side stream beside the live-head and dense kernels: disjoint
 // output rows and workspace regions, joined before returning.  Otherwise
@@ -765,9 +782,12 @@ int run(const saf_mixed_attn_args* a, unsigned which, void* stream, bool may_for
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool has_dec = (which & kDoDecomp) && !pl.decomp.empty();
   const bool has_live = (which & kDoFlash) && !pl.live.empty();
-  const bool dec_side = may_fork && has_dec && has_live && a->decomp_unsplit >= 0;
-  const bool scan_side = may_fork && (which & kDoScan) && !pl.scan.empty() &&
-                         (has_live || has_dec || ((which & kDoDense) && !pl.dense.empty()));
+  const bool dec_side = may_fork && has_dec && has_live && a->decomp_unsplit >= 0 &&
+                        (a->decomp_unsplit > 0 || pv_flops(pl, pl.decomp.size()) >= kSideMinFlops);
+  const double main_us = 2 * pv_flops(pl, has_live ? pl.live.size() : 0) * 1.2e-9 +
+                         pv_flops(pl, (has_dec && !dec_side ? pl.decomp.size() : 0) +
+                                          ((which & kDoDense) ? pl.dense.size() : 0)) * 2e-9;
+  const bool scan_side = may_fork && (which & kDoScan) && !pl.scan.empty() && (dec_side || main_us >= kSideMinMainUs);
   const bool dec_unsplit = a->decomp_unsplit > 0;
   if (!dec_side && !scan_side) {
     if (which & kDoFlash)
@@ -1323,8 +1343,9 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
     }
   }
   // the frozen heads' dV (its own rows of dv, no workspace) on the side
-  // stream beside the live heads' kernels, whose tails leave slots idle
-  const bool fork = !pl.live.empty() && nf > 0;
+  // stream beside the live heads' kernels, whose tails leave slots idle,
+  // where it is long enough to pay for the fork
+  const bool fork = !pl.live.empty() && nf > 0 && pv_flops(pl, nf) >= kSideMinFlops;
   std::unique_lock<std::mutex> lock(g_side_mu, std::defer_lock);
   SideStream* ss = nullptr;
   if (fork) {

@@ -12,9 +12,9 @@ The work runs in libsafattn.so on the current HIP stream: a live-head flash
 kernel on bf16/fp16 MFMA, a dense P.V MFMA kernel, a decomposed P.V kernel
 (factored Toeplitz form or P rebuilt per cell), and, for decomposed heads
 whose pattern is the causal mean, an exponential decay or a sliding window
-(``closed_form=``), a single-pass scan that reads V once.  The scan and the
-decomposed heads run on a second stream beside the live-head kernel, joined
-before the call returns.  Output is in natural head order.
+(``closed_form=``), a single-pass scan that reads V once.  In long calls the
+scan and the decomposed heads run on a second stream beside the live-head
+kernel, joined before the call returns.  Output is in natural head order.
 
 Pattern helpers (``make_rho_band``, ``decomp_logits``, ``decomposed_logz``)
 follow the reference's definitions (/root/reference/kernel/fused_attn.py:50-116).
@@ -223,32 +223,43 @@ def _host_table(t, np_dtype=np.int32):
     """Host copy of a small per-head table, cached on the tensor itself and
     refreshed when its version counter moves (one sync per change, the same
     moment the reference syncs: nanogpt/model.py:853, :875)."""
+    return _table(t, np_dtype)[0]
+
+
+def _table(t, np_dtype=np.int32):
+    """(_host_table(t), its ctypes copy for the argument block)."""
     if t is None:
-        return None
+        return None, None
+    make = _ext.host_i32 if np_dtype is np.int32 else _ext.host_f32
     if not isinstance(t, torch.Tensor):
-        return np.asarray(t, dtype=np_dtype)
+        arr = np.asarray(t, dtype=np_dtype)
+        return arr, make(arr)
     cached = getattr(t, "_saf_host", None)
-    if cached is not None and cached[0] == t._version and cached[1] == t.data_ptr():
-        return cached[2]
+    if cached is not None and cached[0] == t._version and cached[1] == t.data_ptr() and cached[2].dtype == np_dtype:
+        return cached[2], cached[3]
     arr = t.detach().cpu().numpy().astype(np_dtype, copy=False).reshape(-1)
     arr = np.ascontiguousarray(arr)
+    buf = make(arr)
     try:
-        t._saf_host = (t._version, t.data_ptr(), arr)
+        t._saf_host = (t._version, t.data_ptr(), arr, buf)
     except (AttributeError, RuntimeError):
         pass
-    return arr
+    return arr, buf
 
 
 def _row_aligned(t, align):
     if t is None:
         return True
-    if t.stride(-1) != 1 and t.size(-1) != 1:
+    shape, stride = t.shape, t.stride()
+    if stride[-1] != 1 and shape[-1] != 1:
         return False
     es = t.element_size()
     if t.data_ptr() % align:
         return False
-    return all(s <= 1 or (st * es) % align == 0
-               for s, st in zip(t.shape[:-1], t.stride()[:-1]))
+    for s, st in zip(shape[:-1], stride):
+        if s > 1 and (st * es) % align:
+            return False
+    return True
 
 
 def _aligned_view(t, align=16):
@@ -353,8 +364,8 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
                is the give-up drill that tests the error path (every scan
                chunk after the first gives up: NaN rows, and with validate
                a RuntimeError)
-      decomp_unsplit  None (auto) = True when live heads share the call;
-               True: decomposed heads run one workgroup per query block,
+      decomp_unsplit  None (auto) = True when live heads share the call and
+               the decomposed ones are long enough to pay for a fork; True: decomposed heads run one workgroup per query block,
                beside the live-head kernel on a side stream when there is
                one; False: key-segment split with partials and a combine,
                after the live-head kernel on the current stream
@@ -378,142 +389,106 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
             "fused_mixed_attn runs on HIP devices only (got a CPU tensor); "
             "this build has no CPU kernel path")
 
-    frozen_h = _host_table(frozen)
-    hidx_h = None if hidx is None else _host_table(hidx)
-    pidx_h = None if pidx is None else _host_table(pidx)
-    kvidx_h = None if kvidx is None else _host_table(kvidx)
-    ck = cp = None
+    frozen_h, frozen_c = _table(frozen)
+    _, hidx_c = _table(hidx)
+    _, pidx_c = _table(pidx)
+    _, kvidx_c = _table(kvidx)
+    states = frozen_h.tolist()
+    n_live, n_state2 = states.count(0), states.count(2)
+    ck_c = cp_c = None
+    n_scan = 0
     if closed_form is not None:
-        ck = _host_table(closed_form[0], np.int32)
-        cp = _host_table(closed_form[1], np.float32)
+        ck, ck_c = _table(closed_form[0], np.int32)
+        _, cp_c = _table(closed_form[1], np.float32)
+        if n_state2:
+            n_scan = n_state2 - [c for s, c in zip(states, ck.tolist()) if s == 2].count(0)
 
     B, HV, T, HD = v.shape
-    n_live = int((frozen_h == 0).sum())
+    dev, dt = v.device, v.dtype
     needs_grad = torch.is_grad_enabled() and any(
         t is not None and t.requires_grad for t in (q, k, v))
     if needs_grad and n_live and lse is None:
         # the backward recomputes P from the forward's base-2 LSE
-        lse = torch.empty((B, H, T), device=v.device, dtype=torch.float32)
+        lse = torch.empty((B, H, T), device=dev, dtype=torch.float32)
     q_d = k_d = None
     if n_live:
         q_d = _aligned_view(q, 16)
         k_d = _aligned_view(k, 16)
     v_d = _aligned_view(v, 16)
-    if v_d.stride(2) > v_d.stride(1):
+    v_st = v_d.stride()
+    if v_st[2] > v_st[1]:
         # v is a T-major view (the model's (B, T, H, hd) projection output):
         # keep that layout so the caller's transpose(1, 2).reshape is free,
         # as the reference's empty_like(v) does for a dense v (with kvidx the
         # output still has all H query heads)
-        out = torch.empty((B, T, H, HD), device=v.device, dtype=v.dtype).transpose(1, 2)
+        out = torch.empty_strided((B, H, T, HD), (T * H * HD, HD, H * HD, 1), device=dev, dtype=dt)
     elif kv_identity:
         out = torch.empty_like(v_d)
         if not _row_aligned(out, 8):
-            out = torch.empty((B, H, T, HD), device=v.device, dtype=v.dtype)
+            out = torch.empty((B, H, T, HD), device=dev, dtype=dt)
     else:
-        out = torch.empty((B, H, T, HD), device=v.device, dtype=v.dtype)
+        out = torch.empty((B, H, T, HD), device=dev, dtype=dt)
 
-    n_scan = 0
-    if ck is not None:
-        n_scan = int(((frozen_h == 2) & (ck != 0)).sum())
     L = _ext.lib()
-
-    need_dec = alpha is not None and bool(
-        ((frozen_h == 2) & ((ck == 0) if ck is not None else True)).any())
     # the backward runs closed-form heads through their decomposed buffers
-    need_dec = need_dec or (needs_grad and alpha is not None and bool((frozen_h == 2).any()))
+    need_dec = alpha is not None and n_state2 > (0 if needs_grad else n_scan)
 
     args = _ext.SafMixedAttnArgs()
-    args.q = _ext.tensor_desc(q_d)
-    args.k = _ext.tensor_desc(k_d)
-    args.v = _ext.tensor_desc(v_d)
-    args.out = _ext.tensor_desc(out)
-    args.lse = _ext.tensor_desc(lse)
-    args.patt = _ext.tensor_desc(patt)
+    off, put = _ext.ARG_OFFSET, _ext.set_desc
+    if n_live:
+        put(args, off["q"], q_d)
+        put(args, off["k"], k_d)
+    put(args, off["v"], v_d)
+    put(args, off["out"], out)
+    if lse is not None:
+        put(args, off["lse"], lse)
+    if patt is not None:
+        put(args, off["patt"], patt)
     if need_dec:
-        args.alpha = _ext.tensor_desc(alpha)
-        args.rho = _ext.tensor_desc(rho)
-        args.z = _ext.tensor_desc(z)
-    args.n_heads = H
-    keep = [_ext.host_i32(frozen_h), _ext.host_i32(hidx_h), _ext.host_i32(pidx_h),
-            _ext.host_i32(kvidx_h), _ext.host_i32(ck), _ext.host_f32(cp)]
-    args.frozen, args.hidx, args.pidx, args.kvidx, args.closed_kind = keep[:5]
-    args.closed_param = keep[5]
+        put(args, off["alpha"], alpha)
+        put(args, off["rho"], rho)
+        put(args, off["z"], z)
+    keep = (frozen_c, hidx_c, pidx_c, kvidx_c, ck_c, cp_c)
+    _ext.set_tables(args, H, *keep)
     args.sm_scale = float(sm_scale)
-    args.flash_qtiles = int(flash_qtiles)
-    args.scan_spin_limit = int(scan_spin_limit)
+    if flash_qtiles:
+        args.flash_qtiles = int(flash_qtiles)
+    if scan_spin_limit:
+        args.scan_spin_limit = int(scan_spin_limit)
     # scan look-back words + partials of the causally balanced live-head kernel
-    ws_bytes = int(L.saf_mixed_attn_workspace_bytes(args))
+    ws_bytes = L.saf_mixed_attn_workspace_bytes(args)
     if ws_bytes < 0:
         _ext.check(L.saf_mixed_attn_fwd(args, None))  # raises with the validation message
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=v.device) if ws_bytes else None
-    args.workspace = None if ws is None else ws.data_ptr()
-    args.workspace_bytes = ws_bytes
-
-    n_dense = int((frozen_h == 1).sum())
-    n_dec = int((frozen_h == 2).sum()) - n_scan
-
-    work = {"flash": (L.saf_flash_fwd, n_live * B * 4 * HD * T * (T + 1) // 2),
-            "scan": (L.saf_frozen_scan_fwd, n_scan * B * 2 * T * HD * v.element_size()),
-            "dense": (L.saf_frozen_dense_pv_fwd, n_dense * B * 2 * HD * T * (T + 1) // 2),
-            "decomp": (L.saf_frozen_decomp_fwd, n_dec * B * 2 * HD * T * (T + 1) // 2)}
+    if ws_bytes:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        _ext.set_workspace(args, ws.data_ptr(), ws_bytes)
 
     def run():
-        timer = _TIMER
-        cur = torch.cuda.current_stream(v.device)
-
-        def launch(kind, strm):  # one timed per-kind call
-            fn, w = work[kind]
-            e0 = torch.cuda.Event(enable_timing=True)
-            e1 = torch.cuda.Event(enable_timing=True)
-            e0.record(strm)  # creates the HIP events; the library re-records them
-            e1.record(strm)
-            _ext.check(L.saf_time_next_kernel(e0.cuda_event, e1.cuda_event))
-            rc = fn(args, strm.cuda_stream)
-            L.saf_time_next_kernel(None, None)  # never left pending for a later call
-            _ext.check(rc)
-            timer.records[kind].append((e0, e1, w))
-
-        if timer is None:
+        if _TIMER is None:
             # one call: the library runs the closed-form scan and the
             # decomposed heads on its side stream beside the live-head kernel
-            args.decomp_unsplit = {None: 0, True: 1, False: -1}[decomp_unsplit]
-            _ext.check(L.saf_mixed_attn_fwd(args, cur.cuda_stream))
+            # where that pays
+            if decomp_unsplit is not None:
+                args.decomp_unsplit = 1 if decomp_unsplit else -1
+            stream = _ext.current_stream_ptr(dev)
+            rc = L.saf_mixed_attn_fwd(args, stream)
+            if rc:
+                _ext.check(rc)
         else:
-            # the same schedule through the per-kind entry points, each kernel
-            # timed on its own stream: decomposed heads beside live ones run
-            # one workgroup per query block (decomp_unsplit = 1), so the
-            # live-head kernel's workgroups fill the slots their causal
-            # imbalance leaves idle and no key-segment partials are needed
-            unsplit = bool(n_live) if decomp_unsplit is None else bool(decomp_unsplit)
-            args.decomp_unsplit = 1 if unsplit else -1
-            dec_side = bool(n_dec and n_live and unsplit)
-            if (n_scan and (n_live or n_dense or n_dec)) or dec_side:
-                # disjoint output rows and workspace regions; joined before
-                # returning
-                side = _side_stream(v.device)
-                side.wait_stream(cur)
-                if dec_side:
-                    launch("decomp", side)
-                if n_scan:
-                    launch("scan", side)
-                for kind in ("flash", "dense", "decomp"):
-                    if work[kind][1] and not (kind == "decomp" and dec_side):
-                        launch(kind, cur)
-                cur.wait_stream(side)
-            else:
-                for kind in KernelTimer.KINDS:
-                    if work[kind][1]:
-                        launch(kind, cur)
+            stream = _timed_run(args, states, n_scan, n_state2 - n_scan, B, T, HD, v, decomp_unsplit)
         if n_scan and validate:
             # a look-back wait that gave up leaves NaN rows (never a silently
             # incomplete sum); with validate the call also raises
             err = _ext.ctypes.c_int32(0)
-            _ext.check(L.saf_workspace_error(args.workspace, cur.cuda_stream, _ext.ctypes.byref(err)))
+            _ext.check(L.saf_workspace_error(args.workspace, stream, _ext.ctypes.byref(err)))
             if err.value:
                 raise RuntimeError(
                     "closed-form scan: a look-back wait gave up (scan_spin_limit reached); "
                     "the affected rows of the output are NaN")
         return out
+
+    if not needs_grad:
+        return run()
 
     # every tensor the argument block points to stays alive until the backward
     # (out itself is saved by the autograd node and passed back in)
@@ -527,30 +502,87 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
             raise NotImplementedError(
                 "fused_mixed_attn backward with kvidx (GQA) is not implemented "
                 "(as in qwen/kernel/fused_attn.py:605-609 of the reference)")
-        if bool((frozen_h == 2).any()) and alpha is None:
+        if n_state2 and alpha is None:
             raise ValueError("the backward of decomposed heads needs alpha/rho/z")
-        do = dout.contiguous()
-        dq = torch.zeros(q_d.shape, device=v.device, dtype=v.dtype) if n_live else None
-        dk = torch.zeros(k_d.shape, device=v.device, dtype=v.dtype) if n_live else None
-        dv = torch.empty(v_d.shape, device=v.device, dtype=v.dtype)
-        bws = int(L.saf_mixed_attn_bwd_workspace_bytes(args))
+        # the kernels take any layout of aligned, distinct rows (the model's
+        # gradient arrives as a head-major view of a (B, T, C) tensor);
+        # expanded gradients and huge pitches are copied
+        do = dout
+        if not (_row_aligned(do, 16) and HD <= do.stride(2) < (1 << 21)):
+            do = do.contiguous()
+        dq = dk = None
+        if n_live:
+            # zeros only where some slot belongs to no live head
+            used = {i for i, s in enumerate(states) if s == 0}
+            if hidx_c is not None:
+                used = {hidx_c[i] for i in used}
+            make = torch.empty if len(used) == q_d.shape[1] else torch.zeros
+            dq = make(q_d.shape, device=dev, dtype=dt)
+            dk = make(k_d.shape, device=dev, dtype=dt)
+        dv = torch.empty(v_d.shape, device=dev, dtype=dt)
+        bws = L.saf_mixed_attn_bwd_workspace_bytes(args)
         if bws < 0:
             bws = 0
-        bw = torch.empty(max(bws, 1), dtype=torch.uint8, device=v.device)
+        bw = torch.empty(max(bws, 1), dtype=torch.uint8, device=dev)
         bargs = _ext.SafMixedAttnArgs.from_buffer_copy(args)
-        bargs.workspace = bw.data_ptr()
-        bargs.workspace_bytes = bws
-        cur = torch.cuda.current_stream(v.device)
+        _ext.set_workspace(bargs, bw.data_ptr(), bws)
         _ext.check(L.saf_mixed_attn_bwd(bargs, _ext.tensor_desc(do), _ext.tensor_desc(dq),
-                                        _ext.tensor_desc(dk), _ext.tensor_desc(dv), cur.cuda_stream))
+                                        _ext.tensor_desc(dk), _ext.tensor_desc(dv),
+                                        _ext.current_stream_ptr(dev)))
         _ = (keep, held, out_saved)  # what the argument block points to
         gq = dq.to(q.dtype) if dq is not None and q is not None else None
         gk = dk.to(k.dtype) if dk is not None and k is not None else None
         return gq, gk, dv
 
-    if needs_grad:
-        return _MixedAttnFn.apply(q, k, v, run, bwd)
-    return run()
+    return _MixedAttnFn.apply(q, k, v, run, bwd)
+
+
+def _timed_run(args, states, n_scan, n_dec, B, T, HD, v, decomp_unsplit):
+    """The forward's schedule through the per-kind entry points, each kernel
+    timed on its own stream (KernelTimer): decomposed heads beside live ones
+    run one workgroup per query block (decomp_unsplit = 1), so the live-head
+    kernel's workgroups fill the slots their causal imbalance leaves idle and
+    no key-segment partials are needed.  Returns the raw current stream."""
+    L, timer = _ext.lib(), _TIMER
+    n_live, n_dense = states.count(0), states.count(1)
+    work = {"flash": (L.saf_flash_fwd, n_live * B * 4 * HD * T * (T + 1) // 2),
+            "scan": (L.saf_frozen_scan_fwd, n_scan * B * 2 * T * HD * v.element_size()),
+            "dense": (L.saf_frozen_dense_pv_fwd, n_dense * B * 2 * HD * T * (T + 1) // 2),
+            "decomp": (L.saf_frozen_decomp_fwd, n_dec * B * 2 * HD * T * (T + 1) // 2)}
+    cur = torch.cuda.current_stream(v.device)
+
+    def launch(kind, strm):  # one timed per-kind call
+        fn, w = work[kind]
+        e0 = torch.cuda.Event(enable_timing=True)
+        e1 = torch.cuda.Event(enable_timing=True)
+        e0.record(strm)  # creates the HIP events; the library re-records them
+        e1.record(strm)
+        _ext.check(L.saf_time_next_kernel(e0.cuda_event, e1.cuda_event))
+        rc = fn(args, strm.cuda_stream)
+        L.saf_time_next_kernel(None, None)  # never left pending for a later call
+        _ext.check(rc)
+        timer.records[kind].append((e0, e1, w))
+
+    unsplit = bool(n_live) if decomp_unsplit is None else bool(decomp_unsplit)
+    args.decomp_unsplit = 1 if unsplit else -1
+    dec_side = bool(n_dec and n_live and unsplit)
+    if (n_scan and (n_live or n_dense or n_dec)) or dec_side:
+        # disjoint output rows and workspace regions; joined before returning
+        side = _side_stream(v.device)
+        side.wait_stream(cur)
+        if dec_side:
+            launch("decomp", side)
+        if n_scan:
+            launch("scan", side)
+        for kind in ("flash", "dense", "decomp"):
+            if work[kind][1] and not (kind == "decomp" and dec_side):
+                launch(kind, cur)
+        cur.wait_stream(side)
+    else:
+        for kind in KernelTimer.KINDS:
+            if work[kind][1]:
+                launch(kind, cur)
+    return cur.cuda_stream
 
 
 def _validate(q, k, v, patt, frozen, hidx, pidx, alpha, rho, z, rho_band, kvidx):

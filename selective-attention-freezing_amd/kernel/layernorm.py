@@ -16,21 +16,29 @@ import torch
 from . import _ext
 
 
+def _norm_args(x, delta, weight):
+    """The new output (x's shape, contiguous) and the descriptors of x, delta
+    (a copy where its rows are not a view) and weight."""
+    C = x.size(-1)
+    out = torch.empty(x.shape, device=x.device, dtype=x.dtype)
+    if delta is not None and (delta.size(-1) != C or not delta.is_contiguous()):
+        delta = delta.reshape(-1, C)
+    d = _ext.tensor_desc(None) if delta is None else _ext.rows_desc(delta)
+    d.owner = delta  # a reshaped copy lives until the call is enqueued
+    return out, (_ext.rows_desc(x), d, _ext.tensor_desc(weight))
+
+
 def add_layernorm_(x, delta, weight, bias=None, eps=1e-5):
     """x (..., C) residual, updated in place to x + delta (delta None: left
     as is); returns LayerNorm(x) * weight + bias as a new tensor of x's shape."""
     if not x.is_cuda:
         raise RuntimeError("add_layernorm_ runs on HIP devices only (got a CPU tensor)")
-    C = x.size(-1)
-    x2 = x.view(-1, C)
-    d2 = None if delta is None else delta.reshape(-1, C)
-    out = torch.empty_like(x2)
-    L = _ext.lib()
-    rc = L.saf_add_layernorm(_ext.tensor_desc(x2), _ext.tensor_desc(d2), _ext.tensor_desc(weight.detach()),
-                             _ext.tensor_desc(None if bias is None else bias.detach()), float(eps),
-                             _ext.tensor_desc(out), _ext.current_stream_ptr(x.device))
-    _ext.check(rc)
-    return out.view(x.shape)
+    out, args = _norm_args(x, delta, weight)
+    rc = _ext.lib().saf_add_layernorm(*args, _ext.tensor_desc(bias), float(eps), _ext.rows_desc(out),
+                                      _ext.current_stream_ptr(x.device))
+    if rc:
+        _ext.check(rc)
+    return out
 
 
 def add_rmsnorm_(x, delta, weight, eps=1e-6):
@@ -39,12 +47,8 @@ def add_rmsnorm_(x, delta, weight, eps=1e-6):
     tensor of x's shape (Qwen3RMSNorm's rounding)."""
     if not x.is_cuda:
         raise RuntimeError("add_rmsnorm_ runs on HIP devices only (got a CPU tensor)")
-    C = x.size(-1)
-    x2 = x.view(-1, C)
-    d2 = None if delta is None else delta.reshape(-1, C)
-    out = torch.empty_like(x2)
-    L = _ext.lib()
-    rc = L.saf_add_rmsnorm(_ext.tensor_desc(x2), _ext.tensor_desc(d2), _ext.tensor_desc(weight.detach()),
-                           float(eps), _ext.tensor_desc(out), _ext.current_stream_ptr(x.device))
-    _ext.check(rc)
-    return out.view(x.shape)
+    out, args = _norm_args(x, delta, weight)
+    rc = _ext.lib().saf_add_rmsnorm(*args, float(eps), _ext.rows_desc(out), _ext.current_stream_ptr(x.device))
+    if rc:
+        _ext.check(rc)
+    return out

@@ -32,15 +32,23 @@ def _gemm_usable(x, weight):
             and weight.size(0) % _N_MULT == 0 and weight.size(1) % _K_MULT == 0)
 
 
-def _rows(x, weight):
-    K = x.size(-1)
-    x2 = x.reshape(-1, K)
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
-    w = weight.detach()
-    if w.stride(-1) != 1:
-        w = w.contiguous()
-    return x2, w
+def _gemm(fn, x, weight, n_out, *tail):
+    """fn(x, weight, out, *tail, stream) over the rows of x (..., K); returns
+    out (..., n_out)."""
+    if x.is_contiguous():
+        xd = _ext.rows_desc(x)
+    else:
+        x2 = x.reshape(-1, x.size(-1))
+        x2 = x2 if x2.stride(-1) == 1 else x2.contiguous()
+        xd = _ext.tensor_desc(x2)
+    w = weight if weight.stride(-1) == 1 else weight.contiguous()
+    out = torch.empty((*x.shape[:-1], n_out), device=x.device, dtype=x.dtype)
+    if out.numel() == 0:
+        return out
+    rc = fn(xd, _ext.tensor_desc(w), _ext.rows_desc(out), *tail, _ext.current_stream_ptr(x.device))
+    if rc:
+        _ext.check(rc)
+    return out
 
 
 def linear_gelu_usable(x, weight):
@@ -70,15 +78,7 @@ def linear_gelu(x, weight):
     """gelu(x @ weight.T) for x (..., K) and weight (N, K); returns (..., N)."""
     if not x.is_cuda:
         raise RuntimeError("linear_gelu runs on HIP devices only (got a CPU tensor)")
-    x2, w = _rows(x, weight)
-    out = torch.empty(x2.size(0), w.size(0), device=x.device, dtype=x.dtype)
-    if out.numel() == 0:
-        return out.view(*x.shape[:-1], w.size(0))
-    L = _ext.lib()
-    rc = L.saf_linear_gelu(_ext.tensor_desc(x2), _ext.tensor_desc(w), _ext.tensor_desc(out),
-                           _ext.current_stream_ptr(x.device))
-    _ext.check(rc)
-    return out.view(*x.shape[:-1], w.size(0))
+    return _gemm(_ext.lib().saf_linear_gelu, x, weight, weight.size(0))
 
 
 SWIGLU_BLOCK = 64  # rows per gate / up block of the interleaved weight
@@ -104,15 +104,7 @@ def linear_swiglu(x, weight):
     of swiglu_weight(Wg, Wu); returns (..., I)."""
     if not x.is_cuda:
         raise RuntimeError("linear_swiglu runs on HIP devices only (got a CPU tensor)")
-    x2, w = _rows(x, weight)
-    out = torch.empty(x2.size(0), w.size(0) // 2, device=x.device, dtype=x.dtype)
-    if out.numel() == 0:
-        return out.view(*x.shape[:-1], w.size(0) // 2)
-    L = _ext.lib()
-    rc = L.saf_linear_swiglu(_ext.tensor_desc(x2), _ext.tensor_desc(w), _ext.tensor_desc(out),
-                             _ext.current_stream_ptr(x.device))
-    _ext.check(rc)
-    return out.view(*x.shape[:-1], w.size(0) // 2)
+    return _gemm(_ext.lib().saf_linear_swiglu, x, weight, weight.size(0) // 2)
 
 
 def linear_rope_usable(x, weight, n_rope, head_dim, cos):
@@ -131,16 +123,6 @@ def linear_rope(x, weight, n_rope, head_dim, cos, sin):
         raise RuntimeError("linear_rope runs on HIP devices only (got a CPU tensor)")
     if x.dim() != 3:
         raise ValueError("linear_rope takes x as (B, T, K)")
-    T = x.size(1)
-    x2, w = _rows(x, weight)
-    out = torch.empty(x2.size(0), w.size(0), device=x.device, dtype=x.dtype)
-    if out.numel() == 0:
-        return out.view(x.size(0), T, w.size(0))
-    cos2 = cos.reshape(-1, cos.size(-1))
-    sin2 = sin.reshape(-1, sin.size(-1))
-    L = _ext.lib()
-    rc = L.saf_linear_rope(_ext.tensor_desc(x2), _ext.tensor_desc(w), _ext.tensor_desc(out), int(n_rope),
-                           int(head_dim), int(T), _ext.tensor_desc(cos2), _ext.tensor_desc(sin2),
-                           _ext.current_stream_ptr(x.device))
-    _ext.check(rc)
-    return out.view(x.size(0), T, w.size(0))
+    cos2, sin2 = (t.reshape(-1, t.size(-1)) for t in (cos, sin))
+    return _gemm(_ext.lib().saf_linear_rope, x, weight, weight.size(0), int(n_rope), int(head_dim), x.size(1),
+                 _ext.tensor_desc(cos2), _ext.tensor_desc(sin2))
