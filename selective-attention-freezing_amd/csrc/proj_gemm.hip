@@ -41,19 +41,29 @@
 // steps of a tile load the first k tiles of the next, which land while the
 // epilogue runs.  The 16-byte chunks of a tile row are XOR-swizzled by the
 // row so that the reads of a 16-lane group hit distinct banks.
+// Problems of few tiles run the same loop on 128 x 128 tiles, two workgroups
+// of 4 waves (64 x 64 blocks) per CU (proj_small).
 #include "saf_kernels.h"
 
 namespace saf {
 
 namespace {
 
-constexpr int kGBM = 256, kGBN = 256, kGBK = 32, kGStages = 4, kGWaves = 8;
+constexpr int kGBK = 32, kGStages = 4, kGDma = 2;
 constexpr int kGRowBytes = kGBK * 2;          // one k-tile row (64 bytes)
-constexpr int kGTileBytes = kGBM * kGRowBytes;  // one operand's k tile (16 KB)
 constexpr int kGChunks = kGBK / 8;            // 16-byte chunks per row
-constexpr int kGDma = kGBM * kGChunks / (64 * kGWaves);  // DMA loads per thread, operand and step
-static_assert(kGBM == kGBN, "both operand tiles have kGBM rows");
-static_assert(kGDma * 64 * kGWaves == kGBM * kGChunks, "DMA chunks split evenly over the threads");
+
+// Tile shape: kTile rows of both operands; kNT 32-row subtiles of W per wave
+// (two of A); kPerCu workgroups per CU.
+struct BigTile {
+  static constexpr int kTile = 256, kWaves = 8, kNT = 4, kPerCu = 1;
+};
+struct SmallTile {
+  static constexpr int kTile = 128, kWaves = 4, kNT = 2, kPerCu = 2;
+};
+template <typename TL> constexpr bool tile_ok =
+    kGDma * 64 * TL::kWaves == TL::kTile * kGChunks && TL::kWaves * 64 * 32 * TL::kNT == TL::kTile * TL::kTile;
+static_assert(tile_ok<BigTile> && tile_ok<SmallTile>, "DMA chunks and wave blocks split a tile evenly");
 
 // logical chunk c of row r sits at chunk c ^ swz(r): rows r .. r + 15 of one
 // chunk land on 16 distinct 4-bank groups (row pitch 64 bytes); the swizzle
@@ -121,10 +131,15 @@ __device__ __forceinline__ void gelu_group(float (&x)[n]) {
 
 enum : int { kEpiGelu = 0, kEpiRope = 1, kEpiSwiglu = 2 };
 
-// EPI: kEpiGelu, or kEpiRope with head dimension HD (64 or 128)
-template <typename T, int EPI, int HD>
-__global__ __launch_bounds__(64 * kGWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// EPI: kEpiGelu, kEpiSwiglu, or kEpiRope with head dimension HD (64 or 128)
+template <typename T, int EPI, int HD, typename TL>
+__global__ __launch_bounds__(64 * TL::kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void proj_gemm_kernel(const ProjGemmParams p) {
+  constexpr int kGBM = TL::kTile, kGBN = TL::kTile, kGWaves = TL::kWaves, NT = TL::kNT;
+  constexpr int kGTileBytes = TL::kTile * kGRowBytes;  // one operand's k tile
+  // rows between a wave's W subtiles: a small tile's wave has two, which must
+  // hold both members of a rotation pair or a gate and its up features
+  constexpr int kWStep = NT == 2 && (EPI == kEpiSwiglu || (EPI == kEpiRope && HD == 128)) ? 64 : 32;
   // one array per operand and stage, so that the compiler's wait insertion
   // sees that a read of one stage does not depend on the DMAs into the others
   __shared__ __align__(16) char sw0[kGTileBytes], sw1[kGTileBytes], sw2[kGTileBytes], sw3[kGTileBytes];
@@ -202,28 +217,30 @@ void proj_gemm_kernel(const ProjGemmParams p) {
                                                woff[q], so, 0, 0);
   };
 
-  // read offsets of this lane: W rows 128 wn + 32 nt + n32, A rows
-  // 64 wm + 32 mt + n32, logical chunk 2 s + g for k substep s; the 32-row
-  // subtiles nt / mt sit 2 KB apart
+  // read offsets of this lane: W rows w0 + kWStep nt + n32, A rows
+  // 64 wm + 32 mt + n32, logical chunk 2 s + g for k substep s; 32 rows are
+  // 2 KB
+  const int w0 = kWStep == 64 ? 32 * wn : 32 * NT * wn;
   int wrd[2], ard[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    wrd[s] = gtile_off(128 * wn + n32, 2 * s + g);
+    wrd[s] = gtile_off(w0 + n32, 2 * s + g);
     ard[s] = gtile_off(64 * wm + n32, 2 * s + g);
   }
   constexpr int kSub = 32 * kGRowBytes;
 
-  f32x16_t acc[4][2];
-  auto read_sub = [&](auto stage, auto sub, uint4 (&wa)[4], uint4 (&ab)[2]) {
+  f32x16_t acc[NT][2];
+  auto read_sub = [&](auto stage, auto sub, uint4 (&wa)[NT], uint4 (&ab)[2]) {
     constexpr int s = decltype(sub)::value;
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) wa[nt] = *reinterpret_cast<const uint4*>(wst(stage) + wrd[s] + nt * kSub);
+    for (int nt = 0; nt < NT; ++nt)
+      wa[nt] = *reinterpret_cast<const uint4*>(wst(stage) + wrd[s] + nt * (kWStep / 32) * kSub);
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) ab[mt] = *reinterpret_cast<const uint4*>(ast(stage) + ard[s] + mt * kSub);
   };
-  auto mma = [&](const uint4 (&wa)[4], const uint4 (&ab)[2]) {
+  auto mma = [&](const uint4 (&wa)[NT], const uint4 (&ab)[2]) {
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) acc[nt][mt] = Elem<T>::mfma(wa[nt], ab[mt], acc[nt][mt]);
   };
@@ -241,7 +258,7 @@ void proj_gemm_kernel(const ProjGemmParams p) {
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(4 * kGDma));  // step 0 landed, steps 1, 2 in flight
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  uint4 wa0[4], ab0[2], wa1[4], ab1[2];
+  uint4 wa0[NT], ab0[2], wa1[NT], ab1[2];
   read_sub(G0(), Sub0(), wa0, ab0);
 
   // k step j in stage j % 4 (nk is a multiple of 4, so every tile starts at
@@ -275,7 +292,7 @@ void proj_gemm_kernel(const ProjGemmParams p) {
 
   for (int i = 1;; ++i) {
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) acc[nt][mt] = zero16();
     for (int j = 0; j < nk; j += kGStages) {
@@ -287,7 +304,7 @@ void proj_gemm_kernel(const ProjGemmParams p) {
 
     // epilogue of tile cur (the next tile's first k tiles are in flight):
     // lane (n32, g), tile (nt, mt), register 4 q + e holds C[row][col],
-    // row = m0 + 64 wm + 32 mt + n32, col = n0 + 128 wn + 32 nt + 8 q + 4 g + e.
+    // row = m0 + 64 wm + 32 mt + n32, col = n0 + w0 + kWStep nt + 8 q + 4 g + e.
     // v_permlane32_swap(vdst, vsrc) exchanges vdst of lanes 32..63 with vsrc
     // of lanes 0..31: with vdst = piece q = 2 r and vsrc = piece 2 r + 1, lane
     // (n32, 0) ends with columns 16 r + 0..7 and lane (n32, 1) with
@@ -298,13 +315,15 @@ void proj_gemm_kernel(const ProjGemmParams p) {
       const int row = m0 + 64 * wm + 32 * mt + n32;
       if constexpr (EPI == kEpiRope) {
         // the wave's 128 columns are two heads (hd 64: pairs nt 0 / 1 and
-        // 2 / 3, the same d for both) or one (hd 128: pairs nt 0 / 2 and 1 / 3),
-        // all rotated or none (n_rope is a multiple of 128)
-        if (n0 + 128 * wn < p.n_rope) {
+        // 2 / 3, the same d for both) or one (hd 128: pairs nt 0 / 2 and 1 / 3);
+        // a small tile's 64 are one head (pair 0 / 1) or the half of one with
+        // d = 32 wn + 0..31 and its partners; all rotated or none (n_rope is a
+        // multiple of 128)
+        if (n0 + (NT == 4 ? 128 * wn : 0) < p.n_rope) {
           const int t = (row < p.M ? row : 0) % p.T;
           const uint16_t* cs = reinterpret_cast<const uint16_t*>(p.cos) + (int64_t)t * p.cs_st + 4 * g;
           const uint16_t* sn = reinterpret_cast<const uint16_t*>(p.sin) + (int64_t)t * p.sn_st + 4 * g;
-          constexpr int kHalf = HD / 2, kPairs = HD == 64 ? 1 : 2;
+          constexpr int kHalf = HD / 2, kPairs = HD == 64 || NT == 2 ? 1 : 2;
 #pragma unroll
           for (int pi = 0; pi < kPairs; ++pi) {
             // cos / sin at d1 = 32 pi + 8 q + 4 g + e and d1 + hd/2, in the
@@ -312,7 +331,7 @@ void proj_gemm_kernel(const ProjGemmParams p) {
             uint2 c1[4], s1[4], c2[4], s2[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              const int d1 = 32 * pi + 8 * q;
+              const int d1 = (kWStep == 64 ? 32 * wn : 32 * pi) + 8 * q;
               c1[q] = *reinterpret_cast<const uint2*>(cs + d1);
               s1[q] = *reinterpret_cast<const uint2*>(sn + d1);
               c2[q] = *reinterpret_cast<const uint2*>(cs + d1 + kHalf);
@@ -329,8 +348,8 @@ void proj_gemm_kernel(const ProjGemmParams p) {
                 const float fc2 = e % 2 ? Elem<T>::hi(wc2) : Elem<T>::lo(wc2);
                 const float fs2 = e % 2 ? Elem<T>::hi(ws2) : Elem<T>::lo(ws2);
 #pragma unroll
-                for (int hh = 0; hh < 2 / kPairs; ++hh) {
-                  const int lo = HD == 64 ? 2 * hh : pi, hi = HD == 64 ? 2 * hh + 1 : pi + 2;
+                for (int hh = 0; hh < NT / 2 / kPairs; ++hh) {
+                  const int lo = HD == 64 ? 2 * hh : pi, hi = lo + (HD == 64 ? 1 : NT / 2);
                   const float x1 = acc[lo][mt][4 * q + e], x2 = acc[hi][mt][4 * q + e];
                   acc[lo][mt][4 * q + e] = x1 * fc1 - x2 * fs1;
                   acc[hi][mt][4 * q + e] = x2 * fc2 + x1 * fs2;
@@ -340,12 +359,12 @@ void proj_gemm_kernel(const ProjGemmParams p) {
           }
         }
       }
-      // SwiGLU: the wave's 128 columns are 64 gate features (nt 0, 1) and the
-      // same 64 up features (nt 2, 3); it writes their 64 products at output
-      // column n0 / 2 + 64 wn + d, d = 32 nt + 8 q + 4 g + e
-      constexpr int kOutTiles = EPI == kEpiSwiglu ? 2 : 4;
+      // SwiGLU: the wave's columns are 16 NT gate features (nt < NT / 2) and
+      // the same up features (nt + NT / 2); it writes their products at output
+      // column n0 / 2 + 16 NT wn + d, d = 32 nt + 8 q + 4 g + e
+      constexpr int kOutTiles = EPI == kEpiSwiglu ? NT / 2 : NT;
       T* crow = reinterpret_cast<T*>(p.c) + (int64_t)row * p.c_rs +
-                (EPI == kEpiSwiglu ? n0 / 2 + 64 * wn : n0 + 128 * wn) + 8 * g;
+                (EPI == kEpiSwiglu ? n0 / 2 + 16 * NT * wn : n0 + w0) + 8 * g;
 #pragma unroll
       for (int nt = 0; nt < kOutTiles; ++nt)
 #pragma unroll
@@ -357,7 +376,7 @@ void proj_gemm_kernel(const ProjGemmParams p) {
           if constexpr (EPI == kEpiGelu) gelu_group(y);
           if constexpr (EPI == kEpiSwiglu) {
             // silu(x) = x / (1 + e^-x), in fp32, times the up projection
-            const f32x16_t& up = acc[nt + 2][mt];
+            const f32x16_t& up = acc[nt + NT / 2][mt];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
               const float x = y[i];
@@ -372,7 +391,8 @@ void proj_gemm_kernel(const ProjGemmParams p) {
           }
           const auto s0 = __builtin_amdgcn_permlane32_swap(pc[0][0], pc[1][0], false, false);
           const auto s1 = __builtin_amdgcn_permlane32_swap(pc[0][1], pc[1][1], false, false);
-          if (row < p.M) *reinterpret_cast<uint4*>(crow + 32 * nt + 16 * r) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+          if (row < p.M) *reinterpret_cast<uint4*>(crow + (EPI == kEpiSwiglu ? 32 : kWStep) * nt + 16 * r) =
+                make_uint4(s0[0], s1[0], s0[1], s1[1]);
         }
     }
     if (nxt < 0) break;
@@ -430,25 +450,48 @@ hipError_t launch_gelu_inplace(void* x, int64_t n, int dtype, int n_cu, hipStrea
 }
 
 bool proj_gemm_shape_ok(int64_t M, int64_t N, int64_t K) {
-  return M > 0 && N > 0 && K > 0 && N % kGBN == 0 && K % (kGBK * kGStages) == 0;
+  return M > 0 && N > 0 && K > 0 && N % BigTile::kTile == 0 && K % (kGBK * kGStages) == 0;
 }
 
 namespace {
 
-// one workgroup per CU (a multiple of the 8 XCDs), fewer for small problems
+// kPerCu workgroups per CU (a multiple of the 8 XCDs), fewer for small problems
+template <typename TL>
 dim3 proj_grid(const ProjGemmParams& p) {
-  const int tiles = ((p.M + kGBM - 1) / kGBM) * (p.N / kGBN);
+  const int tiles = ((p.M + TL::kTile - 1) / TL::kTile) * (p.N / TL::kTile);
   const int per_xcd = (tiles + 7) / 8;
-  const int n_local = max(1, min(p.n_cu / 8, per_xcd));
+  const int n_local = max(1, min(p.n_cu / 8 * TL::kPerCu, per_xcd));
   return dim3((unsigned)(8 * n_local));
+}
+
+// Small tiles where the big ones would leave half of the CUs or more without
+// work: a 256 x 256 tile takes its 20 to 30 us whether 8 or 256 of them run,
+// four 128 x 128 tiles spread over four CUs.  Measured (us, big / small): GELU
+// N=3072 K=768, M=1024 21.4 / 13.9, M=2048 (96 big tiles) 24.3 / 20.5, M=3072
+// (144) 25.1 / 26.9; RoPE N=2048, M=1024 26.7 / 13.3, M=4096 (128) 29.5 /
+// 26.3, M=6144 (192) 31.6 / 36.2; SwiGLU N=9728 K=896, M=512 (76) 22.8 / 20.4,
+// M=1024 (152) 24.5 / 30.5.
+bool proj_small(const ProjGemmParams& p) {
+  const int big = ((p.M + BigTile::kTile - 1) / BigTile::kTile) * (p.N / BigTile::kTile);
+  return 2 * big <= p.n_cu;
+}
+
+template <typename T, int EPI, int HD>
+void launch_proj_t(const ProjGemmParams& p, hipStream_t s) {
+  if (proj_small(p))
+    hipLaunchKernelGGL((proj_gemm_kernel<T, EPI, HD, SmallTile>), proj_grid<SmallTile>(p), dim3(64 * SmallTile::kWaves),
+                       0, s, p);
+  else
+    hipLaunchKernelGGL((proj_gemm_kernel<T, EPI, HD, BigTile>), proj_grid<BigTile>(p), dim3(64 * BigTile::kWaves), 0,
+                       s, p);
 }
 
 template <int EPI, int HD>
 hipError_t launch_proj(const ProjGemmParams& p, int dtype, hipStream_t s) {
   if (dtype == kBF16)
-    hipLaunchKernelGGL((proj_gemm_kernel<__bf16, EPI, HD>), proj_grid(p), dim3(64 * kGWaves), 0, s, p);
+    launch_proj_t<__bf16, EPI, HD>(p, s);
   else if (dtype == kF16)
-    hipLaunchKernelGGL((proj_gemm_kernel<_Float16, EPI, HD>), proj_grid(p), dim3(64 * kGWaves), 0, s, p);
+    launch_proj_t<_Float16, EPI, HD>(p, s);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
