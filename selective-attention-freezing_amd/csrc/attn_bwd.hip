@@ -89,8 +89,9 @@ __device__ __forceinline__ uint4 neg_halves(uint4 w) {
 
 }  // namespace
 
-// delta[b, slot, i] = sum_d out[b, h, i, d] * dout[b, h, i, d] over the live
-// rows, fp32.  A row is read by delta_lanes(HD) lanes, 16 bytes each, so one
+// delta[b, slot, i] = sum_d out[b, h, i, d] * dout[b, h, i, d] of the rows of
+// the decomposed heads whose parameter gradients follow (the live heads' comes
+// out of the dQ kernel), fp32.  A row is read by delta_lanes(HD) lanes, 16 bytes each, so one
 // load instruction covers whole rows (one lane per row touched 64 rows per
 // instruction), and the lanes' sums meet by shuffles.
 constexpr int delta_lanes(int hd) { return hd <= 32 ? 4 : (hd <= 64 ? 8 : (hd <= 128 ? 16 : 32)); }
@@ -151,19 +152,33 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(const BwdParams p) {
   const T* kbase = reinterpret_cast<const T*>(p.k) + b * p.k_sb + (int64_t)qs * p.k_sh;
   const T* vbase = reinterpret_cast<const T*>(p.v) + b * p.v_sb + (int64_t)h * p.v_sh;
   const T* dobase = reinterpret_cast<const T*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh;
+  const T* obase = reinterpret_cast<const T*>(p.out) + b * p.o_sb + (int64_t)h * p.o_sh;
   T* dqbase = reinterpret_cast<T*>(p.dq) + b * p.dq_sb + (int64_t)qs * p.dq_sh;
 
   const int q0w = qb * BM + wave * 32;
   const int q = q0w + n;
   const bool qv = q < T_len;
-  uint4 qf[NKT], dof[NKT];
+  uint4 qf[NKT], dof[NKT], of[NKT];
 #pragma unroll
   for (int t = 0; t < NKT; ++t) {
     qf[t] = qv ? load16(qbase + (int64_t)q * p.q_st + 16 * t + 8 * g) : make_uint4(0, 0, 0, 0);
     dof[t] = qv ? load16(dobase + (int64_t)q * p.do_st + 16 * t + 8 * g) : make_uint4(0, 0, 0, 0);
+    of[t] = qv ? load16(obase + (int64_t)q * p.o_st + 16 * t + 8 * g) : make_uint4(0, 0, 0, 0);
   }
   const float lse2 = qv ? p.lse[b * p.l_sb + (int64_t)h * p.l_sh + (int64_t)q * p.l_st] : 0.f;
-  const float dl = qv ? p.delta[((int64_t)b * p.n_live + slot) * T_len + q] : 0.f;
+  // delta of this lane's row (each half of the wave holds half of it), stored
+  // for the dK / dV kernel that runs after this one: a pass of its own over
+  // out and dout took 15 us at B=8, 9 live heads, T=4096
+  float dl = 0.f;
+#pragma unroll
+  for (int t = 0; t < NKT; ++t) {
+    const uint32_t wo[4] = {of[t].x, of[t].y, of[t].z, of[t].w}, wd[4] = {dof[t].x, dof[t].y, dof[t].z, dof[t].w};
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      dl += Elem<T>::lo(wo[m]) * Elem<T>::lo(wd[m]) + Elem<T>::hi(wo[m]) * Elem<T>::hi(wd[m]);
+  }
+  dl = half_swap_sum(dl);
+  if (qv && g == 0) p.delta[((int64_t)b * p.n_live + slot) * T_len + q] = dl;
   const float c = p.scale_log2;
   f32x16_t dqa[NDT];
 #pragma unroll
@@ -273,7 +288,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(dkdv_waves_
 void bwd_dkdv_kernel(const BwdParams p) {
   constexpr int BN = kBwdWaves * 32, NKT = HD / 16, NDT = HD / 32, VB = VRow<HD>::BYTES;
   constexpr int kOps = 2 * TileOffsets<T, HD>::VN + 1;  // loads per wave per block
-  constexpr bool kBatch = dkdv_waves_per_eu(HD) == 1;
+  constexpr bool kBatch = HD >= 64;
   __shared__ __align__(16) char q0[VB], q1[VB], q2[VB], o0[VB], o1[VB], o2[VB];
   __shared__ __align__(16) float ls0[4][64], ls1[4][64], ls2[4][64];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -360,10 +375,11 @@ void bwd_dkdv_kernel(const BwdParams p) {
       for (int i2 = 0; i2 < 16; ++i2) dp[i2] = ls[2 + qs2][acc_key(i2, g)];
       uint4 co[2][NDT], cq[2][NDT];  // column operands of the dV / dK products (kBatch)
       if constexpr (kBatch) {
-        // one wave per SIMD: no other wave covers the LDS latency, so the
-        // row operands are read in one batch before the S / dP MFMAs and the
-        // column operands before the softmax VALU work (the scheduler keeps
-        // each read next to its MFMA otherwise)
+        // the row operands are read in one batch before the S / dP MFMAs, the
+        // two chains in turn, and the column operands before the softmax VALU
+        // work (the scheduler keeps each read next to its MFMA otherwise):
+        // hd 128, one wave per SIMD, 1375 -> 1218 us; hd 64, two waves, 373 ->
+        // 358 us (at hd 32 three waves cover the reads)
         uint4 qa[NKT], oa[NKT];
 #pragma unroll
         for (int t = 0; t < NKT; ++t) {
@@ -986,7 +1002,7 @@ static hipError_t bwd_launch(const BwdParams& p, int hd, int which, hipStream_t 
 }
 
 static hipError_t bwd_dispatch(const BwdParams& p, int dtype, int hd, int which, hipStream_t s) {
-  if (dtype == kF32) return which <= 3 ? launch_f32_bwd(p, hd, which, s) : hipErrorInvalidValue;
+  if (dtype == kF32) return which >= 1 && which <= 3 ? launch_f32_bwd(p, hd, which, s) : hipErrorInvalidValue;
   if (dtype == kBF16) return bwd_launch<__bf16>(p, hd, which, s);
   if (dtype == kF16) return bwd_launch<_Float16>(p, hd, which, s);
   return hipErrorInvalidValue;

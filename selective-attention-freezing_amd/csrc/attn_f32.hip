@@ -740,8 +740,6 @@ hipError_t f32_bwd_hd(const BwdParams& p, int which, hipStream_t s) {
   const int64_t nt = (p.T + kR - 1) / kR;
   const dim3 live((unsigned)(nt * p.n_live * p.B)), frozen((unsigned)(nt * p.n_frozen * p.B));
   switch (which) {
-    case 0:  // delta comes out of the dQ kernel
-      break;
     case 1:
       hipLaunchKernelGGL((f32_bwd_dq_kernel<HD>), live, dim3(64 * kW), 0, s, p);
       break;

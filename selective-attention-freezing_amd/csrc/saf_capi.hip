@@ -1355,8 +1355,7 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
   int rc = SAF_OK;
   if (nf > 0) rc = launched(launch_bwd_frozen_dv(p, pl.dtype, pl.HD, ss != nullptr ? ss->s : s), "backward frozen dv");
   if (rc == SAF_OK && !pl.live.empty()) {
-    rc = launched(launch_bwd_delta(p, pl.dtype, pl.HD, s), "backward delta");
-    if (rc == SAF_OK) rc = launched(launch_bwd_dq(p, pl.dtype, pl.HD, s), "backward dq");
+    rc = launched(launch_bwd_dq(p, pl.dtype, pl.HD, s), "backward dq");  // and delta
     if (rc == SAF_OK) rc = launched(launch_bwd_dkdv(p, pl.dtype, pl.HD, s), "backward dk/dv");
   }
   if (ss != nullptr) {

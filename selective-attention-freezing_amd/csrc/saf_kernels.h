@@ -305,8 +305,9 @@ struct BwdParams {
 };
 static_assert(sizeof(BwdParams) <= 4096, "BwdParams must fit the kernel argument segment");
 
-// Backward: delta = rowsum(out * dout) of the live rows; dQ; dK and dV of the
-// live heads; dV of the frozen heads.
+// Backward: dQ and delta = rowsum(out * dout) of the live rows; dK and dV of the
+// live heads (after dQ); dV of the frozen heads.  launch_bwd_delta: delta alone,
+// for the decomposed heads' parameter gradients.
 hipError_t launch_bwd_delta(const BwdParams& p, int dtype, int hd, hipStream_t s);
 hipError_t launch_bwd_dq(const BwdParams& p, int dtype, int hd, hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdParams& p, int dtype, int hd, hipStream_t s);
@@ -316,8 +317,7 @@ hipError_t launch_bwd_frozen_dv(const BwdParams& p, int dtype, int hd, hipStream
 hipError_t launch_bwd_decomp_param(const BwdParams& p, int dtype, int hd, hipStream_t s);
 
 // float32 inputs (attn_f32.hip): the same parameter blocks, no causal split
-// (n_items 0), no work queue; which: 0 nothing (the dQ kernel writes delta),
-// 1 dQ and delta, 2 dK / dV, 3 frozen dV.
+// (n_items 0), no work queue; which: 1 dQ and delta, 2 dK / dV, 3 frozen dV.
 hipError_t launch_f32_live(const FlashParams& p, int hd, hipStream_t s);
 hipError_t launch_f32_frozen(const FrozenParams& p, int hd, int mode, hipStream_t s);
 hipError_t launch_f32_bwd(const BwdParams& p, int hd, int which, hipStream_t s);
