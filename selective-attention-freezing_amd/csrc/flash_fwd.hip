@@ -327,7 +327,7 @@ struct FlashState {
 // registers).  hd 96 / 128: one workgroup's three K and V slots fill most of
 // the CU's LDS, so the workgroup has 8 waves (two per SIMD) sharing them.
 // hd 256: 4 waves, one per SIMD (512 registers each), over two slots per
-// operand.  The host's flash_resident() and flash_block_rows() mirror this.
+// operand.  The host's flash_block_rows() mirrors this.
 template <int HD, int QT>
 constexpr int flash_waves_per_eu() { return HD <= 64 ? (QT == 1 ? 3 : 2) : (HD <= 128 && QT == 1 ? 2 : 1); }
 

@@ -25,7 +25,7 @@
 
 namespace saf {
 
-// Resident decomposed workgroups per CU (decomp_resident() on the host):
+// Resident decomposed workgroups per CU:
 // three up to hd 64; two above, where the factored form's three V' slots and
 // two distance windows take 62.5 KB of LDS (three workgroups need <= 53 KB)
 // and hd 256's 128 accumulator registers per wave need the 256-register

@@ -250,12 +250,6 @@ int cu_count() {
   return cached_cus;
 }
 
-// Resident live-head workgroups per CU (flash_waves_per_eu in the kernel:
-// three 128-query workgroups at hd <= 64, two of 256 queries; one 8-wave
-// workgroup at hd 96 / 128, where its LDS slots fill most of the CU; one
-// 4-wave workgroup of 128 queries at hd 256, one wave per SIMD).
-int flash_resident(int HD, int qt) { return HD <= 64 ? (qt == 1 ? 3 : 2) : 1; }
-
 struct FlashPlan {
   int n_items = 0, seg_len = 0, n_part_per_head = 0, n_split = 0;
   std::vector<int32_t> items;
@@ -263,51 +257,83 @@ struct FlashPlan {
   int64_t part_bytes = 0;  // workspace for the partials
 };
 
-// Splits the key range of the heaviest query blocks into segments of about
-// the average per-slot work, so the causal tail (the last query block walks
-// every key) does not outlast the rest of the grid.  B counts the work units
-// per slot; each writes part_mult sequences' partials.
-FlashPlan plan_flash(int B, int n_slots, int T, int HD, int BM, int per_cu, int part_mult = 1) {
+// Cost of one item, for plan_flash: us per key block (of 64 keys) and query
+// block of the kernel's shape, running alone on its CU.  Fitted to every
+// segment length measured at T = 512 .. 8192, 3 .. 96 (batch, head) pairs
+// (BM = 128 / 256 live at hd <= 64 / 96, 128; 256 / 128 decomposed at
+// hd <= 64 / above; 256 dense, whose cost is the pattern's bytes).
+float flash_block_us(int HD) { return HD <= 64 ? 1.15f : 1.7f; }
+float decomp_block_us(int HD) { return HD <= 64 ? 1.9f : 0.7f; }
+float dense_block_us(bool wide) { return wide ? 1.9f : 1.2f; }
+
+// Key segments for the heaviest query blocks, where they pay: the causal tail
+// (the last query block walks every key) outlasts a grid of few workgroups,
+// but a split writes fp32 partials and needs the combine's launch.  The time
+// of a plan is block_us * blocks + 8 us + partial bytes at 1.6 TB/s, where
+// blocks is the mean of two bounds: the work divided over the CUs (at least
+// the longest item), and the sum one CU gets when the items, longest first,
+// are dealt out in turn.  Measured, us, split by the per-slot work (at least
+// 8 or 16 blocks) / by this rule: hd 64, 12 heads T = 1024 19.7 / 17.2, B = 8
+// 38.6 / 27.3; T = 2048 31.8 / 26.1; T = 4096 55.7 / 51.3; hd 128, 8 heads
+// T = 4096 84 / 72; dense fp32, 6 heads T = 2048 47.5 / 34.4; decomposed, 24
+// heads T = 4096 hd 128 92.6 / 76.1.  B counts the work units per slot; each
+// writes part_mult sequences' partials.
+FlashPlan plan_flash(int B, int n_slots, int T, int HD, int BM, float block_us, int part_mult = 1) {
   FlashPlan fp;
   const int BMb = BM / 64;
   const int nqb = (T + BM - 1) / BM;
   if (nqb <= 1 || nqb > kMaxQblk) return fp;
-  std::vector<int> nkb(nqb);
-  int64_t per_head = 0;
-  for (int qb = 0; qb < nqb; ++qb) {
-    nkb[qb] = (std::min((qb + 1) * BM, T) + 63) / 64;
-    per_head += nkb[qb];
-  }
+  const int nk = (T + 63) / 64;
+  const auto blocks_of = [&](int qb) { return std::min((qb + 1) * BMb, nk); };
   const int64_t nbh = (int64_t)B * n_slots;
-  const int64_t slots = (int64_t)cu_count() * per_cu;
-  int64_t L = (nbh * per_head + slots - 1) / slots;
-  L = std::max<int64_t>(L, 4 * BMb);
-  L = (L + BMb - 1) / BMb * BMb;
-  for (;; L *= 2) {
-    if (L >= nkb[nqb - 1]) return fp;  // nothing to split
-    int64_t n = 0;
-    for (int qb = 0; qb < nqb; ++qb) n += (nkb[qb] + L - 1) / L;
-    if (n <= kMaxItems && L < 65536) break;
-  }
+  const double cus = cu_count();
+  const double work = (double)nbh * ((int64_t)nqb * (nqb - 1) / 2 * BMb + nk) / cus;
+  if (work > 1.5 * nk || block_us * nk < 8.f) return fp;  // unsplit is the better plan
+  const auto cost = [&](int L, int* n_items) {  // L == nk: no split
+    int full = 0, rest = 0, parts = 0;           // items of L blocks, shorter ones, partials (per head)
+    for (int qb = 0; qb < nqb; ++qb) {
+      const int n = blocks_of(qb), f = n / L, r = n % L != 0;
+      full += f;
+      rest += r;
+      if (f + r > 1) parts += f + r;
+    }
+    double dealt = 0.;  // the shorter items' lengths taken as evenly spread
+    for (double i = 0.; i < full + rest; i += cus / nbh)
+      dealt += L * (i < full ? 1. : 1. - (std::floor(i) - full + 0.5) / rest);
+    const double even = std::max<double>(L, work);
+    *n_items = full + rest;
+    return block_us * 0.5 * (even + std::max(dealt, even)) +
+           (parts ? 8. + (double)nbh * part_mult * parts * BM * (HD + 2) * 4 / 1.6e6 : 0.);
+  };
+  int n_items = 0, best_L = nk;
+  double best = cost(nk, &n_items);
+  for (int e = 8; e < nk; e *= 2)
+    for (const int L : {e, e + e / 2}) {  // 8, 12, 16, 24, ...: multiples of BMb
+      if (L >= nk) continue;
+      const double c = cost(L, &n_items);
+      if (c < best && n_items <= kMaxItems) best = c, best_L = L;
+    }
+  if (best_L == nk) return fp;
+  const int L = best_L;
   struct It { int len, qb, seg; };
   std::vector<It> its;
   fp.part_base.assign(kMaxQblk, (int16_t)-1);
   int parts = 0;
   for (int qb = 0; qb < nqb; ++qb) {
-    const int nseg = (int)((nkb[qb] + L - 1) / L);
+    const int nseg = (blocks_of(qb) + L - 1) / L;
     if (nseg > 1) {
       fp.part_base[qb] = (int16_t)parts;
       fp.split_qb.push_back((int16_t)qb);
       parts += nseg;
     }
-    for (int sg = 0; sg < nseg; ++sg) its.push_back({(int)std::min<int64_t>(L, nkb[qb] - sg * L), qb, sg});
+    for (int sg = 0; sg < nseg; ++sg) its.push_back({std::min(L, blocks_of(qb) - sg * L), qb, sg});
   }
   std::stable_sort(its.begin(), its.end(), [](const It& a, const It& b) {
     return a.len != b.len ? a.len > b.len : a.qb > b.qb;
   });
   for (const It& it : its) fp.items.push_back((it.qb << 8) | it.seg);
   fp.n_items = (int)fp.items.size();
-  fp.seg_len = (int)L;
+  fp.seg_len = L;
   fp.n_part_per_head = parts;
   fp.n_split = (int)fp.split_qb.size();
   fp.part_bytes = nbh * part_mult * parts * (int64_t)BM * (HD + 2) * 4;
@@ -379,7 +405,7 @@ int run_flash(const saf_mixed_attn_args* a, const Plan& pl, hipStream_t s) {
   p.scale_log2 = a->sm_scale * kLog2e;
   // split the causal tail when the caller's workspace holds the partials;
   // the workspace's first 256 bytes after the scan region hold the queue word
-  FlashPlan fp = plan_flash(pl.B, p.n_slots, pl.T, pl.HD, BM, flash_resident(pl.HD, qt));
+  FlashPlan fp = plan_flash(pl.B, p.n_slots, pl.T, pl.HD, BM, flash_block_us(pl.HD));
   const int64_t queue_off = scan_ws_bytes(pl), part_off = queue_off + kQueueBytes;
   const bool have_ws = a->workspace != nullptr && reinterpret_cast<uintptr_t>(a->workspace) % 16 == 0;
   // the work queue pays off for the one-workgroup-per-CU kernel above hd 64
@@ -388,7 +414,7 @@ int run_flash(const saf_mixed_attn_args* a, const Plan& pl, hipStream_t s) {
   const bool f32 = pl.dtype == SAF_F32;  // the float32 kernel neither splits nor queues
   if (!f32 && pl.HD > 64 && have_ws && a->workspace_bytes >= part_off) {
     p.queue = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(a->workspace) + queue_off);
-    p.max_grid = cu_count() * flash_resident(pl.HD, qt);
+    p.max_grid = cu_count();
   }
   if (!f32 && fp.n_items && have_ws && a->workspace_bytes >= part_off + fp.part_bytes) {
     char* ws = reinterpret_cast<char*>(a->workspace) + part_off;
@@ -440,8 +466,6 @@ void fill_frozen_common(FrozenParams& p, const saf_tensor_t& v, const saf_tensor
 }
 
 int frozen_qtiles(int hd) { return hd <= 64 ? 2 : 1; }
-// Resident rebuild workgroups per CU (decomp_waves_per_eu in the kernel).
-int decomp_resident(int hd) { return hd > 64 ? 2 : 3; }
 
 // Dense P.V work plan: query blocks of the kernel's shape, balanced over the
 // batch groups that share a pattern.  Larger groups read the pattern fewer
@@ -457,7 +481,7 @@ DensePlan plan_dense(int B, int n_slots, int T, int HD, bool wide, bool can_spli
   DensePlan d;
   const int nqb = (T + dense_block_rows(B, HD) - 1) / dense_block_rows(B, HD);
   for (d.group = dense_batch_group(B, HD, wide);; d.group /= 2) {
-    d.fp = can_split ? plan_flash(B / d.group, n_slots, T, HD, dense_block_rows(B, HD), kDenseResident, d.group)
+    d.fp = can_split ? plan_flash(B / d.group, n_slots, T, HD, dense_block_rows(B, HD), dense_block_us(wide), d.group)
                      : FlashPlan();
     if (d.group == 1 || d.fp.n_items || (int64_t)nqb * n_slots * (B / d.group) >= cu_count()) return d;
   }
@@ -542,7 +566,7 @@ int64_t part_region_bytes(const saf_mixed_attn_args* args, const Plan& pl) {
   if (!pl.live.empty()) {
     const int qt = flash_qtiles_for(args, pl.HD);
     const FlashPlan fp = plan_flash(pl.B, (int)pl.live.size(), pl.T, pl.HD, flash_block_rows(pl.HD, qt),
-                                    flash_resident(pl.HD, qt));
+                                    flash_block_us(pl.HD));
     part = kQueueBytes + fp.part_bytes;
   }
   if (!pl.dense.empty())
@@ -550,7 +574,7 @@ int64_t part_region_bytes(const saf_mixed_attn_args* args, const Plan& pl) {
                               .fp.part_bytes);
   if (!pl.decomp.empty())
     part = std::max(part, plan_flash(pl.B, (int)pl.decomp.size(), pl.T, pl.HD, block_rows(frozen_qtiles(pl.HD)),
-                                     decomp_resident(pl.HD)).part_bytes);
+                                     decomp_block_us(pl.HD)).part_bytes);
   return round256(part);
 }
 
@@ -594,7 +618,7 @@ int run_decomp(const saf_mixed_attn_args* a, const Plan& pl, hipStream_t s, bool
     p.pat_head[i] = (int16_t)h;
   }
   const int BM = block_rows(frozen_qtiles(pl.HD));
-  FlashPlan fp = plan_flash(pl.B, p.n_slots, pl.T, pl.HD, BM, decomp_resident(pl.HD));
+  FlashPlan fp = plan_flash(pl.B, p.n_slots, pl.T, pl.HD, BM, decomp_block_us(pl.HD));
   const int64_t part_off = scan_ws_bytes(pl);
   if (pl.dtype != SAF_F32 && fp.n_items && !unsplit && a->workspace != nullptr &&
       a->workspace_bytes >= part_off + fp.part_bytes && reinterpret_cast<uintptr_t>(a->workspace) % 16 == 0) {

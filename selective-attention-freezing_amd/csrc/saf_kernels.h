@@ -339,7 +339,6 @@ constexpr int dense_batch_group(int B, int hd, bool wide) {
 }
 constexpr int dense_qtiles(int, int) { return 1; }
 constexpr int dense_block_rows(int, int) { return kDenseWaves * 32; }
-constexpr int kDenseResident = 1;
 
 // Waves of a live-head workgroup: 8 for hd 96 / 128 (two per SIMD sharing
 // one set of LDS tiles), else 4 (hd 256: one wave per SIMD, whose 512
