@@ -220,6 +220,12 @@ __device__ __forceinline__ void scan_body(const ScanParams& p, int chunk, int se
   // kLookBack predecessors, nearest first; chunk -1 reads as an inclusive
   // prefix of 0.  Columns are independent, so lanes may look back to
   // different depths.
+  //
+  // One chunk: no status words, so the host launches no clear, and the error
+  // word is reset here (B=1, T=256, hd 64, 12 heads: 7.5 -> 6.5 us and one
+  // launch less; walking two chunks in one workgroup instead of clearing,
+  // T=512, 8.4 -> 9.4 us).
+  if (p.n_chunks == 1 && blockIdx.x == 0 && tid == 0) *p.error = 0u;
   if (tid < 64) {
     const int lane = tid;
     constexpr int NC = (HD + 63) / 64;
@@ -284,8 +290,9 @@ __device__ __forceinline__ void scan_body(const ScanParams& p, int chunk, int se
           }
         }
       }
-      __hip_atomic_store(sw + (int64_t)chunk * HD, pack_word(2u, fmaf(carry, r_ch, a_wg)), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+      if (p.n_chunks > 1)
+        __hip_atomic_store(sw + (int64_t)chunk * HD, pack_word(2u, fmaf(carry, r_ch, a_wg)), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
       sh_carry[col] = carry;
     }
   }

@@ -78,7 +78,8 @@ bool supported_bwd_hd(int64_t hd) { return hd == 32 || hd == 64 || hd == 96 || h
 int n_scan_chunks(int T, int hd) { return (T + scan_chunk_rows(hd) - 1) / scan_chunk_rows(hd); }
 
 // Workspace: [reserved u32, error u32, pad to 256] [status u64 x n] with
-// n = n_seq * n_chunks * hd; the whole block is cleared before a scan.
+// n = n_seq * n_chunks * hd; the whole block is cleared before a scan of more
+// than one chunk.
 struct WsLayout {
   int64_t status_off, total;
 };
@@ -691,7 +692,10 @@ int run_scan(const saf_mixed_attn_args* a, const Plan& pl, hipStream_t s) {
     p.kind[i] = (int8_t)a->closed_kind[h];
     p.param[i] = a->closed_param[h];
   }
-  if (int rc = launched(launch_zero_u32(reinterpret_cast<uint32_t*>(ws), w.total / 4, s), "workspace clear")) return rc;
+  // a sequence of one chunk has no look-back and no status words to clear
+  if (p.n_chunks > 1)
+    if (int rc = launched(launch_zero_u32(reinterpret_cast<uint32_t*>(ws), w.total / 4, s), "workspace clear"))
+      return rc;
   return launched(timed([&] { return launch_scan(p, pl.dtype, pl.HD, s); }, s), "closed-form scan");
 }
 
