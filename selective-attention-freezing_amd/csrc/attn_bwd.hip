@@ -480,7 +480,10 @@ void bwd_dkdv_kernel(const BwdParams p) {
 // frozen slot); query blocks of 64 from the diagonal.  The B operand of
 // dV^T += dO^T P is a column of P for 8 consecutive queries, rebuilt as
 // P[i, j] = 2^((alpha_j + rho_{i-j} - z_i) log2 e); cells with i < j or
-// i >= T are zero.
+// i >= T are zero.  Rebuilding a cell costs an exp2 and three more vector
+// operations, three times the matrix time of its products at hd 64, and P is
+// the same for every sequence: NB = 2 of them share a workgroup and its P
+// (figures and the rule at the launch).
 //
 // dO tiles arrive by DMA two blocks ahead in three static LDS slots (an
 // empty descriptor past the last block, so every block issues the same
@@ -488,11 +491,11 @@ void bwd_dkdv_kernel(const BwdParams p) {
 // block ahead, before that DMA, and written into the next block's slot.  The
 // block ends with a counted wait (the DMA two ahead stays in flight) and a
 // bare barrier: one barrier per block instead of two draining ones.
-template <typename T, int HD>
+template <typename T, int HD, int NB>
 __global__ __launch_bounds__(256) void bwd_decomp_dv_kernel(const BwdParams p) {
   constexpr int BN = kBwdWaves * 32, NDT = HD / 32, VB = VRow<HD>::BYTES;
   constexpr int VN = TileOffsets<T, HD>::VN;  // DMA loads per wave per dO tile
-  __shared__ __align__(16) char o0[VB], o1[VB], o2[VB];
+  __shared__ __align__(16) char o0[NB * VB], o1[NB * VB], o2[NB * VB];
   // decomposed heads: z_q log2 e of the block's 64 queries and rho_d log2 e
   // for every distance d = q - key the block meets (64 + 128 - 1 values)
   __shared__ float zs3[3][64], rs3[3][64 + BN];
@@ -500,10 +503,10 @@ __global__ __launch_bounds__(256) void bwd_decomp_dv_kernel(const BwdParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, g = lane >> 5;
   const int T_len = p.T;
-  const int nbf = p.B * p.n_frozen;
+  const int nbf = p.B / NB * p.n_frozen;
   const int r = blockIdx.x % nbf;
   const int kb = (int)(blockIdx.x / nbf);
-  const int b = r / p.n_frozen, fs = r % p.n_frozen;
+  const int b = NB * (r / p.n_frozen), fs = r % p.n_frozen;  // batch elements b .. b + NB - 1
   if (p.f_kind[fs] != 2) return;
   const int h = p.f_head[fs], ph = p.pat_head[fs];
   const T* dobase = reinterpret_cast<const T*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh;
@@ -513,9 +516,11 @@ __global__ __launch_bounds__(256) void bwd_decomp_dv_kernel(const BwdParams p) {
   const bool kv = kk < T_len;
   float alpha_k = 0.f;
   if (kv) alpha_k = load_as_f32(p.alpha, (int64_t)ph * p.a_sh + (int64_t)kk * p.a_ss, p.a_dtype) * kLog2e;
-  f32x16_t dva[NDT];
+  f32x16_t dva[NB][NDT];
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) dva[dt] = zero16();
+  for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) dva[bb][dt] = zero16();
 
   TileOffsets<T, HD> oo;
   oo.init(wave, lane, p.do_st);
@@ -545,11 +550,14 @@ __global__ __launch_bounds__(256) void bwd_decomp_dv_kernel(const BwdParams p) {
   auto dmin_of = [&](int i) { return 64 * i - kb * BN - (BN - 1); };  // smallest q - key of block i
   auto load_do = [&](int i, auto slotc) {
     constexpr int S = decltype(slotc)::value;
-    oo.load(dobase, p.do_st, 64 * i, i < nqb ? T_len : 0, S == 0 ? o0 : (S == 1 ? o1 : o2), wave);
+#pragma unroll
+    for (int bb = 0; bb < NB; ++bb)
+      oo.load(dobase + bb * p.do_sb, p.do_st, 64 * i, i < nqb ? T_len : 0, (S == 0 ? o0 : (S == 1 ? o1 : o2)) + bb * VB,
+              wave);
   };
   auto meet = [&]() {  // the next block's dO tile has landed (the one after stays in flight)
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(VN));
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(NB * VN));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
@@ -594,7 +602,10 @@ __global__ __launch_bounds__(256) void bwd_decomp_dv_kernel(const BwdParams p) {
       const uint4 bop = make_uint4(Elem<T>::pack2(e8[0], e8[1]), Elem<T>::pack2(e8[2], e8[3]),
                                    Elem<T>::pack2(e8[4], e8[5]), Elem<T>::pack2(e8[6], e8[7]));
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) dva[dt] = Elem<T>::mfma(tile_col_op<HD>(ot, ks, dt, cof), bop, dva[dt]);
+      for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+          dva[bb][dt] = Elem<T>::mfma(tile_col_op<HD>(ot + bb * VB, ks, dt, cof), bop, dva[bb][dt]);
     }
     // the next block's slot was last read two blocks ago
     constexpr int RN = (R + 1) % 3;
@@ -625,7 +636,10 @@ __global__ __launch_bounds__(256) void bwd_decomp_dv_kernel(const BwdParams p) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
   }
-  if (kv) store_out_tile<T, HD>(dvbase + (int64_t)kk * p.dv_st, dva, 1.f, g);
+  if (kv)
+#pragma unroll
+    for (int bb = 0; bb < NB; ++bb)
+      store_out_tile<T, HD>(dvbase + bb * p.dv_sb + (int64_t)kk * p.dv_st, dva[bb], 1.f, g);
 }
 
 // dV of the dense frozen heads, dV[j] = sum_{i >= j} P[i, j] dO[i].  The
@@ -932,7 +946,7 @@ __global__ __launch_bounds__(256) void bwd_decomp_param_kernel(const BwdParams p
   template __global__ void bwd_delta_kernel<T, HD>(const BwdParams);                    \
   template __global__ void bwd_dq_kernel<T, HD>(const BwdParams);                       \
   template __global__ void bwd_dkdv_kernel<T, HD>(const BwdParams);                     \
-  template __global__ void bwd_decomp_dv_kernel<T, HD>(const BwdParams);                \
+  template __global__ void bwd_decomp_dv_kernel<T, HD, 1>(const BwdParams);             \
   template __global__ void bwd_dense_dv_kernel<T, HD, 0>(const BwdParams);              \
   template __global__ void bwd_dense_dv_kernel<T, HD, 1>(const BwdParams);              \
   template __global__ void bwd_dense_dv_kernel<T, HD, 2>(const BwdParams);              \
@@ -940,6 +954,10 @@ __global__ __launch_bounds__(256) void bwd_decomp_param_kernel(const BwdParams p
 #define SAF_BWD_INST_T(T) SAF_BWD_INST(T, 32) SAF_BWD_INST(T, 64) SAF_BWD_INST(T, 96) SAF_BWD_INST(T, 128)
 SAF_BWD_INST_T(__bf16)
 SAF_BWD_INST_T(_Float16)
+template __global__ void bwd_decomp_dv_kernel<__bf16, 32, 2>(const BwdParams);
+template __global__ void bwd_decomp_dv_kernel<__bf16, 64, 2>(const BwdParams);
+template __global__ void bwd_decomp_dv_kernel<_Float16, 32, 2>(const BwdParams);
+template __global__ void bwd_decomp_dv_kernel<_Float16, 64, 2>(const BwdParams);
 #undef SAF_BWD_INST_T
 #undef SAF_BWD_INST
 
@@ -965,8 +983,21 @@ static hipError_t bwd_launch_hd(const BwdParams& p, int which, hipStream_t s) {
     case 3: {
       bool dense = false, decomp = false;
       for (int i = 0; i < p.n_frozen; ++i) (p.f_kind[i] == 1 ? dense : decomp) = true;
-      if (decomp)
-        hipLaunchKernelGGL((bwd_decomp_dv_kernel<T, HD>), dim3((unsigned)(nk * p.B * p.n_frozen)), dim3(256), 0, s, p);
+      if (decomp) {
+        // Two sequences per workgroup where that leaves one and a half
+        // workgroups per CU or more: hd 64, T=4096, forward + backward (us, one
+        // / two), B=8 with 11 frozen heads 428 / 378, 3 (768 workgroups before
+        // pairing) 791 / 774; below, B=8 T=2048 3 heads (384) 296 / 302, B=2
+        // T=4096 3 heads (192) 349 / 361.  Above hd 64 the pair's tiles leave
+        // room for one workgroup per CU (B=8, T=2048, 8 heads hd 128 520 / 529).
+        const int n1 = nk * p.B * p.n_frozen;
+        if (HD <= 64 && p.B % 2 == 0 && n1 >= 3 * p.n_cu) {
+          if constexpr (HD <= 64)
+            hipLaunchKernelGGL((bwd_decomp_dv_kernel<T, HD, 2>), dim3((unsigned)(n1 / 2)), dim3(256), 0, s, p);
+        } else {
+          hipLaunchKernelGGL((bwd_decomp_dv_kernel<T, HD, 1>), dim3((unsigned)n1), dim3(256), 0, s, p);
+        }
+      }
       if (dense) {
         const dim3 grid((unsigned)(8 * p.B * ((nk * p.n_frozen + 7) / 8)));
         // 16-byte rows (the DMA and the vector loads; 32-bit offsets of 64 rows)

@@ -1016,6 +1016,7 @@ int saf_frozen_pv_bwd(const saf_tensor_t* patt, const saf_tensor_t* dy, const in
     return fail(SAF_EUNSUPPORTED, "unsupported patt dtype %s", dtype_name(patt->dtype));
   if (fz_idx == nullptr) return fail(SAF_EINVAL, "fz_idx (host) is required");
   BwdParams p{};
+  p.n_cu = cu_count();
   p.dout = dy->data;
   p.dv = dv->data;
   p.do_sb = dy->stride[0]; p.do_sh = dy->stride[1]; p.do_st = dy->stride[2];
@@ -1298,6 +1299,7 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
   if (pl.T == 0 || pl.B == 0) return SAF_OK;
 
   BwdParams p{};
+  p.n_cu = cu_count();
   p.v = a->v.data;
   p.out = a->out.data;
   p.dout = dout->data;
@@ -1451,6 +1453,7 @@ int saf_decomp_param_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout,
     return fail(SAF_EWORKSPACE, "pattern gradients need a 16-byte aligned %lld-byte workspace (got %lld)",
                 (long long)need, (long long)a->workspace_bytes);
   BwdParams p{};
+  p.n_cu = cu_count();
   p.v = a->v.data;
   p.out = a->out.data;
   p.dout = dout->data;

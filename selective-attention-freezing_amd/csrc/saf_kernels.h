@@ -262,6 +262,7 @@ hipError_t launch_decomp_logz_bwd(const LogzBwdParams& p, hipStream_t s);
 // Live slots index the compact q/k (q_head) and the natural head (out_head);
 // frozen slots list the dense / decomposed heads.
 struct BwdParams {
+  int n_cu;  // compute units of the device
   const void* q;
   const void* k;
   const void* v;
