@@ -365,10 +365,11 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
                chunk after the first gives up: NaN rows, and with validate
                a RuntimeError)
       decomp_unsplit  None (auto) = True when live heads share the call and
-               the decomposed ones are long enough to pay for a fork; True: decomposed heads run one workgroup per query block,
-               beside the live-head kernel on a side stream when there is
-               one; False: key-segment split with partials and a combine,
-               after the live-head kernel on the current stream
+               the decomposed ones are long enough to pay for a fork; True:
+               decomposed heads run one workgroup per query block, beside the
+               live-head kernel on a side stream when there is one; False:
+               key-segment split with partials and a combine, after the
+               live-head kernel on the current stream
     Returns (B, H, T, HD) in natural head order, strided like v (like the
     reference's empty_like(v)).
     """
@@ -400,6 +401,8 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
     if closed_form is not None:
         ck, ck_c = _table(closed_form[0], np.int32)
         _, cp_c = _table(closed_form[1], np.float32)
+        if len(ck_c) != H or len(cp_c) != H:
+            raise ValueError("closed_form must hold one kind and one parameter per output head")
         if n_state2:
             n_scan = n_state2 - [c for s, c in zip(states, ck.tolist()) if s == 2].count(0)
 
