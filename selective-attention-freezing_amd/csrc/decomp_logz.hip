@@ -234,8 +234,10 @@ hipError_t launch_decomp_logz(const LogzParams& p, hipStream_t s) {
 // the output's total times 2^(own + O + W).  A product lost below 2^-126 is then
 // worth at most 2^(own + O + W - 126) |gz_i|: chunks where own + O + W exceeds
 // kLzScale for some output (logits whose maxima lie far above every pair's
-// value) or is not finite run the direct form, one exp2 per pair.  Rows whose z
-// is -inf (every logit -inf) contribute nothing.
+// value) or is not finite run the direct form, one exp2 per pair, and so do
+// chunks with a gz that is not finite: the zero that stands for a pair outside
+// the triangle would turn it into NaN for outputs o > i that the row does not
+// reach.  Rows whose z is -inf (every logit -inf) contribute nothing.
 // H=12, S=8192: 264 us (one exp2 per pair) -> 49 us.
 constexpr float kLzScale = 40.f;
 
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_bwd_kernel(const LogzB
       const bool none = ev[k] == ninf;  // z of a row without a share
       gv[k] = none ? 0.f : gv[k];
       ev[k] = none ? ninf : -ev[k] * kLog2e;
-      W = fmaxf(W, ev[k]);
+      W = fmaxf(W, __builtin_isfinite(gv[k]) ? ev[k] : -ninf);
     }
 #pragma unroll
     for (int k = 0; k < kLzNW; ++k) O = fmaxf(O, ov[k] *= kLog2e);
@@ -326,8 +328,10 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_bwd_kernel(const LogzB
     } else {
       for (int t = t0; t < min(t1, n); ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc[r] = fmaf(as[t], fast_exp2(fixed[r] + ws[t - 4 * lane - r + kLzRows - 1] + es[t]), acc[r]);
+        for (int r = 0; r < 4; ++r) {
+          const float x = fixed[r] + ws[t - 4 * lane - r + kLzRows - 1] + es[t];
+          if (x != ninf) acc[r] = fmaf(as[t], fast_exp2(x), acc[r]);
+        }
 #pragma unroll
       for (int r = 0; r < 4; ++r) tot[r] += acc[r];
     }

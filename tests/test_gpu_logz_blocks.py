@@ -64,3 +64,24 @@ def test_logz_blocks(kind, S):
         # exponent arguments of magnitude x round by 2^-23 |x|
         mag = float(torch.nan_to_num(a, neginf=0.0).abs().max() + torch.nan_to_num(r, neginf=0.0).abs().max())
         assert err <= 1e-5 + 2.0 ** -21 * mag, f"{name}: {err:.2e}"
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_gradient_of_one_row_not_finite(bad):
+    """A gz_i that is not finite reaches the outputs o <= i and no other."""
+    import kernel
+    H, S, i = 1, 2305, 2060
+    a, r = _inputs("learned", H, S)
+    gz = torch.randn(H, S, generator=torch.Generator().manual_seed(1))
+    grads = []
+    for x in (0.0, bad):
+        gz[0, i] = x
+        ad, rd = a.to(DEV).requires_grad_(), r.to(DEV).requires_grad_()
+        z = kernel.decomp_log_normalizers(ad, rd)
+        grads.append(torch.autograd.grad(z, (ad, rd), gz.to(DEV)))
+    for clean, got in zip(*grads):
+        assert not torch.isfinite(got[0, : i + 1]).any()
+        want, rest = clean[0, i + 1:], got[0, i + 1:]
+        assert torch.isfinite(rest).all()
+        # the two forms round their fp32 sums of a few hundred terms differently
+        assert float((rest - want).norm()) <= 1e-5 * float(want.norm())
