@@ -22,8 +22,9 @@
  *   - Every tensor is described by saf_tensor_t: a device pointer, a dtype
  *     code, and 4-D sizes/strides counted in elements.  The innermost stride
  *     must be 1; q/k/v rows must start on 16-byte boundaries and out rows on
- *     8-byte boundaries (status SAF_EALIGN otherwise: make the tensor
- *     contiguous and call again).
+ *     8-byte boundaries, and bf16 / fp16 rows that the kernels read by whole
+ *     pitches (k, v, dout, and q of the backward) must be at least HD apart
+ *     (status SAF_EALIGN otherwise: make the tensor contiguous and call again).
  *   - The caller allocates every buffer, including out, the optional lse and
  *     the workspace.  The library allocates no device memory; its one device
  *     array (the scratch of saf_mixed_attn_fwd_noalloc) exists from the

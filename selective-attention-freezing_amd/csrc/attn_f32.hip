@@ -78,13 +78,22 @@ __device__ __forceinline__ float4 buf_load4(__amdgpu_buffer_rsrc_t r, int off) {
   return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
 }
 
+// Descriptor over the HD-float rows r0 .. T - 1 of a tensor with row pitch st:
+// it ends with the last row's last element, so rows closer than HD (a tensor
+// expanded over T: st = 0; overlapping windows) are read whole too.  Rows past
+// T then read whatever lies before that end; their cells are masked or dropped.
+template <int HD>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const float* base, int64_t st, int r0, int T_len) {
+  return span_rsrc(base + (int64_t)r0 * st, r0 < T_len ? ((int64_t)(T_len - 1 - r0) * st + HD) * 4 : (int64_t)0);
+}
+
 // Rows r0 .. r0 + 31 of a (T, st) fp32 tensor as a row operand.
 template <int HD, bool WHOLE = F32Shape<HD>::kWhole> struct RowFrag {
   static constexpr int NT = F32Shape<HD>::NT;
   float4 r[WHOLE ? NT : 1];
   __amdgpu_buffer_rsrc_t rsrc;
   __device__ __forceinline__ void load(const float* base, int64_t st, int r0, int T_len, int off) {
-    rsrc = rows_rsrc(base, st, r0, T_len);
+    rsrc = tile_rsrc<HD>(base, st, r0, T_len);
     if constexpr (WHOLE) {
       SAF_PIN();
 #pragma unroll
@@ -141,7 +150,7 @@ template <int HD, bool WHOLE = F32Shape<HD>::kWhole> struct ColFrag {
     }
   }
   __device__ __forceinline__ void load(const float* base, int64_t st, int r0, int T_len, int off) {
-    rsrc = rows_rsrc(base, st, r0, T_len);
+    rsrc = tile_rsrc<HD>(base, st, r0, T_len);
     if constexpr (WHOLE) {
       SAF_PIN();
       // the sixteen row offsets are formed here each time: held across the
@@ -182,7 +191,7 @@ __device__ __forceinline__ int acc_row(int i, int g) { return 8 * (i >> 2) + 4 *
 template <int HD>
 __device__ __forceinline__ void stage_tile(float4* dst, const float* base, int64_t st, int r0, int T_len, int wave,
                                            int lane) {
-  const __amdgpu_buffer_rsrc_t r = rows_rsrc(base, st, r0, T_len);
+  const __amdgpu_buffer_rsrc_t r = tile_rsrc<HD>(base, st, r0, T_len);
   for (int t = wave; t < F32Shape<HD>::NT; t += kW) dst[t * 64 + lane] = buf_load4(r, row_off(st, lane) + 32 * t);
 }
 
@@ -499,9 +508,9 @@ void f32_bwd_dq_kernel(const BwdParams p) {
   ColFrag<HD> kc;
   {
     const __amdgpu_buffer_rsrc_t gr =
-        rows_rsrc(reinterpret_cast<const float*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh, p.do_st, q0, T_len);
+        tile_rsrc<HD>(reinterpret_cast<const float*>(p.dout) + b * p.do_sb + (int64_t)h * p.do_sh, p.do_st, q0, T_len);
     const __amdgpu_buffer_rsrc_t orr =
-        rows_rsrc(reinterpret_cast<const float*>(p.out) + b * p.o_sb + (int64_t)h * p.o_sh, p.o_st, q0, T_len);
+        tile_rsrc<HD>(reinterpret_cast<const float*>(p.out) + b * p.o_sb + (int64_t)h * p.o_sh, p.o_st, q0, T_len);
     float acc = 0.f;
     for (int t = wave; t < NT; t += kW) {
       const float4 d = buf_load4(gr, row_off(p.do_st, lane) + 32 * t);

@@ -70,6 +70,30 @@ int check_act(const saf_tensor_t& t, const char* name, int align) {
   return SAF_OK;
 }
 
+// A 16-bit activation that a kernel reads through buffer descriptors of whole
+// pitches (rows_rsrc, RowCursor): rows closer than the head dim would lose their
+// ends.  (The float32 kernels' descriptors end with the last row's last element.)
+int check_pitch(const saf_tensor_t& t, const char* name) {
+  if (t.dtype != SAF_F32 && t.size[2] > 1 && t.stride[2] < t.size[3])
+    return fail(SAF_EALIGN, "%s rows are closer than the head dimension (stride %lld)", name, (long long)t.stride[2]);
+  return SAF_OK;
+}
+
+// One row has no pitch: its stride may be anything, and the kernels' descriptors
+// are formed from it.
+saf_tensor_t one_row(saf_tensor_t t) {
+  if (t.ndim == 4 && t.size[2] == 1) t.stride[2] = t.size[3];
+  return t;
+}
+saf_mixed_attn_args one_row(const saf_mixed_attn_args& a) {
+  saf_mixed_attn_args r = a;
+  r.q = one_row(a.q);
+  r.k = one_row(a.k);
+  r.v = one_row(a.v);
+  r.out = one_row(a.out);
+  return r;
+}
+
 // Head dims of the forward kernels; the backward kernels and the fused
 // RoPE / q-k norm prologue stop at 128.
 bool supported_hd(int64_t hd) { return hd == 32 || hd == 64 || hd == 96 || hd == 128 || hd == 256; }
@@ -182,6 +206,8 @@ int plan_and_validate(const saf_mixed_attn_args* a, unsigned which, Plan& pl, bo
     }
     if (int rc = check_act(q, "q", 16)) return rc;
     if (int rc = check_act(k, "k", 16)) return rc;
+    if (int rc = check_pitch(k, "k")) return rc;
+    if (int rc = check_pitch(v, "v")) return rc;
     const int U = (int)q.size[1];
     for (int h : pl.live) {
       const int slot = a->hidx ? a->hidx[h] : h;
@@ -196,6 +222,7 @@ int plan_and_validate(const saf_mixed_attn_args* a, unsigned which, Plan& pl, bo
       return fail(SAF_EINVAL, "patt must have shape (P, S, S) with S >= T");
     if (p.dtype != SAF_F32 && p.dtype != SAF_BF16 && p.dtype != SAF_F16)
       return fail(SAF_EUNSUPPORTED, "unsupported patt dtype %s", dtype_name(p.dtype));
+    if (int rc = check_pitch(v, "v")) return rc;
     for (int h : pl.dense) {
       const int row = a->pidx ? a->pidx[h] : h;
       if (row < 0 || row >= p.size[0])
@@ -218,6 +245,7 @@ int plan_and_validate(const saf_mixed_attn_args* a, unsigned which, Plan& pl, bo
     }
   }
   if ((which & kDoScan) && !pl.scan.empty()) {
+    if (int rc = check_pitch(v, "v")) return rc;
     // the scan addresses one chunk of rows with 32-bit buffer offsets
     const int64_t lim = (int64_t)1 << 31, es = 2, ch = scan_chunk_rows(pl.HD);
     if (v.stride[2] * es * ch >= lim || o.stride[2] * es * ch >= lim)
@@ -806,6 +834,11 @@ constexpr double kSideMinMainUs = 240;
 // everything runs in order on `stream`.
 int run(const saf_mixed_attn_args* a, unsigned which, void* stream, bool may_fork = false) {
   Plan pl;
+  saf_mixed_attn_args args;
+  if (a != nullptr) {
+    args = one_row(*a);
+    a = &args;
+  }
   if (int rc = plan_and_validate(a, which, pl)) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool has_dec = (which & kDoDecomp) && !pl.decomp.empty();
@@ -972,6 +1005,7 @@ int saf_frozen_pv_fwd(const saf_tensor_t* patt, const saf_tensor_t* v, const int
   if (out->size[0] != B || out->size[1] != nf || out->size[2] != T || out->size[3] != HD || out->dtype != v->dtype)
     return fail(SAF_EINVAL, "out must be (B, nf, T, hd) in v's dtype");
   if (int rc = check_act(*v, "v", 16)) return rc;
+  if (int rc = check_pitch(*v, "v")) return rc;
   if (int rc = check_act(*out, "out", 8)) return rc;
   if (nf == 0 || T == 0 || B == 0) return SAF_OK;
   if (!present(*patt) || patt->ndim != 3 || patt->size[1] < T || patt->size[2] < T)
@@ -987,7 +1021,7 @@ int saf_frozen_pv_fwd(const saf_tensor_t* patt, const saf_tensor_t* v, const int
     vh.push_back(f);
     ph.push_back(fz_idx[f]);
   }
-  return run_dense(*patt, *v, *out, B, T, HD, v->dtype, oh, vh, ph, nullptr, 0,
+  return run_dense(*patt, one_row(*v), one_row(*out), B, T, HD, v->dtype, oh, vh, ph, nullptr, 0,
                    reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -1008,6 +1042,7 @@ int saf_frozen_pv_bwd(const saf_tensor_t* patt, const saf_tensor_t* dy, const in
   if (dy->size[0] != B || dy->size[1] != nf || dy->size[2] != T || dy->size[3] != HD || dy->dtype != dv->dtype)
     return fail(SAF_EINVAL, "dy must be (B, nf, T, hd) in dv's dtype");
   if (int rc = check_act(*dy, "dy", 16)) return rc;
+  if (int rc = check_pitch(*dy, "dy")) return rc;
   if (int rc = check_act(*dv, "dv", 8)) return rc;
   if (nf == 0 || T == 0 || B == 0) return SAF_OK;
   if (!present(*patt) || patt->ndim != 3 || patt->size[1] < T || patt->size[2] < T)
@@ -1019,7 +1054,7 @@ int saf_frozen_pv_bwd(const saf_tensor_t* patt, const saf_tensor_t* dy, const in
   p.n_cu = cu_count();
   p.dout = dy->data;
   p.dv = dv->data;
-  p.do_sb = dy->stride[0]; p.do_sh = dy->stride[1]; p.do_st = dy->stride[2];
+  p.do_sb = dy->stride[0]; p.do_sh = dy->stride[1]; p.do_st = one_row(*dy).stride[2];
   p.dv_sb = dv->stride[0]; p.dv_sh = dv->stride[1]; p.dv_st = dv->stride[2];
   p.B = B;
   p.T = T;
@@ -1267,6 +1302,11 @@ int64_t saf_mixed_attn_bwd_workspace_bytes(const saf_mixed_attn_args* args) {
 int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, const saf_tensor_t* dq,
                        const saf_tensor_t* dk, const saf_tensor_t* dv, void* stream) {
   Plan pl;
+  saf_mixed_attn_args args;
+  if (a != nullptr) {
+    args = one_row(*a);
+    a = &args;
+  }
   if (int rc = plan_and_validate(a, kDoFlash | kDoDense | kDoDecomp, pl, false)) return rc;
   if (a->kvidx != nullptr)
     return fail(SAF_EUNSUPPORTED, "backward with kvidx (GQA) is not implemented (forward / prefill only)");
@@ -1281,7 +1321,10 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
   if (!present(*dout) || !same4(*dout, a->out)) return fail(SAF_EINVAL, "dout must match out's shape and dtype");
   if (!present(*dv) || !same4(*dv, a->v)) return fail(SAF_EINVAL, "dv must match v's shape and dtype");
   if (int rc = check_act(*dout, "dout", 16)) return rc;
+  if (int rc = check_pitch(*dout, "dout")) return rc;
   if (int rc = check_act(*dv, "dv", 8)) return rc;
+  if (!pl.live.empty())
+    if (int rc = check_pitch(a->q, "q")) return rc;
   // closed-form heads run as decomposed heads here: their alpha/rho/z are needed
   std::vector<int> fz_dec = pl.decomp;
   fz_dec.insert(fz_dec.end(), pl.scan.begin(), pl.scan.end());
@@ -1306,7 +1349,7 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
   p.dv = dv->data;
   p.v_sb = a->v.stride[0]; p.v_sh = a->v.stride[1]; p.v_st = a->v.stride[2];
   p.o_sb = a->out.stride[0]; p.o_sh = a->out.stride[1]; p.o_st = a->out.stride[2];
-  p.do_sb = dout->stride[0]; p.do_sh = dout->stride[1]; p.do_st = dout->stride[2];
+  p.do_sb = dout->stride[0]; p.do_sh = dout->stride[1]; p.do_st = one_row(*dout).stride[2];
   p.dv_sb = dv->stride[0]; p.dv_sh = dv->stride[1]; p.dv_st = dv->stride[2];
   p.B = pl.B;
   p.T = pl.T;
@@ -1446,6 +1489,7 @@ int saf_decomp_param_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout,
   for (int i = 0; i < 4; ++i)
     if (dout->size[i] != a->out.size[i]) return fail(SAF_EINVAL, "dout must match out's shape and dtype");
   if (int rc = check_act(*dout, "dout", 16)) return rc;
+  if (int rc = check_pitch(*dout, "dout")) return rc;
   if (int rc = check_act(a->out, "out", 16)) return rc;
   if ((int)heads.size() > kMaxHeads) return fail(SAF_EUNSUPPORTED, "too many decomposed heads");
   const int64_t need = saf_decomp_param_bwd_workspace_bytes(a);
@@ -1459,7 +1503,7 @@ int saf_decomp_param_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout,
   p.dout = dout->data;
   p.v_sb = a->v.stride[0]; p.v_sh = a->v.stride[1]; p.v_st = a->v.stride[2];
   p.o_sb = a->out.stride[0]; p.o_sh = a->out.stride[1]; p.o_st = a->out.stride[2];
-  p.do_sb = dout->stride[0]; p.do_sh = dout->stride[1]; p.do_st = dout->stride[2];
+  p.do_sb = dout->stride[0]; p.do_sh = dout->stride[1]; p.do_st = one_row(*dout).stride[2];
   p.B = pl.B;
   p.T = pl.T;
   p.n_live = (int)heads.size();   // the decomposed heads take the live slots here

@@ -12,7 +12,7 @@ V at or past T get zero gradient.
 import torch
 
 from . import _ext
-from .fused_attn import _aligned_view, _host_table, _row_aligned
+from .fused_attn import _aligned_view, _host_table
 
 HAVE_TRITON = False   # this build has no Triton; kept for import compatibility
 
@@ -58,9 +58,7 @@ def frozen_pv(patt, v, fz_idx, T):
 
     def bwd(dy):
         """dv (v's shape, contiguous) = P^T dy over the first T rows."""
-        dy_d = dy.to(v.dtype)
-        if not _row_aligned(dy_d, 16):
-            dy_d = dy_d.contiguous()
+        dy_d = _aligned_view(dy.to(v.dtype), 16)
         make = torch.empty if Tv == T else torch.zeros
         dv = make((B, nf, Tv, hd), device=v.device, dtype=v.dtype)
         stream = _ext.current_stream_ptr(v.device)

@@ -262,8 +262,19 @@ def _row_aligned(t, align):
     return True
 
 
+def _rows_apart(t):
+    """False where the rows of a (B, N, T, hd) tensor are closer than hd
+    (expanded over T, overlapping windows): the 16-bit kernels read rows at
+    least hd apart."""
+    shape = t.shape
+    return shape[2] <= 1 or t.stride(2) >= shape[3]
+
+
 def _aligned_view(t, align=16):
-    return t if _row_aligned(t, align) else t.contiguous()
+    """t, or a contiguous copy where its rows are not aligned or too close."""
+    if t is None or (_row_aligned(t, align) and _rows_apart(t)):
+        return t
+    return t.contiguous()
 
 
 class KernelTimer:
@@ -507,11 +518,12 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
                 "(as in qwen/kernel/fused_attn.py:605-609 of the reference)")
         if n_state2 and alpha is None:
             raise ValueError("the backward of decomposed heads needs alpha/rho/z")
-        # the kernels take any layout of aligned, distinct rows (the model's
-        # gradient arrives as a head-major view of a (B, T, C) tensor);
-        # expanded gradients and huge pitches are copied
-        do = dout
-        if not (_row_aligned(do, 16) and HD <= do.stride(2) < (1 << 21)):
+        # the kernels take any layout of aligned rows (the model's gradient
+        # arrives as a head-major view of a (B, T, C) tensor; a gradient
+        # expanded over batch or heads is only read); rows closer than HD and
+        # huge pitches are copied
+        do = _aligned_view(dout, 16)
+        if do.stride(2) >= 1 << 21:
             do = do.contiguous()
         dq = dk = None
         if n_live:

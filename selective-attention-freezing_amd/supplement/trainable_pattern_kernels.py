@@ -19,7 +19,7 @@ import numpy as np
 import torch
 
 import kernel._ext as _ext
-from kernel.fused_attn import _host_table, decomposed_logz
+from kernel.fused_attn import _host_table, _rows_apart, decomposed_logz
 
 
 @torch.no_grad()
@@ -53,7 +53,7 @@ def pattern_gradients(out, value, alpha, rho, z, states, grad):
     L = _ext.lib()
     a, r, zz = (t.detach() for t in (alpha, rho, z))
     a, r, zz = (t if t.stride(-1) == 1 else t.contiguous() for t in (a, r, zz))
-    go = grad if grad.stride(-1) == 1 else grad.contiguous()
+    go = grad if grad.stride(-1) == 1 and _rows_apart(grad) else grad.contiguous()
     args = _ext.SafMixedAttnArgs()
     args.v = _ext.tensor_desc(value)
     args.out = _ext.tensor_desc(out)

@@ -124,3 +124,23 @@ def test_host_table_cached_per_tensor_and_version():
     assert F._host_table(t.clone()) is not b          # another tensor: its own copy
     assert F._host_table(None) is None
     assert F._host_table([1, 2]).tolist() == [1, 2]
+
+
+def test_close_rows_refused():
+    """16-bit rows closer than the head dim, which the kernels' descriptors cut
+    short, are refused where they would be read so; one row has no pitch."""
+    L = _ext.lib()
+    for name in ("k", "v"):
+        a = _args()
+        getattr(a, name).stride[2] = 0
+        assert L.saf_mixed_attn_fwd(ctypes.byref(a), None) == _ext.SAF_EALIGN
+        assert "closer than" in L.saf_last_error().decode()
+    d, p = (_ext.SafTensor.from_buffer_copy(_args().v) for _ in range(2))
+    d.stride[2] = 32
+    p.ndim, p.dtype = 3, _ext.SAF_F32
+    for i, n in enumerate((4, 64, 64)):
+        p.size[i], p.stride[i] = n, (4096, 64, 1)[i]
+    fz = (ctypes.c_int32 * 4)(0, 1, 2, 3)
+    out = _args().v
+    assert L.saf_frozen_pv_bwd(p, d, fz, 4, 64, out, None) == _ext.SAF_EALIGN
+    assert L.saf_frozen_pv_fwd(p, d, fz, 4, 64, out, None) == _ext.SAF_EALIGN
