@@ -535,8 +535,11 @@ int run_dense(const saf_tensor_t& patt, const saf_tensor_t& v, const saf_tensor_
   p.patt_elems = 1 + (patt.size[0] - 1) * patt.stride[0] + (patt.size[1] - 1) * patt.stride[1] +
                  (patt.size[2] - 1) * patt.stride[2];
   const int es = elem_size(patt.dtype);
+  // the lanes' offsets span a block of 256 rows in 32 bits, from a descriptor
+  // of at most 2 GiB
   p.patt_vec = patt.stride[2] == 1 && reinterpret_cast<uintptr_t>(patt.data) % 16 == 0 &&
-               (patt.stride[1] * es) % 16 == 0 && (patt.stride[0] * es) % 16 == 0;
+               (patt.stride[1] * es) % 16 == 0 && (patt.stride[0] * es) % 16 == 0 && patt.stride[1] >= 0 &&
+               patt.stride[1] * es * dense_block_rows(B, HD) < ((int64_t)1 << 31);
   // the descriptor ends with the 16-byte piece that holds the last element: an
   // odd count of 16-bit elements would end inside a 32-bit word, which then
   // reads as zero

@@ -61,3 +61,25 @@ def test_dense_pattern_forms(dtype, patt, layout, T, S, B, hd):
         assert torch.isfinite(got).all(), name
         rel = float((got - want).norm() / want.norm())
         assert rel <= tol, f"{name}: rel {rel:.2e} > {tol:.2e}"
+
+
+@pytest.mark.parametrize("patt", ["float32", "same"])
+def test_dense_pattern_wide_pitch(patt):
+    """Pattern rows 64 MB apart (one head's columns of a wide buffer): rows past
+    the 2 GB that a buffer descriptor spans are read through pointers."""
+    import kernel
+    T = S = 48
+    pitch = (64 << 20) // (4 if patt == "float32" else 2)
+    pd = torch.float32 if patt == "float32" else torch.bfloat16
+    P, ref = _pattern(1, S, T, "plain", pd, seed=3)
+    wide = torch.empty(S * pitch, device=DEV, dtype=pd).as_strided((1, S, S), (S * pitch, pitch, 1))
+    wide.copy_(P)
+    g = torch.Generator().manual_seed(T)
+    v, dy = (torch.randn(2, 2, T, 64, generator=g).bfloat16() for _ in range(2))
+    vd = v.to(DEV).requires_grad_()
+    y = kernel.frozen_pv(wide, vd, torch.zeros(2, dtype=torch.int32, device=DEV), T)
+    y.backward(dy.to(DEV))
+    W = ref.bfloat16().double()
+    for got, want, name in ((y, W @ v.double(), "y"), (vd.grad, W.transpose(1, 2) @ dy.double(), "dv")):
+        rel = float((got.detach().double().cpu() - want).norm() / want.norm())
+        assert rel <= 1.5 * 2.0 ** -8, f"{name}: rel {rel:.2e}"
