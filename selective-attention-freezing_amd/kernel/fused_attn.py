@@ -236,7 +236,9 @@ def _table(t, np_dtype=np.int32):
         return arr, make(arr)
     cached = getattr(t, "_saf_host", None)
     if cached is not None and cached[0] == t._version and cached[1] == t.data_ptr() and cached[2].dtype == np_dtype:
-        return cached[2], cached[3]
+        # the copy of a CPU table may be its own memory, which numpy can edit
+        # without moving the version: its ctypes twin is formed at each call
+        return cached[2], make(cached[2]) if t.device.type == "cpu" else cached[3]
     arr = t.detach().cpu().numpy().astype(np_dtype, copy=False).reshape(-1)
     arr = np.ascontiguousarray(arr)
     buf = make(arr)

@@ -144,3 +144,16 @@ def test_close_rows_refused():
     out = _args().v
     assert L.saf_frozen_pv_bwd(p, d, fz, 4, 64, out, None) == _ext.SAF_EALIGN
     assert L.saf_frozen_pv_fwd(p, d, fz, 4, 64, out, None) == _ext.SAF_EALIGN
+
+
+def test_cpu_table_sharing_memory():
+    """A routing table on the CPU that shares memory with numpy: an edit through
+    numpy moves no version, and both the host copy and its ctypes twin follow."""
+    import numpy as np
+    from kernel import fused_attn as F
+    arr = np.array([0, 2, 1, 0], dtype=np.int32)
+    t = torch.from_numpy(arr)
+    for states in ([0, 2, 1, 0], [2, 0, 0, 1]):
+        arr[:] = states
+        host, twin = F._table(t)
+        assert host.tolist() == states and list(twin) == states
