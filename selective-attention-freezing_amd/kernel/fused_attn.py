@@ -414,8 +414,8 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
     if closed_form is not None:
         ck, ck_c = _table(closed_form[0], np.int32)
         _, cp_c = _table(closed_form[1], np.float32)
-        if len(ck_c) != H or len(cp_c) != H:
-            raise ValueError("closed_form must hold one kind and one parameter per output head")
+        if len(ck_c) != H or len(cp_c) < H:  # the library reads H of each
+            raise ValueError("closed_form must hold one kind and at least one parameter per output head")
         if n_state2:
             n_scan = n_state2 - [c for s, c in zip(states, ck.tolist()) if s == 2].count(0)
 
