@@ -146,6 +146,12 @@ typedef struct saf_mixed_attn_args {
  * a single kernel. */
 int saf_mixed_attn_fwd(const saf_mixed_attn_args* args, void* stream);
 
+/* The kernels that saf_mixed_attn_fwd of these arguments runs on its second
+ * stream: 1 the decomposed heads, 2 the closed-form scan (3 both, 0 neither), or
+ * -1 for invalid arguments.  For callers that put the subsets below on streams
+ * of their own; enqueues nothing. */
+int saf_mixed_attn_side_kernels(const saf_mixed_attn_args* args);
+
 /* saf_mixed_attn_fwd without a caller workspace, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid allocation).  No counterpart in the reference (its

@@ -829,6 +829,20 @@ constexpr double kSideMinFlops = 8e9;
 // 62 against 24.
 constexpr double kSideMinMainUs = 240;
 
+// The kernels that a forking call runs on the side stream by these rules: 1 the
+// decomposed heads, 2 the closed-form scan.
+int side_kernels(const saf_mixed_attn_args* a, const Plan& pl, unsigned which) {
+  const bool has_dec = (which & kDoDecomp) && !pl.decomp.empty();
+  const bool has_live = (which & kDoFlash) && !pl.live.empty();
+  const bool dec = has_dec && has_live && a->decomp_unsplit >= 0 &&
+                   (a->decomp_unsplit > 0 || pv_flops(pl, pl.decomp.size()) >= kSideMinFlops);
+  const double main_us = 2 * pv_flops(pl, has_live ? pl.live.size() : 0) * 1.2e-9 +
+                         pv_flops(pl, (has_dec && !dec ? pl.decomp.size() : 0) +
+                                          ((which & kDoDense) ? pl.dense.size() : 0)) * 2e-9;
+  const bool scan = (which & kDoScan) && !pl.scan.empty() && (dec || main_us >= kSideMinMainUs);
+  return (dec ? 1 : 0) | (scan ? 2 : 0);
+}
+
 // The head kinds of `which`.  With may_fork (saf_mixed_attn_fwd) and work
 // enough (above), the HBM-bound closed-form scan and, when live heads share the call, the
 // decomposed heads (one workgroup per query block, unless decomp_unsplit < 0)
@@ -844,14 +858,8 @@ int run(const saf_mixed_attn_args* a, unsigned which, void* stream, bool may_for
   }
   if (int rc = plan_and_validate(a, which, pl)) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const bool has_dec = (which & kDoDecomp) && !pl.decomp.empty();
-  const bool has_live = (which & kDoFlash) && !pl.live.empty();
-  const bool dec_side = may_fork && has_dec && has_live && a->decomp_unsplit >= 0 &&
-                        (a->decomp_unsplit > 0 || pv_flops(pl, pl.decomp.size()) >= kSideMinFlops);
-  const double main_us = 2 * pv_flops(pl, has_live ? pl.live.size() : 0) * 1.2e-9 +
-                         pv_flops(pl, (has_dec && !dec_side ? pl.decomp.size() : 0) +
-                                          ((which & kDoDense) ? pl.dense.size() : 0)) * 2e-9;
-  const bool scan_side = may_fork && (which & kDoScan) && !pl.scan.empty() && (dec_side || main_us >= kSideMinMainUs);
+  const int side = may_fork ? side_kernels(a, pl, which) : 0;
+  const bool dec_side = side & 1, scan_side = side & 2;
   const bool dec_unsplit = a->decomp_unsplit > 0;
   if (!dec_side && !scan_side) {
     if (which & kDoFlash)
@@ -987,6 +995,11 @@ int add_norm(const char* what, bool rms, const saf_tensor_t* x, const saf_tensor
 extern "C" {
 
 int saf_mixed_attn_fwd(const saf_mixed_attn_args* args, void* stream) { return run(args, kDoAll, stream, true); }
+int saf_mixed_attn_side_kernels(const saf_mixed_attn_args* args) {
+  Plan pl;
+  if (plan_and_validate(args, kDoAll, pl, false)) return -1;
+  return side_kernels(args, pl, kDoAll);
+}
 int saf_flash_fwd(const saf_mixed_attn_args* args, void* stream) { return run(args, kDoFlash, stream); }
 int saf_frozen_dense_pv_fwd(const saf_mixed_attn_args* args, void* stream) { return run(args, kDoDense, stream); }
 int saf_frozen_decomp_fwd(const saf_mixed_attn_args* args, void* stream) { return run(args, kDoDecomp, stream); }

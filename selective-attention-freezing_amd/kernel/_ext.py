@@ -22,8 +22,8 @@ _DTYPE_CODE = {torch.float32: SAF_F32, torch.float16: SAF_F16,
                torch.bfloat16: SAF_BF16, torch.int32: SAF_I32}
 
 # Exported symbols, in header order (checked by the CPU test suite).
-EXPORTS = ("saf_mixed_attn_fwd", "saf_mixed_attn_fwd_noalloc", "saf_flash_fwd", "saf_frozen_dense_pv_fwd",
-           "saf_frozen_decomp_fwd", "saf_frozen_scan_fwd", "saf_mixed_attn_bwd",
+EXPORTS = ("saf_mixed_attn_fwd", "saf_mixed_attn_side_kernels", "saf_mixed_attn_fwd_noalloc", "saf_flash_fwd",
+           "saf_frozen_dense_pv_fwd", "saf_frozen_decomp_fwd", "saf_frozen_scan_fwd", "saf_mixed_attn_bwd",
            "saf_mixed_attn_bwd_workspace_bytes", "saf_decomp_param_bwd", "saf_decomp_param_bwd_workspace_bytes",
            "saf_frozen_pv_fwd", "saf_frozen_pv_bwd",
            "saf_rope_qk_inplace", "saf_qk_rmsnorm_rope_inplace", "saf_add_layernorm",
@@ -81,6 +81,8 @@ def lib():
             fn = getattr(L, name)
             fn.argtypes = [P(SafMixedAttnArgs), ctypes.c_void_p]
             fn.restype = ctypes.c_int
+        L.saf_mixed_attn_side_kernels.argtypes = [P(SafMixedAttnArgs)]
+        L.saf_mixed_attn_side_kernels.restype = ctypes.c_int
         L.saf_mixed_attn_bwd.argtypes = [P(SafMixedAttnArgs)] + [P(SafTensor)] * 4 + [ctypes.c_void_p]
         L.saf_mixed_attn_bwd.restype = ctypes.c_int
         L.saf_mixed_attn_bwd_workspace_bytes.argtypes = [P(SafMixedAttnArgs)]

@@ -308,9 +308,9 @@ _SIDE_STREAMS = {}
 
 
 def _side_stream(device):
-    """A second stream per device (default priority) for the closed-form scan
-    and the decomposed heads when each kernel of a call is timed
-    (KernelTimer); untimed calls use the library's own side stream."""
+    """A second stream per device (default priority) for the kernels that the
+    library runs on its own side stream, when each kernel of a call is timed
+    (KernelTimer)."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
     if idx not in _SIDE_STREAMS:
         _SIDE_STREAMS[idx] = torch.cuda.Stream(device=idx)
@@ -556,10 +556,10 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
 
 def _timed_run(args, states, n_scan, n_dec, B, T, HD, v, decomp_unsplit):
     """The forward's schedule through the per-kind entry points, each kernel
-    timed on its own stream (KernelTimer): decomposed heads beside live ones
-    run one workgroup per query block (decomp_unsplit = 1), so the live-head
-    kernel's workgroups fill the slots their causal imbalance leaves idle and
-    no key-segment partials are needed.  Returns the raw current stream."""
+    timed on its own stream (KernelTimer): what the library would put on its
+    side stream (saf_mixed_attn_side_kernels) runs on a second torch stream,
+    decomposed heads there one workgroup per query block.  Returns the raw
+    current stream."""
     L, timer = _ext.lib(), _TIMER
     n_live, n_dense = states.count(0), states.count(1)
     work = {"flash": (L.saf_flash_fwd, n_live * B * 4 * HD * T * (T + 1) // 2),
@@ -580,25 +580,23 @@ def _timed_run(args, states, n_scan, n_dec, B, T, HD, v, decomp_unsplit):
         _ext.check(rc)
         timer.records[kind].append((e0, e1, w))
 
-    unsplit = bool(n_live) if decomp_unsplit is None else bool(decomp_unsplit)
-    args.decomp_unsplit = 1 if unsplit else -1
-    dec_side = bool(n_dec and n_live and unsplit)
-    if (n_scan and (n_live or n_dense or n_dec)) or dec_side:
+    if decomp_unsplit is not None:
+        args.decomp_unsplit = 1 if decomp_unsplit else -1
+    sides = L.saf_mixed_attn_side_kernels(args)
+    on_side = [kind for bit, kind in ((1, "decomp"), (2, "scan")) if sides > 0 and sides & bit]
+    if on_side:
         # disjoint output rows and workspace regions; joined before returning
         side = _side_stream(v.device)
         side.wait_stream(cur)
-        if dec_side:
-            launch("decomp", side)
-        if n_scan:
-            launch("scan", side)
-        for kind in ("flash", "dense", "decomp"):
-            if work[kind][1] and not (kind == "decomp" and dec_side):
-                launch(kind, cur)
+        asked, args.decomp_unsplit = args.decomp_unsplit, 1  # the side stream's decomposed heads do not split
+        for kind in on_side:
+            launch(kind, side)
+        args.decomp_unsplit = asked
+    for kind in KernelTimer.KINDS:
+        if work[kind][1] and kind not in on_side:
+            launch(kind, cur)
+    if on_side:
         cur.wait_stream(side)
-    else:
-        for kind in KernelTimer.KINDS:
-            if work[kind][1]:
-                launch(kind, cur)
     return cur.cuda_stream
 
 

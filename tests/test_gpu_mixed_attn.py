@@ -535,10 +535,9 @@ def test_decomposed_beside_live_heads_unsplit_vs_split(with_scan):
 def test_timed_per_kind_path_matches_single_call():
     """With a KernelTimer installed, fused_mixed_attn runs each head kind
     through its own entry point (saf_flash_fwd, saf_frozen_dense_pv_fwd,
-    saf_frozen_decomp_fwd, saf_frozen_scan_fwd; scan and decomposed heads on
-    a second stream) and times each kernel; without one it makes the single
-    saf_mixed_attn_fwd call, which forks the library's own side stream.  Both
-    give the same rows (the scan's look-back order may move a last fp32 bit,
+    saf_frozen_decomp_fwd, saf_frozen_scan_fwd) and times each kernel; without
+    one it makes the single saf_mixed_attn_fwd call (here both in order on one
+    stream: the call is too short to fork).  Both give the same rows (the scan's look-back order may move a last fp32 bit,
     so one bf16 step is allowed) and the timer records every kind."""
     K = _kernel()
     B, H, T, hd, S = 2, 8, 1500, 64, 1536
@@ -574,3 +573,35 @@ def test_timed_per_kind_path_matches_single_call():
                                     None, None, patt=patt.numpy(), alpha=f64(alpha), rho=f64(rho), z=f64(z),
                                     sm_scale=scale_of(hd))
     compare(y_one, ref, what="single call")
+
+
+@pytest.mark.parametrize("B,T,forks", [(2, 700, False), (8, 2900, True)])
+def test_timed_schedule_forks_where_the_call_does(B, T, forks, monkeypatch):
+    """The timed per-kind schedule puts the scan and the decomposed heads on a
+    second stream in calls where the library does (8 GFLOP of decomposed
+    heads), and in no others."""
+    K = _kernel()
+    from kernel import fused_attn
+    H, hd, S = 5, 64, (T + 63) // 64 * 64
+    frozen, hidx, live = routing(H, {1: 2, 2: 2, 3: 2})
+    alpha, rho, z = make_decomp(H, S, seed=8, scale=0.6)
+    ca, cr, cz = closed_params(H, S, {3: ("decay", 0.05)})
+    alpha[3], rho[3], z[3] = ca[3], cr[3], cz[3]
+    cf = K.classify_closed_form(alpha, rho, z)
+    q, k, v = qkv(B, H, T, hd, seed=4, dtype=torch.bfloat16)
+    args = (q[:, live].to(DEV), k[:, live].to(DEV), v.to(DEV), None, frozen.to(DEV), hidx.to(DEV))
+    kw = dict(alpha=alpha.to(DEV), rho=rho.to(DEV), z=z.to(DEV), closed_form=cf)
+    y_one = K.fused_mixed_attn(*args, **kw)
+    used = []
+    side = fused_attn._side_stream
+    monkeypatch.setattr(fused_attn, "_side_stream", lambda dev: used.append(dev) or side(dev))
+    K.set_kernel_timer(K.KernelTimer())
+    try:
+        y_timed = K.fused_mixed_attn(*args, **kw)
+    finally:
+        K.set_kernel_timer(None)
+    torch.cuda.synchronize()
+    assert bool(used) == forks
+    d = (y_one.float() - y_timed.float()).abs()
+    step = (y_one.float().abs() * 2.0 ** -7).clamp_min(2.0 ** -12)
+    assert bool((d <= step).all()), f"timed and single-call paths differ by {d.max().item():.3e}"
