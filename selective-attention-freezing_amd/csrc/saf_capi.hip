@@ -287,18 +287,25 @@ struct FlashPlan {
 };
 
 // Cost of one item, for plan_flash: us per key block (of 64 keys) and query
-// block of the kernel's shape, running alone on its CU.  Fitted to every
-// segment length measured at T = 512 .. 8192, 3 .. 96 (batch, head) pairs
-// (BM = 128 / 256 live at hd <= 64 / 96, 128; 256 / 128 decomposed at
-// hd <= 64 / above; 256 dense, whose cost is the pattern's bytes).
-float flash_block_us(int HD) { return HD <= 64 ? 1.15f : 1.7f; }
-float decomp_block_us(int HD) { return HD <= 64 ? 1.9f : 0.7f; }
+// block of the kernel's shape, running alone on its CU.  Fitted with the rate
+// of the partials to every segment length measured at 13 shapes of each head
+// dim, T = 1024 .. 8192, 2 .. 48 (batch, head) pairs (BM = 128 live at hd 32, 64,
+// 256, 256 at 96, 128; 256 decomposed at hd <= 64, 128 above; 256 dense, whose
+// cost is the pattern's bytes).  The chosen length is then within 2% of the best
+// one in the geometric mean of each head dim.  Decomposed hd 256 has no factored
+// form: its blocks rebuild P, and the value of hd 128 left them unsplit (12
+// heads, T = 2048 107 us where segments of 8 blocks take 67; T = 4096 208 / 134).
+float flash_block_us(int HD) { return HD == 128 ? 1.15f : 1.0f; }
+float decomp_block_us(int HD) { return HD == 256 ? 4.5f : 1.0f; }
+// Rate at which the partials are written and summed, TB/s: the decomposed
+// kernels' blocks leave more of the memory free than the live and dense ones'.
+constexpr float kPartRate = 1.6f, kDecompPartRate = 3.2f;
 float dense_block_us(bool wide) { return wide ? 1.9f : 1.2f; }
 
 // Key segments for the heaviest query blocks, where they pay: the causal tail
 // (the last query block walks every key) outlasts a grid of few workgroups,
 // but a split writes fp32 partials and needs the combine's launch.  The time
-// of a plan is block_us * blocks + 8 us + partial bytes at 1.6 TB/s, where
+// of a plan is block_us * blocks + 8 us + partial bytes at part_rate, where
 // blocks is the mean of two bounds: the work divided over the CUs (at least
 // the longest item), and the sum one CU gets when the items, longest first,
 // are dealt out in turn.  Measured, us, split by the per-slot work (at least
@@ -307,7 +314,8 @@ float dense_block_us(bool wide) { return wide ? 1.9f : 1.2f; }
 // T = 4096 84 / 72; dense fp32, 6 heads T = 2048 47.5 / 34.4; decomposed, 24
 // heads T = 4096 hd 128 92.6 / 76.1.  B counts the work units per slot; each
 // writes part_mult sequences' partials.
-FlashPlan plan_flash(int B, int n_slots, int T, int HD, int BM, float block_us, int part_mult = 1) {
+FlashPlan plan_flash(int B, int n_slots, int T, int HD, int BM, float block_us, float part_rate = kPartRate,
+                     int part_mult = 1) {
   FlashPlan fp;
   const int BMb = BM / 64;
   const int nqb = (T + BM - 1) / BM;
@@ -332,14 +340,13 @@ FlashPlan plan_flash(int B, int n_slots, int T, int HD, int BM, float block_us, 
     const double even = std::max<double>(L, work);
     *n_items = full + rest;
     return block_us * 0.5 * (even + std::max(dealt, even)) +
-           (parts ? 8. + (double)nbh * part_mult * parts * BM * (HD + 2) * 4 / 1.6e6 : 0.);
+           (parts ? 8. + (double)nbh * part_mult * parts * BM * (HD + 2) * 4 / (part_rate * 1e6) : 0.);
   };
   int n_items = 0, best_L = nk;
   double best = cost(nk, &n_items);
   for (int e = 8; e < nk; e *= 2)
-    for (const int L : {e, e + e / 2}) {  // 8, 12, 16, 24, ...: multiples of BMb
-      if (L >= nk) continue;
-      const double c = cost(L, &n_items);
+    for (int L = e; L < std::min(2 * e, nk); L += std::max(e / 4, 4)) {  // 8, 12, 16, 20, ..., 32, 40, ...
+      const double c = cost(L, &n_items);                                // multiples of BMb
       if (c < best && n_items <= kMaxItems) best = c, best_L = L;
     }
   if (best_L == nk) return fp;
@@ -510,7 +517,8 @@ DensePlan plan_dense(int B, int n_slots, int T, int HD, bool wide, bool can_spli
   DensePlan d;
   const int nqb = (T + dense_block_rows(B, HD) - 1) / dense_block_rows(B, HD);
   for (d.group = dense_batch_group(B, HD, wide);; d.group /= 2) {
-    d.fp = can_split ? plan_flash(B / d.group, n_slots, T, HD, dense_block_rows(B, HD), dense_block_us(wide), d.group)
+    d.fp = can_split ? plan_flash(B / d.group, n_slots, T, HD, dense_block_rows(B, HD), dense_block_us(wide), kPartRate,
+                                  d.group)
                      : FlashPlan();
     if (d.group == 1 || d.fp.n_items || (int64_t)nqb * n_slots * (B / d.group) >= cu_count()) return d;
   }
@@ -606,7 +614,7 @@ int64_t part_region_bytes(const saf_mixed_attn_args* args, const Plan& pl) {
                               .fp.part_bytes);
   if (!pl.decomp.empty())
     part = std::max(part, plan_flash(pl.B, (int)pl.decomp.size(), pl.T, pl.HD, block_rows(frozen_qtiles(pl.HD)),
-                                     decomp_block_us(pl.HD)).part_bytes);
+                                     decomp_block_us(pl.HD), kDecompPartRate).part_bytes);
   return round256(part);
 }
 
@@ -650,7 +658,7 @@ int run_decomp(const saf_mixed_attn_args* a, const Plan& pl, hipStream_t s, bool
     p.pat_head[i] = (int16_t)h;
   }
   const int BM = block_rows(frozen_qtiles(pl.HD));
-  FlashPlan fp = plan_flash(pl.B, p.n_slots, pl.T, pl.HD, BM, decomp_block_us(pl.HD));
+  FlashPlan fp = plan_flash(pl.B, p.n_slots, pl.T, pl.HD, BM, decomp_block_us(pl.HD), kDecompPartRate);
   const int64_t part_off = scan_ws_bytes(pl);
   if (pl.dtype != SAF_F32 && fp.n_items && !unsplit && a->workspace != nullptr &&
       a->workspace_bytes >= part_off + fp.part_bytes && reinterpret_cast<uintptr_t>(a->workspace) % 16 == 0) {

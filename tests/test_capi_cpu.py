@@ -184,3 +184,28 @@ def test_side_kernels(B, T, n_dec, n_scan, asked, want):
     assert _ext.lib().saf_mixed_attn_side_kernels(ctypes.byref(a)) == want
     a.n_heads = 0
     assert _ext.lib().saf_mixed_attn_side_kernels(ctypes.byref(a)) == -1
+
+
+def _split_bytes(state, H, T, hd, B=1, patt_dtype=_ext.SAF_F32, pitch=None):
+    """Workspace of H heads of one state beyond what every length of it needs:
+    the partials of split query blocks (a plan that does not split has none)."""
+    a = _args(H=H, T=T, hd=hd, frozen=[state] * H)
+    for t in (a.q, a.k, a.v, a.out):
+        t.size[0] = B
+    for t in (a.alpha, a.rho, a.z):
+        t.data, t.dtype, t.ndim = 0x100000, _ext.SAF_F32, 2
+        t.size[0], t.size[1], t.stride[0], t.stride[1] = H, T, T, 1
+    pitch = pitch or T
+    a.patt.data, a.patt.dtype, a.patt.ndim = 0x100000, patt_dtype, 3
+    for i, (n, st) in enumerate(((H, pitch * T), (T, pitch), (T, 1))):
+        a.patt.size[i], a.patt.stride[i] = n, st
+    n = _ext.lib().saf_mixed_attn_workspace_bytes(ctypes.byref(a))
+    assert n >= 0
+    return n
+
+
+@pytest.mark.parametrize("B,H,T", [(1, 12, 2048), (4, 3, 2048), (1, 12, 4096), (1, 3, 8192)])
+def test_decomposed_hd256_splits(B, H, T):
+    """Decomposed heads of hd 256 rebuild P cell by cell: their long query blocks
+    are split where those of hd 128 may not be (half the time at these shapes)."""
+    assert _split_bytes(2, H, T, 256, B) > 0
