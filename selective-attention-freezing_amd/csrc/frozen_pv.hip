@@ -1064,7 +1064,8 @@ static void launch_dense_t(const FrozenParams& p, hipStream_t s) {
   const dim3 grid((unsigned)(8 * (p.B / NB) * ((groups + 7) / 8)));
   // fp32 patterns take the fast path where their raw operands fit the
   // registers (hd <= 128; half the batch group)
-  if constexpr (std::is_same<T, PT>::value || (std::is_same<PT, float>::value && NB * (HD / 32) <= 4)) {
+  if constexpr (std::is_same<T, PT>::value ||
+                (std::is_same<PT, float>::value && HD <= 128 && NB <= dense_batch_group(4, HD, true))) {
     if (p.patt_vec) {
       hipLaunchKernelGGL((frozen_dense_kernel<T, PT, HD, QT, NB, true>), grid, dim3(64 * kDenseWaves), 0, s, p);
       return;
@@ -1075,14 +1076,13 @@ static void launch_dense_t(const FrozenParams& p, hipStream_t s) {
 
 template <typename T, typename PT, int HD>
 static void launch_dense_nb(const FrozenParams& p, hipStream_t s) {
-  constexpr bool wide = std::is_same<PT, float>::value;
-  if constexpr (dense_batch_group(4, HD, wide) >= 4) {
+  if constexpr (dense_batch_group(4, HD, false) >= 4) {
     if (p.batch_group == 4) {
       launch_dense_t<T, PT, HD, 4>(p, s);
       return;
     }
   }
-  if constexpr (dense_batch_group(4, HD, wide) >= 2) {
+  if constexpr (dense_batch_group(4, HD, false) >= 2) {
     if (p.batch_group == 2) {
       launch_dense_t<T, PT, HD, 2>(p, s);
       return;

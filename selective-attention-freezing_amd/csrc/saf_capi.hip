@@ -300,7 +300,16 @@ float decomp_block_us(int HD) { return HD == 256 ? 4.5f : 1.0f; }
 // Rate at which the partials are written and summed, TB/s: the decomposed
 // kernels' blocks leave more of the memory free than the live and dense ones'.
 constexpr float kPartRate = 1.6f, kDecompPartRate = 3.2f;
-float dense_block_us(bool wide) { return wide ? 1.9f : 1.2f; }
+// How the dense kernel reads a pattern (frozen_pv.hip): in the activation dtype
+// or in fp32 by 16-byte pieces in flight across blocks (fp32 up to hd 128, two
+// loads per operand), or element by element with a wait per block (other types,
+// strides and unaligned rows).
+enum DenseForm { kDenseFast, kDenseWide, kDenseGeneral };
+float dense_block_us(DenseForm f, int HD) {
+  if (f == kDenseGeneral) return HD == 256 ? 4.5f : 3.2f;
+  if (f == kDenseWide) return 1.9f;
+  return HD == 256 ? 2.2f : 1.2f;
+}
 
 // Key segments for the heaviest query blocks, where they pay: the causal tail
 // (the last query block walks every key) outlasts a grid of few workgroups,
@@ -503,6 +512,20 @@ void fill_frozen_common(FrozenParams& p, const saf_tensor_t& v, const saf_tensor
 
 int frozen_qtiles(int hd) { return hd <= 64 ? 2 : 1; }
 
+// Rows that the fast forms take: 16-byte pieces, and lane offsets that span a
+// block of 256 rows in 32 bits, from a descriptor of at most 2 GiB.
+bool dense_vec(const saf_tensor_t& patt, int B, int HD) {
+  const int es = elem_size(patt.dtype);
+  return patt.stride[2] == 1 && reinterpret_cast<uintptr_t>(patt.data) % 16 == 0 && (patt.stride[1] * es) % 16 == 0 &&
+         (patt.stride[0] * es) % 16 == 0 && patt.stride[1] >= 0 &&
+         patt.stride[1] * es * dense_block_rows(B, HD) < ((int64_t)1 << 31);
+}
+DenseForm dense_form(const saf_tensor_t& patt, int act_dtype, int B, int HD) {
+  if (!dense_vec(patt, B, HD)) return kDenseGeneral;
+  if (patt.dtype == act_dtype) return kDenseFast;
+  return patt.dtype == SAF_F32 && HD <= 128 ? kDenseWide : kDenseGeneral;
+}
+
 // Dense P.V work plan: query blocks of the kernel's shape, balanced over the
 // batch groups that share a pattern.  Larger groups read the pattern fewer
 // times; where the plan has nothing to split (short sequences, or no
@@ -513,19 +536,15 @@ struct DensePlan {
   FlashPlan fp;
   int group = 1;
 };
-DensePlan plan_dense(int B, int n_slots, int T, int HD, bool wide, bool can_split) {
+DensePlan plan_dense(int B, int n_slots, int T, int HD, DenseForm form, bool can_split) {
   DensePlan d;
-  const int nqb = (T + dense_block_rows(B, HD) - 1) / dense_block_rows(B, HD);
-  for (d.group = dense_batch_group(B, HD, wide);; d.group /= 2) {
-    d.fp = can_split ? plan_flash(B / d.group, n_slots, T, HD, dense_block_rows(B, HD), dense_block_us(wide), kPartRate,
-                                  d.group)
+  const int BM = dense_block_rows(B, HD), nqb = (T + BM - 1) / BM;
+  for (d.group = dense_batch_group(B, HD, form == kDenseWide);; d.group /= 2) {
+    d.fp = can_split ? plan_flash(B / d.group, n_slots, T, HD, BM, dense_block_us(form, HD), kPartRate, d.group)
                      : FlashPlan();
     if (d.group == 1 || d.fp.n_items || (int64_t)nqb * n_slots * (B / d.group) >= cu_count()) return d;
   }
 }
-
-// A pattern in fp32 for 16-bit activations.
-bool dense_wide(const saf_tensor_t& patt, int act_dtype) { return patt.dtype == SAF_F32 && act_dtype != SAF_F32; }
 
 // Dense P.V over the heads listed; with a workspace large enough for the
 // plan's partials, long query blocks are split into key segments (the flash
@@ -543,11 +562,7 @@ int run_dense(const saf_tensor_t& patt, const saf_tensor_t& v, const saf_tensor_
   p.patt_elems = 1 + (patt.size[0] - 1) * patt.stride[0] + (patt.size[1] - 1) * patt.stride[1] +
                  (patt.size[2] - 1) * patt.stride[2];
   const int es = elem_size(patt.dtype);
-  // the lanes' offsets span a block of 256 rows in 32 bits, from a descriptor
-  // of at most 2 GiB
-  p.patt_vec = patt.stride[2] == 1 && reinterpret_cast<uintptr_t>(patt.data) % 16 == 0 &&
-               (patt.stride[1] * es) % 16 == 0 && (patt.stride[0] * es) % 16 == 0 && patt.stride[1] >= 0 &&
-               patt.stride[1] * es * dense_block_rows(B, HD) < ((int64_t)1 << 31);
+  p.patt_vec = dense_vec(patt, B, HD);
   // the descriptor ends with the 16-byte piece that holds the last element: an
   // odd count of 16-bit elements would end inside a 32-bit word, which then
   // reads as zero
@@ -560,10 +575,10 @@ int run_dense(const saf_tensor_t& patt, const saf_tensor_t& v, const saf_tensor_
     p.v_head[i] = (int16_t)v_head[i];
     p.pat_head[i] = (int16_t)pat_head[i];
   }
-  const bool wide = dense_wide(patt, dtype);
-  DensePlan dp = plan_dense(B, p.n_slots, T, HD, wide, true);
+  const DenseForm form = dense_form(patt, dtype, B, HD);
+  DensePlan dp = plan_dense(B, p.n_slots, T, HD, form, true);
   if (dp.fp.n_items && (ws == nullptr || ws_bytes < dp.fp.part_bytes || reinterpret_cast<uintptr_t>(ws) % 16 != 0))
-    dp = plan_dense(B, p.n_slots, T, HD, wide, false);
+    dp = plan_dense(B, p.n_slots, T, HD, form, false);
   p.batch_group = dp.group;
   FlashPlan& fp = dp.fp;
   if (dtype != SAF_F32 && fp.n_items) {
@@ -610,8 +625,8 @@ int64_t part_region_bytes(const saf_mixed_attn_args* args, const Plan& pl) {
     part = kQueueBytes + fp.part_bytes;
   }
   if (!pl.dense.empty())
-    part = std::max(part, plan_dense(pl.B, (int)pl.dense.size(), pl.T, pl.HD, dense_wide(args->patt, pl.dtype), true)
-                              .fp.part_bytes);
+    part = std::max(part, plan_dense(pl.B, (int)pl.dense.size(), pl.T, pl.HD,
+                                     dense_form(args->patt, pl.dtype, pl.B, pl.HD), true).fp.part_bytes);
   if (!pl.decomp.empty())
     part = std::max(part, plan_flash(pl.B, (int)pl.decomp.size(), pl.T, pl.HD, block_rows(frozen_qtiles(pl.HD)),
                                      decomp_block_us(pl.HD), kDecompPartRate).part_bytes);

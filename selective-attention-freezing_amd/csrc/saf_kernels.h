@@ -330,12 +330,12 @@ inline int block_rows(int qt) { return 4 * 32 * qt; }
 // query tile of 32 rows each) serves a group of NB batch elements that share
 // every pattern operand, at most as many as 128 accumulator registers per
 // wave allow: 4 at hd <= 64 (batch a multiple of 4), 2 at hd <= 128 (even
-// batch), else 1; half of that for fp32 patterns, whose raw operands take
-// twice the registers.  One workgroup per CU (its three V slots fill most of
-// the LDS at hd 128).
+// batch), else 1; half of that where fp32 patterns keep raw operands in
+// flight (wide), which take twice the registers.  One workgroup per CU (its
+// three V slots fill most of the LDS at hd 128).
 constexpr int kDenseWaves = 8;
 constexpr int dense_batch_group(int B, int hd, bool wide) {
-  const int cap = (hd <= 64 ? 4 : (hd <= 128 ? 2 : 1)) / (wide && hd <= 128 ? 2 : 1);
+  const int cap = (hd <= 64 ? 4 : (hd <= 128 ? 2 : 1)) / (wide ? 2 : 1);
   return B % 4 == 0 && cap >= 4 ? 4 : (B % 2 == 0 && cap >= 2 ? 2 : 1);
 }
 constexpr int dense_qtiles(int, int) { return 1; }

@@ -209,3 +209,11 @@ def test_decomposed_hd256_splits(B, H, T):
     """Decomposed heads of hd 256 rebuild P cell by cell: their long query blocks
     are split where those of hd 128 may not be (half the time at these shapes)."""
     assert _split_bytes(2, H, T, 256, B) > 0
+
+
+@pytest.mark.parametrize("B,H,T,hd", [(8, 3, 3001, 64), (4, 8, 4097, 128), (1, 3, 2049, 256)])
+@pytest.mark.parametrize("dtype", [_ext.SAF_BF16, _ext.SAF_F16, _ext.SAF_F32])
+def test_dense_patterns_of_odd_pitch_split(B, H, T, hd, dtype):
+    """Patterns that are read element by element (rows off 16-byte boundaries)
+    cost several times the fast forms' block: their long query blocks are split."""
+    assert _split_bytes(1, H, T, hd, B, patt_dtype=dtype, pitch=T) > 0
