@@ -127,8 +127,8 @@ typedef struct saf_mixed_attn_args {
                                    workgroup per query block on the library's side stream
                                    beside the live-head kernel when live heads share the call
                                    (its workgroups fill the slots the causal imbalance leaves
-                                   idle) and they are long enough to pay for the fork
-                                   (8 GFLOP); otherwise, and in saf_frozen_decomp_fwd, their
+                                   idle) and that pays for the fork
+                                   (saf_mixed_attn_side_kernels); otherwise, and in saf_frozen_decomp_fwd, their
                                    long query blocks are split into key segments (fp32 partials in
                                    the workspace region the live-head and dense kernels also
                                    use, then a combine);

@@ -838,13 +838,54 @@ int side_join_locked(SideStream* ss, hipStream_t s) {
 // Flops of one causal P.V product over n heads of every sequence.
 double pv_flops(const Plan& pl, size_t n) { return (double)pl.B * (double)n * pl.HD * (double)pl.T * pl.T; }
 
-// When forking pays: a fork and join cost about 35 us of host time and a few
+// When forking pays: a fork and join cost 35 to 45 us of host time and about 10
 // us on the caller's stream, against which the side kernel's time is hidden.
-// Decomposed heads (and the backward's frozen dV) of 8 GFLOP and more run
-// beside the live heads: B=8, T=3001 (13.8 GFLOP) 142 us forked, 146 in
-// order; forward + backward at B=8, T=4096 (26 GFLOP) 851 against 902; B=4,
-// T=2048 (3.2 GFLOP) 71 either way, with its backward 249 against 223.
-constexpr double kSideMinFlops = 8e9;
+//
+// Decomposed heads beside live ones run one workgroup per query block, and the
+// longest walks every key block.  `load` is the live heads' work per CU in units
+// of that longest walk.  Measured forked / in order, us (in order: split into
+// key segments after the live heads), 12 heads of which 3 decomposed unless
+// said, T = 1024 .. 8192, B = 1 .. 16:
+//   hd <= 64   the walk (T = 4096 55 us at hd 64) has to fit under the live
+//              heads: load 4.6 (B=8, T=4096) 210 / 225, 3.6 (B=8, T=3000) 140 /
+//              143; below 3 it sticks out: load 2.4 (B=8, T=2048) 90 / 87, 2.3
+//              (B=4, T=4096) 144 / 135, 0.6 (B=1, T=4096) 83 / 74
+//   hd 96, 128 one live workgroup fills a CU: decomposed ones pay beside it
+//              while CUs are left without one: load 0.6 (B=2, T=4096) 145 / 174,
+//              (B=4, T=2048) 92 / 112, 1.2 (B=4, T=4096) 236 / 240; B=8, T=2048
+//              148 / 147; T = 1024 64 / 60
+//   hd 256     rebuilds P, 4 us a block unsplit: only short calls that leave
+//              most CUs idle, T = 1024 B=1 82 / 94; B=1, T=2048 135 either way,
+//              T=4096 276 / 244
+//   float32    neither form splits, and 32-row workgroups fill the chip early:
+//              hd 128 B=1, T=4096 413 / 453, B=2, T=2048 229 / 244, B=4, T=2048
+//              421 / 414; hd 64 B=1, T=4096 275 / 269
+bool decomp_beside_live(const Plan& pl) {
+  const int nk = (pl.T + 63) / 64;
+  const double pairs = (double)pl.B * (double)pl.live.size();
+  const int BM = flash_block_rows(pl.HD, 1), nqb = (pl.T + BM - 1) / BM;
+  const double load = pairs * nqb * (nqb + 1) / 2 * (BM / 64) / cu_count() / nk;
+  if (pl.dtype == SAF_F32) return pl.HD > 64 && nk >= 32 && pairs * nk <= 2.25 * cu_count();
+  if (pl.HD <= 64) return load >= 3;
+  if (pl.HD == 256) return nk <= 16 && load < 0.5;
+  return nk >= 32 && load < 1.25;
+}
+// The backward's frozen dV hides beside dQ and dK / dV wherever these are long
+// enough, since each workgroup walks its blocks in turn at B = 1 as at B = 8 (3.8
+// us per 64 rows for the three kernels up to hd 64, 5.6 above; the rates are the
+// kernels' own): from an estimate of 170 us on.  Forward + backward, forked /
+// in order, us: hd 64 B=8, T=2048 (206) 282 / 308, B=2, T=4096 (243) 289 / 358,
+// B=4, T=3000, 6 decomposed (191) 268 / 315; hd 128 B=1, T=2048 (179) 232 / 268,
+// B=4, T=2048 (207) 315 / 358; dense fp32 patterns B=2, T=4096 301 / 336, hd 128
+// B=2, T=4096 541 / 604.  Below, the host's share decides: hd 64 B=4, T=2048
+// (122) 177 / 211 on a fast host and 202 / 194 on a slow one, B=8, T=1536 (102)
+// 203 / 181, T=1024 133 / 156 and 206 / 160.
+constexpr double kSideMinBwdUs = 170;
+double bwd_us(const Plan& pl, size_t n_frozen) {
+  const bool f32 = pl.dtype == SAF_F32;
+  const double work = pv_flops(pl, pl.live.size()) * (f32 ? 5e-8 : 9e-9) + pv_flops(pl, n_frozen) * (f32 ? 1e-8 : 5e-9);
+  return std::max(work, (pl.T + 63) / 64 * (pl.HD <= 64 ? 3.8 : 5.6));
+}
 // The scan (10 us or so) runs beside the other kernels when these take about
 // 240 us: one 16384-token layer 347 us either way and a 12-layer prefill of
 // them 7.40 against 7.45 ms, but B=8, T=4096 185 us forked, 184 in order;
@@ -858,7 +899,7 @@ int side_kernels(const saf_mixed_attn_args* a, const Plan& pl, unsigned which) {
   const bool has_dec = (which & kDoDecomp) && !pl.decomp.empty();
   const bool has_live = (which & kDoFlash) && !pl.live.empty();
   const bool dec = has_dec && has_live && a->decomp_unsplit >= 0 &&
-                   (a->decomp_unsplit > 0 || pv_flops(pl, pl.decomp.size()) >= kSideMinFlops);
+                   (a->decomp_unsplit > 0 || decomp_beside_live(pl));
   const double main_us = 2 * pv_flops(pl, has_live ? pl.live.size() : 0) * 1.2e-9 +
                          pv_flops(pl, (has_dec && !dec ? pl.decomp.size() : 0) +
                                           ((which & kDoDense) ? pl.dense.size() : 0)) * 2e-9;
@@ -1457,7 +1498,7 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
   // the frozen heads' dV (its own rows of dv, no workspace) on the side
   // stream beside the live heads' kernels, whose tails leave slots idle,
   // where it is long enough to pay for the fork
-  const bool fork = !pl.live.empty() && nf > 0 && pv_flops(pl, nf) >= kSideMinFlops;
+  const bool fork = !pl.live.empty() && nf > 0 && bwd_us(pl, nf) >= kSideMinBwdUs;
   std::unique_lock<std::mutex> lock(g_side_mu, std::defer_lock);
   SideStream* ss = nullptr;
   if (fork) {

@@ -378,7 +378,7 @@ def fused_mixed_attn(q, k, v, patt, frozen, hidx=None, pidx=None,
                chunk after the first gives up: NaN rows, and with validate
                a RuntimeError)
       decomp_unsplit  None (auto) = True when live heads share the call and
-               the decomposed ones are long enough to pay for a fork; True:
+               that pays for a fork (saf_mixed_attn_side_kernels); True:
                decomposed heads run one workgroup per query block, beside the
                live-head kernel on a side stream when there is one; False:
                key-segment split with partials and a combine, after the

@@ -159,26 +159,36 @@ def test_cpu_table_sharing_memory():
         assert host.tolist() == states and list(twin) == states
 
 
-@pytest.mark.parametrize("B,T,n_dec,n_scan,asked,want", [
-    (1, 1024, 2, 0, 0, 0),     # 0.13 GFLOP of decomposed heads: in order
-    (1, 1024, 2, 1, 1, 3),     # asked for: the scan goes along
-    (8, 4096, 1, 0, 0, 1),     # 8.6 GFLOP
-    (8, 4096, 1, 0, -1, 0),
-    (8, 4096, 0, 1, 0, 0),     # 40 us of live heads
-    (8, 16384, 0, 1, 0, 2),
-    (8, 16384, 1, 1, -1, 2),
+@pytest.mark.parametrize("hd,B,T,n_live,n_dec,n_scan,asked,want", [
+    (64, 1, 1024, 1, 2, 0, 0, 0),
+    (64, 1, 1024, 1, 2, 1, 1, 3),      # asked for: the scan goes along
+    (64, 8, 4096, 9, 3, 0, 0, 1),      # hd 64: the live heads outlast a decomposed walk
+    (64, 8, 4096, 9, 3, 0, -1, 0),
+    (64, 4, 4096, 9, 3, 0, 0, 0),
+    (64, 8, 2048, 9, 3, 0, 0, 0),
+    (64, 8, 3001, 9, 3, 1, 0, 3),
+    (32, 8, 3000, 9, 3, 0, 0, 1),
+    (128, 4, 2048, 9, 3, 0, 0, 1),     # hd 128: CUs are left without a live workgroup
+    (128, 1, 1024, 9, 3, 0, 0, 0),
+    (128, 8, 4096, 9, 3, 0, 0, 0),
+    (96, 2, 4096, 9, 3, 0, 0, 1),
+    (256, 1, 1024, 9, 3, 0, 0, 1),
+    (256, 2, 4096, 9, 3, 0, 0, 0),
+    (64, 8, 4096, 1, 0, 1, 0, 0),      # 40 us of live heads
+    (64, 8, 16384, 1, 0, 1, 0, 2),
+    (64, 8, 16384, 1, 1, 1, -1, 2),
 ])
-def test_side_kernels(B, T, n_dec, n_scan, asked, want):
+def test_side_kernels(hd, B, T, n_live, n_dec, n_scan, asked, want):
     """Which kernels leave the caller's stream: one rule for the call and for
     the per-kind schedule that is timed."""
-    H = 1 + n_dec + n_scan
-    a = _args(H=H, T=T, frozen=[0] + [2] * (n_dec + n_scan))
+    H = n_live + n_dec + n_scan
+    a = _args(H=H, T=T, hd=hd, frozen=[0] * n_live + [2] * (n_dec + n_scan))
     for t in (a.q, a.k, a.v, a.out):
         t.size[0] = B
     for t in (a.alpha, a.rho, a.z):
         t.data, t.dtype, t.ndim = 0x100000, _ext.SAF_F32, 2
         t.size[0], t.size[1], t.stride[0], t.stride[1] = H, T, T, 1
-    kinds = (ctypes.c_int32 * H)(*[0] * (1 + n_dec), *[1] * n_scan)
+    kinds = (ctypes.c_int32 * H)(*[0] * (n_live + n_dec), *[1] * n_scan)
     prm = (ctypes.c_float * H)()
     a.closed_kind, a.closed_param, a.decomp_unsplit = kinds, prm, asked
     assert _ext.lib().saf_mixed_attn_side_kernels(ctypes.byref(a)) == want

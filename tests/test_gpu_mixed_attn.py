@@ -493,9 +493,9 @@ def test_invalid_args_raise():
 
 @pytest.mark.parametrize("with_scan", [False, True])
 def test_decomposed_beside_live_heads_unsplit_vs_split(with_scan):
-    """Decomposed heads next to live heads run one workgroup per query block
-    on the side stream, beside the live-head kernel (the default); forced
-    back to the key-segment split with partials and a combine on the current
+    """Decomposed heads next to live heads made to run one workgroup per query
+    block on the side stream, beside the live-head kernel (decomp_unsplit=True,
+    the default where it pays for a fork); made to run as the key-segment split with partials and a combine on the current
     stream (decomp_unsplit=False) they give the same rows to fp32 rounding,
     both within the bound of the float64 oracle.  The live rows are
     bit-identical.  T = 3000 at B = 4 makes the split plan cut the long
@@ -517,7 +517,7 @@ def test_decomposed_beside_live_heads_unsplit_vs_split(with_scan):
     cf = K.classify_closed_form(alpha, rho, z) if closed else None
     args = (q[:, live].to(DEV), k[:, live].to(DEV), v.to(DEV), None, frozen.to(DEV), hidx.to(DEV))
     kw = dict(alpha=alpha.to(DEV), rho=rho.to(DEV), z=z.to(DEV), closed_form=cf)
-    y_side = K.fused_mixed_attn(*args, **kw)
+    y_side = K.fused_mixed_attn(*args, decomp_unsplit=True, **kw)
     y_split = K.fused_mixed_attn(*args, decomp_unsplit=False, **kw)
     torch.cuda.synchronize()
     assert torch.equal(y_side[:, live], y_split[:, live])
@@ -575,14 +575,13 @@ def test_timed_per_kind_path_matches_single_call():
     compare(y_one, ref, what="single call")
 
 
-@pytest.mark.parametrize("B,T,forks", [(2, 700, False), (8, 2900, True)])
-def test_timed_schedule_forks_where_the_call_does(B, T, forks, monkeypatch):
+@pytest.mark.parametrize("B,T,hd,forks", [(2, 700, 64, False), (2, 2100, 128, True)])
+def test_timed_schedule_forks_where_the_call_does(B, T, hd, forks, monkeypatch):
     """The timed per-kind schedule puts the scan and the decomposed heads on a
-    second stream in calls where the library does (8 GFLOP of decomposed
-    heads), and in no others."""
+    second stream in calls where the library does, and in no others."""
     K = _kernel()
     from kernel import fused_attn
-    H, hd, S = 5, 64, (T + 63) // 64 * 64
+    H, S = 5, (T + 63) // 64 * 64
     frozen, hidx, live = routing(H, {1: 2, 2: 2, 3: 2})
     alpha, rho, z = make_decomp(H, S, seed=8, scale=0.6)
     ca, cr, cz = closed_params(H, S, {3: ("decay", 0.05)})
