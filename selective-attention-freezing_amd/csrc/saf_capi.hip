@@ -1497,8 +1497,13 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
   }
   // the frozen heads' dV (its own rows of dv, no workspace) on the side
   // stream beside the live heads' kernels, whose tails leave slots idle,
-  // where it is long enough to pay for the fork
-  const bool fork = !pl.live.empty() && nf > 0 && bwd_us(pl, nf) >= kSideMinBwdUs;
+  // where it is long enough to pay for the fork.  Not under graph capture: a
+  // forked forward captured together with its forked backward ended the host
+  // process inside hipStreamEndCapture, for a cause that is not known
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipError_t e = hipStreamIsCapturing(s, &cs); e != hipSuccess)
+    return fail(SAF_ELAUNCH, "hipStreamIsCapturing failed: %s", hipGetErrorString(e));
+  const bool fork = cs == hipStreamCaptureStatusNone && !pl.live.empty() && nf > 0 && bwd_us(pl, nf) >= kSideMinBwdUs;
   std::unique_lock<std::mutex> lock(g_side_mu, std::defer_lock);
   SideStream* ss = nullptr;
   if (fork) {

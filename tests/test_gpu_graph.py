@@ -1,9 +1,9 @@
 """HIP graph capture of the prefill (the reference's checkpoint bench
 captures one, nanogpt/bench_checkpoint_prefill.py:87-109).
 
-A model with live, dense, generic decomposed and closed-form heads (the
-closed-form scan runs on a second stream joined inside the capture) is
-captured once; the graph is replayed three times with eager prefills and
+A model with live, dense, generic decomposed and closed-form heads, short
+enough to run on one stream (test_gpu_side_stream.py captures calls that fork),
+is captured once; the graph is replayed three times with eager prefills and
 synchronisations in between, and every replay is compared with the eager
 output of the same tokens (the scan's look-back order can move a last bit:
 cosine >= 0.99999) and with the fp32 oracle."""
