@@ -28,14 +28,16 @@ def _inputs(kind, H, S):
         r = torch.where(torch.arange(S) < 70, r, torch.tensor(float("-inf")))
     elif kind == "spike":   # a key far above the rest: rows before it lie below its chunk's scale
         a[:, S // 2] = 120.0
-    elif kind == "wide":    # logits of scale 40
+    elif kind == "wide":    # logits of scale 40: past the product form's range
         a, r = 80 * a, 40 * torch.randn(H, S, generator=g)
+    elif kind == "scale20":  # logits of scale 20: rows 2^-80 to 2^-132 below their chunk's scale
+        a, r = 40 * a, 20 * r
     elif kind == "late":    # the first keys absent: rows without any key
         a[:, : min(S - 1, 130)] = float("-inf")
     return a, r
 
 
-@pytest.mark.parametrize("kind", ["learned", "decay", "window", "spike", "wide", "late"])
+@pytest.mark.parametrize("kind", ["learned", "decay", "window", "spike", "wide", "scale20", "late"])
 @pytest.mark.parametrize("S", [1, 5, 255, 256, 257, 2047, 2050, 2305, 4099])
 def test_logz_blocks(kind, S):
     import kernel
