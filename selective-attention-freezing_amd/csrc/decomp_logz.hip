@@ -61,6 +61,9 @@ __device__ __forceinline__ void group_max(float (&x)[N], float (*red)[kLzWaves],
     for (int q = 0; q < kLzWaves; ++q) x[i] = fmaxf(x[i], red[i][q]);
 }
 
+// A NaN counts as +inf in a maximum that scales: what it scales is then NaN too.
+__device__ __forceinline__ float top(float m, float x) { return fmaxf(m, x != x ? __builtin_inff() : x); }
+
 // acc[r] += sum over steps of 4 terms of as[t + u] * win(r, u), the window
 // sliding by 4 elements per step.  UP: the window moves up with t (win index
 // 3 + u - r), else down (3 + r - u); p is this lane's first low quad.
@@ -183,9 +186,9 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_kernel(const LogzParam
   for (int j0 = 0; j0 < jend; j0 += kLzChunk) {
     float mx[2] = {ninf, ninf};
 #pragma unroll
-    for (int k = 0; k < kLzNA; ++k) mx[0] = fmaxf(mx[0], av[k] *= kLog2e);
+    for (int k = 0; k < kLzNA; ++k) mx[0] = top(mx[0], av[k] *= kLog2e);
 #pragma unroll
-    for (int k = 0; k < kLzNW; ++k) mx[1] = fmaxf(mx[1], rv[k] *= kLog2e);
+    for (int k = 0; k < kLzNW; ++k) mx[1] = top(mx[1], rv[k] *= kLog2e);
     group_max(mx, red, lane, w);  // its barrier: the previous chunk is consumed
     const float A = mx[0], R = mx[1], sc = A + R;
     if (sc != ninf) {

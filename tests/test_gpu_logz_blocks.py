@@ -87,3 +87,18 @@ def test_gradient_of_one_row_not_finite(bad):
         assert torch.isfinite(rest).all()
         # the two forms round their fp32 sums of a few hundred terms differently
         assert float((rest - want).norm()) <= 1e-5 * float(want.norm())
+
+
+@pytest.mark.parametrize("which,lo,hi", [("alpha", 2048, 4096), ("alpha", 0, 2048), ("rho", 2000, 4500)])
+def test_keys_not_a_number(which, lo, hi):
+    """Rows that meet a NaN are NaN, also where a whole chunk of keys or of
+    distances is; the others are what they are without it."""
+    import kernel
+    H, S = 1, 4500
+    a, r = _inputs("learned", H, S)
+    clean = kernel.decomposed_logz(a.to(DEV), r.to(DEV))
+    (a if which == "alpha" else r)[:, lo:hi] = float("nan")
+    z = kernel.decomposed_logz(a.to(DEV), r.to(DEV))
+    assert torch.isnan(z[:, lo:]).all()
+    # rows of the NaN's block take the direct form: fp32 rounding of z
+    assert lo == 0 or float((z - clean)[:, :lo].abs().max()) <= 1e-5
