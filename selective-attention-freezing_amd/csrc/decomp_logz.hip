@@ -287,11 +287,12 @@ hipError_t launch_decomp_logz(const LogzParams& p, hipStream_t s) {
 // gz_i times a probability <= 1).  Both are one sweep over the rows i >= o of an
 // output index o: o's own logit part (alpha_j for dalpha, rho_d for drho) times a
 // correlation of w_i = gz_i 2^(-z_i) with the other vector's exponentials at
-// i - o, in the forward's layout: per chunk of rows w' = gz_i 2^(-z_i - W) and
+// i - o, in the forward's layout: per chunk of rows w' = gz_i 2^(-z_i - W - G) and
 // o' = 2^(other - O) (W, O the maxima over the chunk's rows and over the elements
-// it can meet), 4 outputs per lane, one FMA per pair, and the chunk's sums join
-// the output's total times 2^(own + O + W).  A product lost below 2^-126 is then
-// worth at most 2^(own + O + W - 126): chunks where own + O + W exceeds kLzScale for some output (logits
+// it can meet, 2^G the power of two at its largest |gz|), 4 outputs per lane, one
+// FMA per pair, and the chunk's sums join the output's total times 2^(own + O + W
+// + G).  A product lost below 2^-126 is then worth at most 2^(own + O + W - 125)
+// of that |gz|: chunks where own + O + W exceeds kLzScale for some output (logits
 // whose maxima lie far above every pair's value) or is not finite run the direct
 // form, one exp2 per pair over the same sliding window, and so do chunks with a
 // gz that is not finite: the zero that stands for a pair outside the triangle
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_bwd_kernel(const LogzB
   __shared__ __align__(16) float es[kLzChunk];  // direct form: -z log2 e
   __shared__ __align__(16) float ws[kLzWin];    // o' (direct form: other log2 e)
   __shared__ float part[kLzWaves][kLzRows];
-  __shared__ float red[2][kLzWaves];
+  __shared__ float red[3][kLzWaves];
 
   const float ninf = -__builtin_inff();
   const int S = p.S;
@@ -346,24 +347,26 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_bwd_kernel(const LogzB
   };
   load(o0);
   for (int c0 = o0; c0 < S; c0 += kLzChunk) {
-    float mx[2] = {ninf, ninf};
+    float mx[3] = {ninf, ninf, 0.f};
 #pragma unroll
     for (int k = 0; k < kLzNA; ++k) {
       const bool none = ev[k] == ninf;  // z of a row without a share
       gv[k] = none ? 0.f : gv[k];
       ev[k] = none ? ninf : -ev[k] * kLog2e;
       mx[0] = fmaxf(mx[0], __builtin_isfinite(gv[k]) ? ev[k] : -ninf);
+      mx[2] = fmaxf(mx[2], fabsf(gv[k]));
     }
 #pragma unroll
     for (int k = 0; k < kLzNW; ++k) mx[1] = fmaxf(mx[1], ov[k] *= kLog2e);
     group_max(mx, red, lane, w);  // its barrier: the previous chunk is consumed
     const float W = mx[0], O = mx[1], sc = O + W;
+    const int G = __builtin_amdgcn_frexp_expf(mx[2]);
     const bool fast = fmx + sc <= kLzScale;  // false where not comparable
 #pragma unroll
     for (int k = 0; k < kLzNA; ++k) {
       const int t = tid + k * kLzThreads;
       // a row without a share (ev -inf) adds nothing whatever the maxima are
-      as[t] = fast ? (ev[k] == ninf ? 0.f : gv[k] * fast_exp2(ev[k] - W)) : gv[k];
+      as[t] = fast ? (ev[k] == ninf ? 0.f : __builtin_ldexpf(gv[k], -G) * fast_exp2(ev[k] - W)) : gv[k];
       if (!fast) es[t] = ev[k];
     }
 #pragma unroll
@@ -385,7 +388,7 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_bwd_kernel(const LogzB
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float c = fixed[r] + sc;
-        tot[r] = fmaf(acc[r], c == ninf ? 0.f : fast_exp2(c), tot[r]);
+        tot[r] += __builtin_ldexpf(acc[r] * (c == ninf ? 0.f : fast_exp2(c)), G);
       }
     } else {
       if (W == -ninf)  // a gz that is not finite

@@ -89,6 +89,29 @@ def test_gradient_of_one_row_not_finite(bad):
         assert float((rest - want).norm()) <= 1e-5 * float(want.norm())
 
 
+@pytest.mark.parametrize("exp", [-112, -104, 60, 115])
+def test_gradient_scales_with_gz(exp):
+    """gz times a power of two gives the gradients times that power, also where
+    the logits' maxima lie far above every pair's value (a stripe's products
+    then hold gz times up to 2^40 less than a pair is worth)."""
+    import kernel
+    H, S = 1, 700
+    a, r = _inputs("learned", H, S)
+    a[:, 300] += 13.5   # peaks that no row meets together: maxima 2^38 above any pair
+    r[:, 500] += 13.5
+    gz = torch.randn(H, S, generator=torch.Generator().manual_seed(2))
+    grads = []
+    for f in (1.0, 2.0 ** exp):
+        ad, rd = a.to(DEV).requires_grad_(), r.to(DEV).requires_grad_()
+        z = kernel.decomp_log_normalizers(ad, rd)
+        grads.append(torch.autograd.grad(z, (ad, rd), (gz * f).to(DEV)))
+    for one, got, name in zip(*grads, ("dalpha", "drho")):
+        got = got.double() * 2.0 ** -exp
+        # what 2^exp takes below the normal numbers is lost: 2^-126 / 2^exp
+        err = (got - one.double()).abs()
+        assert (err <= 1e-6 * one.double().abs() + 2.0 ** (-126 - exp)).all(), f"{name}: {float(err.max()):.2e}"
+
+
 @pytest.mark.parametrize("which,lo,hi", [("alpha", 2048, 4096), ("alpha", 0, 2048), ("rho", 2000, 4500)])
 def test_keys_not_a_number(which, lo, hi):
     """Rows that meet a NaN are NaN, also where a whole chunk of keys or of
