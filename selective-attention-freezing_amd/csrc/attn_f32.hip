@@ -26,7 +26,7 @@
 // over ColFrag row i: P and dS never leave their registers.
 //
 // Bound by the matrix pipe: at B=4, 12 heads (9 live), T=1000, hd 64 the
-// forward + backward takes 322 us against 1762 us on the vector ALUs
+// forward + backward takes 297 us against 1759 us on the vector ALUs
 // (64 x 64 tiles in LDS, one workgroup per tile); the forward alone at B=8,
 // 12 live heads, T=2000 runs at 115 TFLOP/s (25 before).
 //

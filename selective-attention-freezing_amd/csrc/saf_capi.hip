@@ -1500,10 +1500,12 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
   // where it is long enough to pay for the fork.  Not under graph capture: a
   // forked forward captured together with its forked backward ended the host
   // process inside hipStreamEndCapture, for a cause that is not known
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipError_t e = hipStreamIsCapturing(s, &cs); e != hipSuccess)
-    return fail(SAF_ELAUNCH, "hipStreamIsCapturing failed: %s", hipGetErrorString(e));
-  const bool fork = cs == hipStreamCaptureStatusNone && !pl.live.empty() && nf > 0 && bwd_us(pl, nf) >= kSideMinBwdUs;
+  bool fork = !pl.live.empty() && nf > 0 && bwd_us(pl, nf) >= kSideMinBwdUs;
+  if (fork) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    fork = hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // the default stream cannot be asked while another one is captured
+  }
   std::unique_lock<std::mutex> lock(g_side_mu, std::defer_lock);
   SideStream* ss = nullptr;
   if (fork) {
