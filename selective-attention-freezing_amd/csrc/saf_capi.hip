@@ -1503,8 +1503,9 @@ int saf_mixed_attn_bwd(const saf_mixed_attn_args* a, const saf_tensor_t* dout, c
   bool fork = !pl.live.empty() && nf > 0 && bwd_us(pl, nf) >= kSideMinBwdUs;
   if (fork) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    fork = hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
-    (void)hipGetLastError();  // the default stream cannot be asked while another one is captured
+    const hipError_t e = hipStreamIsCapturing(s, &cs);
+    if (e != hipSuccess) (void)hipGetLastError();  // the default stream, while another one is captured
+    fork = e == hipSuccess && cs == hipStreamCaptureStatusNone;
   }
   std::unique_lock<std::mutex> lock(g_side_mu, std::defer_lock);
   SideStream* ss = nullptr;
