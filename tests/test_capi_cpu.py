@@ -227,3 +227,19 @@ def test_dense_patterns_of_odd_pitch_split(B, H, T, hd, dtype):
     """Patterns that are read element by element (rows off 16-byte boundaries)
     cost several times the fast forms' block: their long query blocks are split."""
     assert _split_bytes(1, H, T, hd, B, patt_dtype=dtype, pitch=T) > 0
+
+
+def test_aligned_view_keeps_what_both_rules_accept():
+    """_aligned_view's one pass over shape and strides against the two rules it
+    stands for, over strides, sizes of one, offsets and types."""
+    import random
+    from kernel import fused_attn as F
+    r = random.Random(1)
+    for _ in range(3000):
+        shape = [r.choice([1, 2, 3]) for _ in range(3)] + [r.choice([1, 32, 64])]
+        stride = [r.choice([0, 1, 8, 16, 24, 32, 64, 65, 72, 128, 4096]) for _ in range(3)] + [r.choice([0, 1, 2])]
+        base = torch.zeros(30000, dtype=r.choice([torch.bfloat16, torch.float32]))
+        x = base.as_strided(shape, stride, r.choice([0, 1, 8]))
+        kept = F._aligned_view(x, 16) is x
+        # contiguous() returns a tensor that counts as contiguous already
+        assert kept == (F._row_aligned(x, 16) and F._rows_apart(x)) or x.is_contiguous(), (shape, stride)
