@@ -26,7 +26,7 @@
 // pair.  H=12, us, one exp2 per logit always / a direct form from 2^-80 on, of one
 // 64-row block at a time with two LDS reads per pair / now: logits of scale 20
 // S=2048 18 / 37 / 12, S=8192 130 / 212 / 64; of scale 40, where most groups run both
-// forms, S=8192 130 / - / 133 (S=2048, 96 work-groups, 18 / - / 31).
+// forms, S=2048 17 / - / 14, S=8192 130 / - / 133.
 //
 // Bound by FMA issue (S(S+1)/2 per head; HBM traffic is 3 S 4 bytes):
 // H=12, S=8192: 135 us (one exp2 per logit) -> 23 us; S=16384: 321 -> 61 us.
@@ -34,14 +34,13 @@
 
 namespace saf {
 
-constexpr int kLzRows = 256;           // rows (outputs) of a work-group
+constexpr int kLzRows = 256;           // rows (outputs) of a work-group (64 where these are few: launch)
 constexpr int kLzWaves = 8;
 constexpr int kLzThreads = 64 * kLzWaves;
 constexpr int kLzChunk = 2048;         // keys per chunk
 constexpr int kLzWin = kLzChunk + kLzRows;
 constexpr int kLzNA = kLzChunk / kLzThreads;                       // staged values per thread
 constexpr int kLzNW = (kLzWin + kLzThreads - 1) / kLzThreads;
-static_assert(kLzWaves * kLzRows <= kLzWin, "the direct form's row maxima fit the window");
 constexpr int kLzBias = 52;                       // forward: exponent added to a' and to r'
 constexpr float kLzLow = 3.725290298461914e-09f;  // 2^-28: 2^-132 of the scale and both biases
 constexpr float kLn2 = 0.6931471805599453f;
@@ -151,24 +150,31 @@ __device__ __forceinline__ float biased_exp2(float x) {
   return __builtin_ldexpf(fast_exp2(x - n), (int)n + kLzBias);
 }
 
+// ROWS rows per work-group, 256 or 64: 64 lanes cover them (4 each) LG times over,
+// each time with another share of the keys.
+template <int ROWS>
 __global__ __launch_bounds__(kLzThreads) void decomp_logz_kernel(const LogzParams p) {
+  constexpr int LG = kLzRows / ROWS, kUnits = kLzWaves * LG;  // shares of a chunk's keys
+  constexpr int kWin = kLzChunk + ROWS, kNW = (kWin + kLzThreads - 1) / kLzThreads;
+  static_assert(kUnits * ROWS <= kWin, "the direct form's row maxima fit the window");
   __shared__ __align__(16) float as[kLzChunk];
-  __shared__ __align__(16) float rs[kLzWin];
-  __shared__ float part[kLzWaves][kLzRows];
+  __shared__ __align__(16) float rs[kWin];
+  __shared__ float part[kUnits][ROWS];
   __shared__ float red[2][kLzWaves];
 
   const float ninf = -__builtin_inff();
   const int S = p.S;
-  const int nblk = (S + kLzRows - 1) / kLzRows;
-  const int i0 = (nblk - 1 - (int)blockIdx.y) * kLzRows;  // heaviest first
-  const int h = blockIdx.x;
+  const int nblk = (S + ROWS - 1) / ROWS;
+  const int h = blockIdx.x % p.H;
+  const int i0 = (nblk - 1 - (int)(blockIdx.x / p.H)) * ROWS;  // heaviest first
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rl = lane % (ROWS / 4), unit = w * LG + lane / (ROWS / 4);
   const float* alpha = p.alpha + (int64_t)h * p.a_hs;
   const float* rho = p.rho + (int64_t)h * p.r_hs;
-  const int jend = min(i0 + kLzRows, S);  // keys any row of the block can see
+  const int jend = min(i0 + ROWS, S);  // keys any row of the block can see
 
   float M = ninf, tot[4] = {0.f, 0.f, 0.f, 0.f};
-  float av[kLzNA], rv[kLzNW];
+  float av[kLzNA], rv[kNW];
   auto load = [&](int j0) {  // this thread's share of a chunk's keys and window
     const int dlo = i0 - j0 - kLzChunk + 1;  // distance of window element 0
 #pragma unroll
@@ -177,9 +183,9 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_kernel(const LogzParam
       av[k] = j < jend ? alpha[j] : ninf;
     }
 #pragma unroll
-    for (int k = 0; k < kLzNW; ++k) {
+    for (int k = 0; k < kNW; ++k) {
       const int x = tid + k * kLzThreads, d = dlo + x;
-      rv[k] = (x < kLzWin && d >= 0 && d < S) ? rho[d] : ninf;
+      rv[k] = (x < kWin && d >= 0 && d < S) ? rho[d] : ninf;
     }
   };
   load(0);
@@ -188,39 +194,39 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_kernel(const LogzParam
 #pragma unroll
     for (int k = 0; k < kLzNA; ++k) mx[0] = top(mx[0], av[k] *= kLog2e);
 #pragma unroll
-    for (int k = 0; k < kLzNW; ++k) mx[1] = top(mx[1], rv[k] *= kLog2e);
+    for (int k = 0; k < kNW; ++k) mx[1] = top(mx[1], rv[k] *= kLog2e);
     group_max(mx, red, lane, w);  // its barrier: the previous chunk is consumed
     const float A = mx[0], R = mx[1], sc = A + R;
     if (sc != ninf) {
 #pragma unroll
       for (int k = 0; k < kLzNA; ++k) as[tid + k * kLzThreads] = biased_exp2(av[k] - A);
 #pragma unroll
-      for (int k = 0; k < kLzNW; ++k)
-        if (tid + k * kLzThreads < kLzWin) rs[tid + k * kLzThreads] = biased_exp2(rv[k] - R);
+      for (int k = 0; k < kNW; ++k)
+        if (tid + k * kLzThreads < kWin) rs[tid + k * kLzThreads] = biased_exp2(rv[k] - R);
     }
     __syncthreads();
     load(j0 + kLzChunk);  // lands while the products run
     __builtin_amdgcn_sched_barrier(0);
     if (sc == ninf) continue;  // every logit of the chunk is -inf
     const int n = min(kLzChunk, jend - j0);
-    const int quota = ((n + kLzWaves - 1) / kLzWaves + 3) / 4 * 4;  // keys past n are zero
+    const int quota = ((n + kUnits - 1) / kUnits + 3) / 4 * 4;  // keys past n are zero
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    // window element of (row 4 lane + r, key t): 4 lane + r + kLzChunk - 1 - t
+    // window element of (row 4 rl + r, key t): 4 rl + r + kLzChunk - 1 - t
     const int n4 = (n + 3) / 4 * 4;
-    slide<false>(acc, as, rs + 4 * lane + kLzChunk - 4, min(w * quota, n4), min((w + 1) * quota, n4));
+    slide<false>(acc, as, rs + 4 * rl + kLzChunk - 4, min(unit * quota, n4), min((unit + 1) * quota, n4));
     const float Mn = fmaxf(M, sc), f0 = fast_exp2(M - Mn), f1 = fast_exp2(sc - Mn);
 #pragma unroll
     for (int r = 0; r < 4; ++r) tot[r] = fmaf(acc[r], f1, tot[r] * f0);
     M = Mn;
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) part[w][4 * lane + r] = tot[r];
+  for (int r = 0; r < 4; ++r) part[unit][4 * rl + r] = tot[r];
   __syncthreads();
-  bool low = false;  // of this thread's row (the first kLzRows threads)
-  if (tid < kLzRows && i0 + tid < S) {
+  bool low = false;  // of this thread's row (the first ROWS threads)
+  if (tid < ROWS && i0 + tid < S) {
     float s = 0.f;
 #pragma unroll
-    for (int q = 0; q < kLzWaves; ++q) s += part[q][tid];
+    for (int q = 0; q < kUnits; ++q) s += part[q][tid];
     low = !(s >= kLzLow && s < __builtin_inff());  // NaN included
     const float e = (float)(__builtin_amdgcn_frexp_expf(s) - 2 * kLzBias);
     if (!low) p.z[(int64_t)h * p.z_hs + i0 + tid] = (M + (e + log2f(__builtin_amdgcn_frexp_mantf(s)))) * kLn2;
@@ -238,14 +244,14 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_kernel(const LogzParam
 #pragma unroll
     for (int k = 0; k < kLzNA; ++k) as[tid + k * kLzThreads] = av[k] * kLog2e;
 #pragma unroll
-    for (int k = 0; k < kLzNW; ++k)
-      if (tid + k * kLzThreads < kLzWin) rs[tid + k * kLzThreads] = rv[k] * kLog2e;
+    for (int k = 0; k < kNW; ++k)
+      if (tid + k * kLzThreads < kWin) rs[tid + k * kLzThreads] = rv[k] * kLog2e;
     __syncthreads();
     load(j0 + kLzChunk);
     const int n = min(kLzChunk, jend - j0), n8 = (n + 7) / 8 * 8;  // keys past n are -inf
-    const int quota = ((n + kLzWaves - 1) / kLzWaves + 7) / 8 * 8;
-    const int t0 = min(w * quota, n8), t1 = min((w + 1) * quota, n8);
-    const float* const win = rs + 4 * lane + kLzChunk - 4;
+    const int quota = ((n + kUnits - 1) / kUnits + 7) / 8 * 8;
+    const int t0 = min(unit * quota, n8), t1 = min((unit + 1) * quota, n8);
+    const float* const win = rs + 4 * rl + kLzChunk - 4;
     if (t0 < t1) {
       if (check)
         slide_lse<true>(m, s, as, win, t0, t1);
@@ -254,28 +260,35 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_kernel(const LogzParam
     }
   }
   __syncthreads();
-  float* const pm = rs;  // [wave][row] maxima
+  float* const pm = rs;  // [unit][row] maxima
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    pm[w * kLzRows + 4 * lane + r] = m[r];
-    part[w][4 * lane + r] = s[r];
+    pm[unit * ROWS + 4 * rl + r] = m[r];
+    part[unit][4 * rl + r] = s[r];
   }
   __syncthreads();
   if (low) {
     float mx = ninf, sum = 0.f;
 #pragma unroll
-    for (int q = 0; q < kLzWaves; ++q) mx = fmaxf(mx, pm[q * kLzRows + tid]);
+    for (int q = 0; q < kUnits; ++q) mx = fmaxf(mx, pm[q * ROWS + tid]);
     const float ref = mx == ninf ? 0.f : mx;
 #pragma unroll
-    for (int q = 0; q < kLzWaves; ++q) sum += part[q][tid] * fast_exp2(pm[q * kLzRows + tid] - ref);
+    for (int q = 0; q < kUnits; ++q) sum += part[q][tid] * fast_exp2(pm[q * ROWS + tid] - ref);
     p.z[(int64_t)h * p.z_hs + i0 + tid] = (ref + log2f(sum)) * kLn2;  // log2f(0): no key at all, -inf
   }
 }
 
 hipError_t launch_decomp_logz(const LogzParams& p, hipStream_t s) {
   const int nblk = (p.S + kLzRows - 1) / kLzRows;
-  // heads first: a CU's second work-group is lighter than its first
-  hipLaunchKernelGGL(decomp_logz_kernel, dim3(p.H, nblk), dim3(kLzThreads), 0, s, p);
+  // Heads first: a CU's second work-group is lighter than its first.  64 rows
+  // where 256 would leave CUs without a work-group.  256 / 64, us, learned logits
+  // and scale 40 (both forms): 12 heads S=2048 (96 groups of 256) 7.1 / 6.3 and 29.6
+  // / 14.2, S=4096 (192) 11.6 / 10.6 and 57 / 33; 24 heads S=3072 (288) 10.8 / 12.4
+  // and 46 / 36, S=8192 (768) 31 / 46 and 199 / 182.
+  if ((int64_t)nblk * p.H < p.n_cu)
+    hipLaunchKernelGGL(decomp_logz_kernel<64>, dim3((unsigned)p.H * ((p.S + 63) / 64)), dim3(kLzThreads), 0, s, p);
+  else
+    hipLaunchKernelGGL(decomp_logz_kernel<kLzRows>, dim3((unsigned)p.H * nblk), dim3(kLzThreads), 0, s, p);
   return hipGetLastError();
 }
 
@@ -312,9 +325,9 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_bwd_kernel(const LogzB
 
   const float ninf = -__builtin_inff();
   const int S = p.S;
-  const int o0 = (int)blockIdx.y * kLzRows;   // heaviest first
-  const int h = (int)blockIdx.x >> 1;
-  const bool dr = blockIdx.x & 1;              // 0: dalpha, 1: drho
+  const int o0 = (int)(blockIdx.x / (2 * p.H)) * kLzRows;  // heaviest first
+  const int h = (int)(blockIdx.x % (2 * p.H)) >> 1;
+  const bool dr = blockIdx.x & 1;                          // 0: dalpha, 1: drho
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const float* alpha = p.alpha + (int64_t)h * p.a_hs;
   const float* rho = p.rho + (int64_t)h * p.r_hs;
@@ -412,7 +425,7 @@ __global__ __launch_bounds__(kLzThreads) void decomp_logz_bwd_kernel(const LogzB
 
 hipError_t launch_decomp_logz_bwd(const LogzBwdParams& p, hipStream_t s) {
   const int nblk = (p.S + kLzRows - 1) / kLzRows;
-  hipLaunchKernelGGL(decomp_logz_bwd_kernel, dim3(2 * p.H, nblk), dim3(kLzThreads), 0, s, p);
+  hipLaunchKernelGGL(decomp_logz_bwd_kernel, dim3(2u * p.H * nblk), dim3(kLzThreads), 0, s, p);
   return hipGetLastError();
 }
 

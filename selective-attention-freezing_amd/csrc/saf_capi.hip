@@ -1324,6 +1324,7 @@ int saf_decomposed_logz(const saf_tensor_t* alpha, const saf_tensor_t* rho, cons
     return fail(SAF_EUNSUPPORTED, "decomposed_logz: H = %lld, S = %lld out of range", (long long)H, (long long)S);
   if (H == 0 || S == 0) return SAF_OK;
   LogzParams p{};
+  p.n_cu = cu_count();
   p.alpha = static_cast<const float*>(alpha->data);
   p.rho = static_cast<const float*>(rho->data);
   p.z = static_cast<float*>(z->data);

@@ -239,6 +239,7 @@ struct LogzParams {
   float* z;
   int64_t a_hs, r_hs, z_hs;  // head (row) strides, elements
   int H, S;
+  int n_cu;  // compute units of the device
 };
 
 hipError_t launch_decomp_logz(const LogzParams& p, hipStream_t s);

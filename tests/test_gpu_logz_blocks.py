@@ -125,3 +125,19 @@ def test_keys_not_a_number(which, lo, hi):
     assert torch.isnan(z[:, lo:]).all()
     # rows of the NaN's block take the direct form: fp32 rounding of z
     assert lo == 0 or float((z - clean)[:, :lo].abs().max()) <= 1e-5
+
+
+@pytest.mark.parametrize("kind", ["learned", "window", "spike", "wide", "scale20", "late"])
+@pytest.mark.parametrize("H,S", [(26, 2305), (32, 2048), (129, 257), (256, 255)])
+def test_logz_rows_of_256(kind, H, S):
+    """Calls with a work-group of 256 rows for every CU (the tests above have
+    fewer and take 64) against each head alone."""
+    import kernel
+    a, r = (t.to(DEV) for t in _inputs(kind, H, S))
+    z = kernel.decomposed_logz(a, r).double()
+    for h in range(0, H, 1 if H < 100 else 17):
+        one = kernel.decomposed_logz(a[h:h + 1].contiguous(), r[h:h + 1].contiguous())[0].double()
+        fin = torch.isfinite(one)
+        assert torch.equal(fin, torch.isfinite(z[h]))
+        assert bool(((z[h] - one).abs()[fin] <= 1e-5 * (1 + one.abs()[fin])).all()), f"head {h}"
+
